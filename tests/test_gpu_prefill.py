@@ -100,6 +100,28 @@ def test_prefill_f16_kv_matches_single_steps(n, a_start, a_count, layers):
         o.close()
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 32, 33, 64, 65, 129, 193])
+def test_prefill_column_widths(n):
+    """The edges of the GEMM's column widths: one column up to the whole 16,
+    32 or 64 of the thin grids, then the multiples of 64, with the K slices
+    each width picks (1e-3, the bar of the other prefill tests: both sides
+    are f32 sums, which differ by about 1e-5)."""
+    print(f"[prefill] 1 layer, {n} tokens", flush=True)
+    g = gpu_engine(n_layers=1, max_seq=256)
+    o = oracle_engine(n_layers=1, max_seq=256)
+    try:
+        tokens = np.random.default_rng(1000 + n).integers(0, 131072, n)
+        g.prefill(tokens)
+        oracle_prefill(o, tokens, 0, 0, None)
+        assert g.position == n
+        check_kv(g, o, 1, n)
+        assert max_rel_err(g.debug_read("hidden", 3072), o.buffer("hidden")) < 1e-3
+        assert max_rel_err(g.debug_read("normed", 3072), o.buffer("normed")) < 1e-3
+    finally:
+        g.destroy()
+        o.close()
+
+
 def test_prefill_two_chunks_after_context():
     """300 tokens on top of 10 cached positions in 256-token chunks: chunks
     of 256 and 44, the second attending to the first through the cache."""

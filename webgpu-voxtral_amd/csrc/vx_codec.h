@@ -19,7 +19,7 @@
 //   - the input conv's B is gathered straight from the codes (vqLookup,
 //     fsqDequant and concatCodecInput fused into the packing).
 // Tokens are processed in column chunks of at most CX_MAXT; a chunk's B
-// holds nc = 2 * nt columns (nt = tokens rounded up to 128, hi then lo),
+// holds nc = 2 * nt columns (nt = gm_cols(tokens), hi then lo),
 // each column's K halves contiguous; the GEMM output C is [nc][M].
 #pragma once
 #include "vx_prefill.h"

@@ -1593,31 +1593,31 @@ static int pf_gemm_setup(vx_engine *e) {
 
 // pf_c[s][col][m] for s < *ns: the ns K-slice partial sums of
 // W[M][K] x pf_b (2 nt rows of K halves)
-static int pf_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nt, int *ns) {
-  if (M % GM_BM || K % GM_BK || nt % GM_BN)
+static int pf_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nt, int n, int *ns) {
+  if (M % GM_BM || K % GM_BK || n < 1 || nt != gm_cols(n))
     return fail(e, VX_E_STATE, "prefill GEMM shape M %d K %d nt %d", M, K, nt);
   const GemmPlan p = gemm_plan(M, K, nt, e->cus);
-  if (p.slices != 1 && p.slices != 2 && p.slices != 4 && p.slices != 8)
+  if (p.slices < 1 || p.slices > 8)
     return fail(e, VX_E_STATE, "prefill GEMM plan with %d slices", p.slices);
   if ((size_t)p.slices * nt * M > (size_t)PF_NC * 2 * HID)
     return fail(e, VX_E_STATE, "prefill GEMM output (%d slices of %d x %d) exceeds its buffer", p.slices, nt, M);
-  gemm_launch(p, e->st, W, M, K, (const uint16_t *)e->pf_b, nt, e->pf_c);
+  gemm_launch(p, e->st, W, M, K, (const uint16_t *)e->pf_b, nt, n, e->pf_c);
   *ns = p.slices;
   return VX_OK;
 }
 
 // cx_c[s][col][m] for s < *ns: the codec chunk's K-slice partial sums of
 // W[M][K] x cx_b (nc = 2 nt rows of K halves)
-static int cx_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nc, int *ns) {
+static int cx_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nc, int n, int *ns) {
   const int nt = nc / 2;
-  if (M % GM_BM || K % GM_BK || nt % GM_BN)
+  if (M % GM_BM || K % GM_BK || n < 1 || nt != gm_cols(n))
     return fail(e, VX_E_STATE, "codec GEMM shape M %d K %d nt %d", M, K, nt);
   const GemmPlan p = gemm_plan(M, K, nt, e->cus);
-  if (p.slices != 1 && p.slices != 2 && p.slices != 4 && p.slices != 8)
+  if (p.slices < 1 || p.slices > 8)
     return fail(e, VX_E_STATE, "codec GEMM plan with %d slices", p.slices);
   if ((size_t)p.slices * nt * M > CX_CCAP)
     return fail(e, VX_E_STATE, "codec GEMM output (%d slices of %d x %d) exceeds its buffer", p.slices, nt, M);
-  gemm_launch(p, e->st, W, M, K, (const uint16_t *)e->cx_b, nt, e->cx_c);
+  gemm_launch(p, e->st, W, M, K, (const uint16_t *)e->cx_b, nt, n, e->cx_c);
   *ns = p.slices;
   return VX_OK;
 }
@@ -1625,7 +1625,7 @@ static int cx_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nc, int *n
 static int enqueue_prefill_chunk(vx_engine *e, int n, int tok0, int vstart, int vcount,
                                  bool has_voice) {
   int rc = VX_OK, ns = 1;
-  const int nt = pf_nt(n);
+  const int nt = gm_cols(n);
   hipStream_t st = e->st;
   const int pos0 = e->host_pos;
   hipLaunchKernelGGL(pf_embed_kernel, dim3(n, DIM / 256), dim3(256), 0, st, e->tok_emb, e->pf_tok,
@@ -1637,7 +1637,7 @@ static int enqueue_prefill_chunk(vx_engine *e, int n, int tok0, int vstart, int 
   for (int l = 0; l < e->cfg.n_layers; l++) {
     const LayerW &W = e->L[l];
     const bool next = l + 1 < e->cfg.n_layers;
-    if ((rc = pf_gemm(e, W.wqkv, QKV_ROWS, DIM, nt, &ns))) return rc;
+    if ((rc = pf_gemm(e, W.wqkv, QKV_ROWS, DIM, nt, n, &ns))) return rc;
     gm_with_slices(ns, [&](auto NS) {
       hipLaunchKernelGGL(pf_qkv_epi_kernel<NS>, dim3(n, QKV_ROWS / 2 / 256), blk, 0, st, e->pf_c, nt,
                          e->pf_q, e->kc(l), e->vc(l), e->kv_f32, e->max_seq, pos0, e->inv_freq);
@@ -1650,18 +1650,18 @@ static int enqueue_prefill_chunk(vx_engine *e, int n, int tok0, int vstart, int 
       hipLaunchKernelGGL(pf_attn_mfma_kernel<uint16_t>, dim3(nt / PFA_T, NKV), dim3(256 * PFA_KG),
                          PFA_LDS, st, e->pf_q, (const uint16_t *)e->kc(l), (const uint16_t *)e->vc(l),
                          e->max_seq, pos0, n, nt, e->pf_b);
-    if ((rc = pf_gemm(e, W.wo, DIM, QD, nt, &ns))) return rc;
+    if ((rc = pf_gemm(e, W.wo, DIM, QD, nt, n, &ns))) return rc;
     gm_with_slices(ns, [&](auto NS) {
       hipLaunchKernelGGL((pf_resid_pack_kernel<true, NS>), dim3(nt), blk, 0, st, e->pf_c, n, nt, e->pf_x,
                          W.ffn_norm, e->cfg.norm_eps, e->pf_b);
     });
     // W1 and W3 are adjacent in the arena: one GEMM over the stacked rows
-    if ((rc = pf_gemm(e, W.w1, 2 * HID, DIM, nt, &ns))) return rc;
+    if ((rc = pf_gemm(e, W.w1, 2 * HID, DIM, nt, n, &ns))) return rc;
     gm_with_slices(ns, [&](auto NS) {
       hipLaunchKernelGGL(pf_swiglu_pack_kernel<NS>, dim3(nt, HID / 8 / 128), dim3(128), 0, st, e->pf_c, n,
                          nt, e->pf_b);
     });
-    if ((rc = pf_gemm(e, W.w2, DIM, HID, nt, &ns))) return rc;
+    if ((rc = pf_gemm(e, W.w2, DIM, HID, nt, n, &ns))) return rc;
     gm_with_slices(ns, [&](auto NS) {
       if (next)
         hipLaunchKernelGGL((pf_resid_pack_kernel<true, NS>), dim3(nt), blk, 0, st, e->pf_c, n, nt, e->pf_x,
@@ -1916,10 +1916,10 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
   const CodecW &w = e->cw;
   const int levels = e->cfg.acoustic_levels;
   const dim3 blk(256);
-  // token chunks [t0, t0 + n) with nc = 2 * round_up(n, 128) B columns
+  // token chunks [t0, t0 + n) with nc = 2 gm_cols(n) B columns
   auto chunks = [&](int TT, auto &&body) {
     for (int t0 = 0; t0 < TT; t0 += e->cx_chunk) {
-      const int n = std::min(e->cx_chunk, TT - t0), nc = 2 * ((n + 127) / 128 * 128);
+      const int n = std::min(e->cx_chunk, TT - t0), nc = 2 * gm_cols(n);
       body(t0, n, nc);
     }
   };
@@ -1935,7 +1935,7 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
     hipLaunchKernelGGL(cx_pack_in_kernel, dim3(nc / 2), dim3(128), 0, st, e->cx_cb, e->cx_sem,
                        e->cx_ac, levels, t0, n, nc, e->cx_b);
     int ns = 1;
-    if (!rc) rc = cx_gemm(e, e->cx_ain, CD, CKIN, nc, &ns);
+    if (!rc) rc = cx_gemm(e, e->cx_ain, CD, CKIN, nc, n, &ns);
     gm_with_slices(ns, [&](auto NS) {
       hipLaunchKernelGGL(cx_scale_rows_epi_kernel<NS>, dim3(n, CD / 256), blk, 0, st, e->cx_c, CD, nc, t0,
                          e->cx_rs_in, CD, e->cx_x, CD);
@@ -1951,7 +1951,7 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
         hipLaunchKernelGGL(cx_pack_kernel<true>, dim3(nc / 2), blk, 0, st, x, CD, t0, n, nc,
                            L.attn_norm, CX_NORM_EPS, e->cx_b);
         int ns = 1;
-        if (!rc) rc = cx_gemm(e, L.wqkv, 3 * CD, CD, nc, &ns);
+        if (!rc) rc = cx_gemm(e, L.wqkv, 3 * CD, CD, nc, n, &ns);
         gm_with_slices(ns, [&](auto NS) {
           hipLaunchKernelGGL(cx_qkv_epi_kernel<NS>, dim3(n, 3 * CNH / 4), blk, 0, st, e->cx_c, nc, t0,
                              L.q_norm, L.k_norm, e->cx_q, e->cx_k, e->cx_v);
@@ -1963,7 +1963,7 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
         hipLaunchKernelGGL(cx_pack_kernel<false>, dim3(nc / 2), blk, 0, st, e->cx_attn, CD, t0, n,
                            nc, nullptr, 0.f, e->cx_b);
         int ns = 1;
-        if (!rc) rc = cx_gemm(e, L.wo, CD, CD, nc, &ns);
+        if (!rc) rc = cx_gemm(e, L.wo, CD, CD, nc, n, &ns);
         gm_with_slices(ns, [&](auto NS) {
           hipLaunchKernelGGL(cx_resid_epi_kernel<NS>, dim3(n, CD / 256), blk, 0, st, e->cx_c, nc, t0,
                              L.attn_scale, x);
@@ -1973,13 +1973,13 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
         hipLaunchKernelGGL(cx_pack_kernel<true>, dim3(nc / 2), blk, 0, st, x, CD, t0, n, nc,
                            L.ffn_norm, CX_NORM_EPS, e->cx_b);
         int ns = 1;
-        if (!rc) rc = cx_gemm(e, L.w13, 2 * CHID, CD, nc, &ns);
+        if (!rc) rc = cx_gemm(e, L.w13, 2 * CHID, CD, nc, n, &ns);
         // the gate/up GEMM has consumed B: the SwiGLU epilogue refills it
         gm_with_slices(ns, [&](auto NS) {
           hipLaunchKernelGGL(cx_swiglu_epi_kernel<NS>, dim3(nc / 2, CHID / 8 / 256), blk, 0, st, e->cx_c,
                              nc, n, e->cx_b);
         });
-        if (!rc) rc = cx_gemm(e, L.w2, CD, CHID, nc, &ns);
+        if (!rc) rc = cx_gemm(e, L.w2, CD, CHID, nc, n, &ns);
         gm_with_slices(ns, [&](auto NS) {
           hipLaunchKernelGGL(cx_resid_epi_kernel<NS>, dim3(n, CD / 256), blk, 0, st, e->cx_c, nc, t0,
                              L.ffn_scale, x);
@@ -1993,7 +1993,7 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
       hipLaunchKernelGGL(cx_pack_up_kernel, dim3(nc / 2), blk, 0, st, x, e->cx_s_up[s], t0, n, nc,
                          e->cx_b);
       int ns = 1;
-      if (!rc) rc = cx_gemm(e, e->cx_aup[s], 2 * CD, CKUP, nc, &ns);
+      if (!rc) rc = cx_gemm(e, e->cx_aup[s], 2 * CD, CKUP, nc, n, &ns);
       gm_with_slices(ns, [&](auto NS) {
         hipLaunchKernelGGL(cx_up_epi_kernel<NS>, dim3(n, 2 * CD / 256), blk, 0, st, e->cx_c, nc, t0, x2);
       });
@@ -2013,7 +2013,7 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
   chunks(TT, [&](int t0, int n, int nc) {
     hipLaunchKernelGGL(cx_pack_out_kernel, dim3(nc / 2), blk, 0, st, x, t0, n, nc, e->cx_b);
     int ns = 1;
-    if (!rc) rc = cx_gemm(e, e->cx_aout, CPATCH_ROWS, CKOUT, nc, &ns);
+    if (!rc) rc = cx_gemm(e, e->cx_aout, CPATCH_ROWS, CKOUT, nc, n, &ns);
     gm_with_slices(ns, [&](auto NS) {
       hipLaunchKernelGGL(cx_scale_rows_epi_kernel<NS>, dim3(n, 1), blk, 0, st, e->cx_c, CPATCH_ROWS, nc,
                          t0, e->cx_rs_out, CPATCH, e->cx_audio, CPATCH);

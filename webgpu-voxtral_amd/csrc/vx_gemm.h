@@ -201,27 +201,29 @@ __device__ __forceinline__ void gm_iteration(const GmLane &L, unsigned char *sme
 }
 
 // Split-K grid: block (x, s) computes tile x (XCD-grouped, m-major) over K
-// slice s of KS = gridDim.y and writes C block s.  Needs M % 256 == 0,
-// nt % 64 == 0, K % (64 KS) == 0.
+// slice s of KS = gridDim.y (K / 64 k-tiles in KS near-equal runs) and writes
+// C block s.  Needs M % 256 == 0, nt % 64 == 0, K % 64 == 0, KS <= K / 64.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_split_kernel(
     const uint16_t *__restrict__ W, int M, int K, const uint16_t *__restrict__ B, int nt, float *__restrict__ C,
     int ldc) {
   extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
   const GmLane L(threadIdx.x);
   const int n_tiles = nt / GM_BN, m_tiles = M / GM_BM;
-  // tiles m-major; the blocks b with b % 8 == x take the x-th eighth.
-  // Workgroups are dealt to the 8 XCDs round-robin (from a starting XCD that
-  // varies between launches), so blocks with equal b % 8 share an XCD: the
-  // column tiles sharing a weight tile run together and one L2 serves the
-  // re-reads
+  // tiles m-major; the blocks b with b % 8 == x take the x-th eighth (the
+  // first tiles % 8 eighths hold one more).  Workgroups are dealt to the 8
+  // XCDs round-robin (from a starting XCD that varies between launches), so
+  // blocks with equal b % 8 share an XCD: the column tiles sharing a weight
+  // tile run together and one L2 serves the re-reads.  (Without the grouping
+  // O at 320 columns, 60 tiles in 4 slices, took 28.5 us against 23.)
   int mt, ntl;
   {
-    const int b = blockIdx.x, tiles = m_tiles * n_tiles;
-    const int tile = (tiles & 7) == 0 ? (b & 7) * (tiles >> 3) + (b >> 3) : b;
+    const int x = blockIdx.x & 7, tiles = m_tiles * n_tiles;
+    const int tile = x * (tiles >> 3) + min(x, tiles & 7) + (blockIdx.x >> 3);
     mt = tile / n_tiles;
     ntl = tile - mt * n_tiles;
   }
-  const int kh = K / gridDim.y, kb = blockIdx.y * kh, nk = kh / GM_BK, last = nk - 1;
+  const int kt0 = (int)(blockIdx.y * (K / GM_BK) / gridDim.y), kb = kt0 * GM_BK;
+  const int nk = (int)((blockIdx.y + 1) * (K / GM_BK) / gridDim.y) - kt0, last = nk - 1;
   const uint16_t *base[GM_LOADS];
 #pragma unroll
   for (int i = 0; i < GM_LOADS; i++) {
@@ -364,24 +366,176 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   __builtin_amdgcn_s_waitcnt(gm_vmcnt(0));
 }
 
+// Thin grid, for chunks of at most GT_MAXN columns: the product is then bound
+// by the weight stream (two flops per weight byte and column), so what
+// matters is bytes in flight on every CU and few bytes of everything else.
+// Block (x, s): BM = 32 RT weight rows, K slice s of gridDim.y, all NT
+// columns.  A k-tile's BM + 2 NT rows are staged as above (ring of S stages,
+// 48-72 KB, so two or three blocks share a CU and one's barriers run under
+// the others' loads), but the four waves split the k-tile's 64 halves, 16
+// each, instead of its rows: every staged byte is read from LDS once (rows
+// split over waves would read the B rows four times), and each wave holds the
+// block's whole BM x 2 NT product, RT x NT / 16 tiles of
+// v_mfma_f32_32x32x16_f16 whose columns are the hi rows, then the lo rows.
+// At the end the four waves' hi and lo sums are added through LDS in a fixed
+// order and only the live columns col < n are written.  NTW: the weight loads
+// carry the non-temporal hint, as each weight is read by one block only.
+// Weights cycled from HBM, all of M x K = 18432 x 3072 (113 MB): 16 columns
+// 21.6 us (23.8 without the hint), 32 columns 26.7 us, where the split grid
+// takes 54 us (at its 128 columns) and the decode GEMV 18.4 us for one;
+// 3072 x 9216: 11.7 and 14.0 us against 25; 1024 x 1024: 2.6 and 2.8 us
+// against 6.5.
+constexpr int GT_MAXN = 64;
+template <int RT, int NT>
+struct GtShape {
+  static constexpr int BM = 32 * RT;
+  static constexpr int STAGE = (BM + 2 * NT) * GM_ROWB;
+  static constexpr int LOADS = (BM + 2 * NT) / 32;  // direct loads per wave per k-tile
+  static constexpr int CT = NT / 16;                // 32-column tiles of the 2 NT B rows
+  static constexpr int S = NT == 16 ? (RT == 1 ? 6 : 4) : NT == 32 && RT == 1 ? 4 : 3;
+  static constexpr int RW = 36;                     // floats per reduction row: 32 weight rows + pad
+  static constexpr int RED = 4 * 2 * NT * RW * 4;   // reduction area in bytes
+  static constexpr int LDS = S * STAGE > RED ? S * STAGE : RED;
+};
+
+// waits until at most min(younger, S - 2) k-tiles of L loads are in flight
+template <int S, int L>
+__device__ __forceinline__ void gt_wait(int younger) {
+  if constexpr (S > 2) {
+    if (younger >= S - 2)
+      __builtin_amdgcn_s_waitcnt(gm_vmcnt(L * (S - 2)));
+    else
+      gt_wait<S - 1, L>(younger);
+  } else {
+    __builtin_amdgcn_s_waitcnt(gm_vmcnt(0));
+  }
+}
+
+template <bool NTW>
+__device__ __forceinline__ void gt_direct(const uint16_t *src, unsigned char *lds_row_block) {
+  __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)lds_row_block, 16, 0,
+                                   NTW ? 2 : 0);
+}
+
+template <int RT, int NT, bool NTW>
+__global__ __launch_bounds__(256) void gemm_thin_kernel(const uint16_t *__restrict__ W, int K,
+                                                        const uint16_t *__restrict__ B, int n,
+                                                        float *__restrict__ C, int ldc) {
+  using G = GtShape<RT, NT>;
+  constexpr int S = G::S;
+  extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, h = lane >> 5;
+  const int m0 = blockIdx.x * G::BM, nk = K / GM_BK;
+  const int k0 = (int)(blockIdx.y * nk / gridDim.y), cnt = (int)((blockIdx.y + 1) * nk / gridDim.y) - k0;
+  // direct load i of this wave fills stage rows 8 (4 i + wave) .. + 8: weight
+  // rows for i < RT, then the B rows (hi, lo)
+  const uint16_t *src[G::LOADS];
+#pragma unroll
+  for (int i = 0; i < G::LOADS; i++) {
+    const int row = 8 * (4 * i + wave) + (lane >> 3), chunk = (lane & 7) ^ gm_key(row);
+    src[i] = (i < RT ? W + (size_t)(m0 + row) * K : B + (size_t)(row - G::BM) * K) + k0 * GM_BK + chunk * 8;
+  }
+  auto issue = [&](int stage) {
+#pragma unroll
+    for (int i = 0; i < G::LOADS; i++) {
+      unsigned char *dst = gm_smem + stage * G::STAGE + (4 * i + wave) * 1024;
+      if (i < RT) gt_direct<NTW>(src[i], dst);
+      else gt_direct<false>(src[i], dst);
+      src[i] += GM_BK;
+    }
+  };
+  gm_f32x16 acc[RT][G::CT];
+#pragma unroll
+  for (int i = 0; i < RT; i++)
+#pragma unroll
+    for (int j = 0; j < G::CT; j++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
+#pragma unroll
+  for (int s = 0; s < S - 1; s++)
+    if (s < cnt) issue(s);
+  const int c = 2 * wave + h;  // this lane's 16-byte chunk of every row
+  int stage = 0, fill = S - 1;
+  for (int t = 0; t < cnt; t++) {
+    gt_wait<S, G::LOADS>(cnt - 1 - t);
+    // every wave's part of k-tile t is in, and every wave has read k-tile
+    // t - 1, whose stage k-tile t + S - 1 takes
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + S - 1 < cnt) issue(fill);
+    const unsigned char *st = gm_smem + stage * G::STAGE;
+    gm_h8 a[RT], b[G::CT];
+#pragma unroll
+    for (int i = 0; i < RT; i++) {
+      const int row = 32 * i + r;
+      a[i] = *(const gm_h8 *)(st + row * GM_ROWB + ((c ^ gm_key(row)) << 4));
+    }
+#pragma unroll
+    for (int j = 0; j < G::CT; j++) {
+      const int row = G::BM + 32 * j + r;
+      b[j] = *(const gm_h8 *)(st + row * GM_ROWB + ((c ^ gm_key(row)) << 4));
+    }
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+      for (int j = 0; j < G::CT; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[j], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_s_waitcnt(GM_LGKM0);  // this wave's reads are done before the next barrier
+    stage = stage + 1 == S ? 0 : stage + 1;
+    fill = fill + 1 == S ? 0 : fill + 1;
+  }
+  float *red = (float *)gm_smem;
+  C += (size_t)blockIdx.y * NT * ldc;
+#pragma unroll
+  for (int i = 0; i < RT; i++) {
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < G::CT; j++)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; g4++)
+        *(gm_f32x4 *)(red + (wave * 2 * NT + 32 * j + r) * G::RW + 8 * g4 + 4 * h) =
+            gm_f32x4{acc[i][j][4 * g4], acc[i][j][4 * g4 + 1], acc[i][j][4 * g4 + 2], acc[i][j][4 * g4 + 3]};
+    __syncthreads();
+    for (int o = tid; o < NT * 8; o += 256) {
+      const int col = o >> 3, m = 4 * (o & 7);
+      if (col < n) {
+        gm_f32x4 v = *(const gm_f32x4 *)(red + col * G::RW + m);
+#pragma unroll
+        for (int w = 1; w < 4; w++) v += *(const gm_f32x4 *)(red + (w * 2 * NT + col) * G::RW + m);
+#pragma unroll
+        for (int w = 0; w < 4; w++) v += *(const gm_f32x4 *)(red + (w * 2 * NT + NT + col) * G::RW + m);
+        *(gm_f32x4 *)(C + (size_t)col * ldc + m0 + 32 * i + m) = v;
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------- host side
+// columns (hi, and as many lo) of a chunk of n tokens
+inline int gm_cols(int n) { return n <= 16 ? 16 : n <= 32 ? 32 : (n + GM_BN - 1) / GM_BN * GM_BN; }
+
 struct GemmPlan {
+  int thin = 0;    // thin grid: 32-row tiles per block (0: another grid)
   bool stream = false;
-  int ks = 1;      // split grid: K slices
+  int ks = 1;      // split and thin grids: K slices
   int grid = 0;    // stream grid: blocks
   int share = 0;   // stream grid: k-tiles per block
   int slices = 1;  // C blocks the consumer sums
 };
 
 // Calls f(std::integral_constant<int, NS>) for the slice counts a plan can
-// produce (ns in {1, 2, 4, 8}), so the consumer kernels sum a compile-time
-// number of slices; false for any other count.
+// produce (ns in 1 .. 8), so the consumer kernels sum a compile-time number
+// of slices; false for any other count.
 template <typename F>
 inline bool gm_with_slices(int ns, F &&f) {
   switch (ns) {
     case 1: f(std::integral_constant<int, 1>{}); return true;
     case 2: f(std::integral_constant<int, 2>{}); return true;
+    case 3: f(std::integral_constant<int, 3>{}); return true;
     case 4: f(std::integral_constant<int, 4>{}); return true;
+    case 5: f(std::integral_constant<int, 5>{}); return true;
+    case 6: f(std::integral_constant<int, 6>{}); return true;
+    case 7: f(std::integral_constant<int, 7>{}); return true;
     case 8: f(std::integral_constant<int, 8>{}); return true;
     default: return false;
   }
@@ -399,9 +553,28 @@ inline int gemm_stream_slices(int m_tiles, int nk, int L) {
   return most == 1 ? 1 : most == 2 ? 2 : most <= 4 ? 4 : most <= 8 ? 8 : 0;
 }
 
+// Thin grid: 64-row blocks where M has enough of them for KS <= 8 slices to
+// give every CU three blocks, else 32-row blocks.  KS then is the largest
+// power of two that keeps the grid within 4.5 blocks per CU (1.5 rounds of
+// three) and leaves a block at least 4 k-tiles (2 while the grid is smaller
+// than the device): more slices hide more latency, but each costs its share
+// of the pipeline's fill and of C.
+inline GemmPlan gemm_thin_plan(int M, int K, int nt, int cus) {
+  GemmPlan p;
+  const int nk = K / GM_BK;
+  p.thin = nt == 64 || M / 64 * 8 >= 3 * cus ? 2 : 1;
+  const int blocks = M / (32 * p.thin);
+  while (p.ks < 8 && blocks * p.ks * 2 * 2 <= 9 * cus &&
+         nk / (p.ks * 2) >= (blocks * p.ks < cus ? 2 : 4))
+    p.ks *= 2;
+  p.slices = p.ks;
+  return p;
+}
+
 // cus: the device's compute units (8 XCDs).  Shapes must satisfy
-// M % 256 == 0, nt % 64 == 0, K % 64 == 0.
+// M % 256 == 0, K % 64 == 0, nt = gm_cols(n).
 inline GemmPlan gemm_plan(int M, int K, int nt, int cus) {
+  if (nt < GT_MAXN || (nt == GT_MAXN && M <= 2048)) return gemm_thin_plan(M, K, nt, cus);
   GemmPlan p;
   const int m_tiles = M / GM_BM, n_tiles = nt / GM_BN, tiles = m_tiles * n_tiles, nk = K / GM_BK;
   if (tiles > cus) {
@@ -415,25 +588,69 @@ inline GemmPlan gemm_plan(int M, int K, int nt, int cus) {
     }
     return p;  // split grid, K whole, several rounds
   }
-  // At most one block per CU: K split in KS slices.  (The balanced grid on
-  // all CUs, with a tile cut into up to 8 segments, measured slower for these
-  // shapes: QKV, O and down of the 256-token prompt took 2-5 us more each.)
-  while (p.ks < 8 && tiles * p.ks * 2 <= cus && (nk % (p.ks * 2)) == 0 && nk / (p.ks * 2) >= 2) p.ks *= 2;
+  // At most one block per CU: K split in KS slices, as many as pay: a k-tile
+  // takes a block about 0.65 us, and a slice of C is written and read again
+  // at about 3 TB/s.  (Powers of two that fill the CUs, without the second
+  // term, took 33.0 us for gate/up at 64 columns, KS 2, where KS 3 takes 27.2,
+  // and 18.0 us with the reader of C for 1024 x 1024 at 512 columns, KS 8.
+  // The balanced grid on all CUs, with a tile cut into up to 8 segments,
+  // measured slower for these shapes: QKV, O and down of the 256-token prompt
+  // took 2-5 us more each.)
+  double best = 0;
+  for (int ks = 1; ks <= 8 && tiles * ks <= cus && (ks == 1 || nk / ks >= 2); ks++) {
+    const double us = 0.65 * ((nk + ks - 1) / ks) + ks * (8.0 * nt * M / 3e6);
+    if (ks == 1 || us < best) {
+      best = us;
+      p.ks = ks;
+    }
+  }
   p.slices = p.ks;
   return p;
 }
 
-// both kernels use 144 KB of dynamic LDS
+// f(kernel, LDS bytes) for every thin kernel a plan can name
+template <typename F>
+inline void gm_with_thin(int rt, int nt, bool ntw, F &&f) {
+  auto pick = [&](auto RT, auto NT) {
+    using G = GtShape<RT, NT>;
+    if (ntw) f(gemm_thin_kernel<RT, NT, true>, G::LDS);
+    else f(gemm_thin_kernel<RT, NT, false>, G::LDS);
+  };
+  std::integral_constant<int, 1> one;
+  std::integral_constant<int, 2> two;
+  if (nt == 16) rt == 1 ? pick(one, std::integral_constant<int, 16>{}) : pick(two, std::integral_constant<int, 16>{});
+  else if (nt == 32) rt == 1 ? pick(one, std::integral_constant<int, 32>{}) : pick(two, std::integral_constant<int, 32>{});
+  else if (nt == 64) pick(two, std::integral_constant<int, 64>{});
+}
+
+// the kernels' dynamic LDS: 144 KB for the tiles of 256 x 64, 48 or 72 KB for
+// the thin ones
 inline hipError_t gemm_setup() {
   hipError_t e = hipFuncSetAttribute((const void *)gemm_split_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      GM_LDS);
-  if (e != hipSuccess) return e;
-  return hipFuncSetAttribute((const void *)gemm_stream_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, GM_LDS);
+  if (e == hipSuccess)
+    e = hipFuncSetAttribute((const void *)gemm_stream_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, GM_LDS);
+  for (int rt = 1; rt <= 2; rt++)
+    for (int nt : {16, 32, 64})
+      for (bool ntw : {false, true})
+        gm_with_thin(rt, nt, ntw, [&](auto kernel, int lds) {
+          if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        });
+  return e;
 }
 
+// n: the live columns of the nt (the thin grid writes only those).  A thin
+// weight stream of a matrix past the L2s' size (32 MB) is non-temporal; the
+// codec's matrices (2-17 MB, 298 MB in all) stay allocating, so that a
+// decode of a few frames finds part of them in the 256 MB last-level cache.
 inline void gemm_launch(const GemmPlan &p, hipStream_t st, const uint16_t *W, int M, int K, const uint16_t *B,
-                        int nt, float *C) {
-  if (p.stream)
+                        int nt, int n, float *C) {
+  if (p.thin)
+    gm_with_thin(p.thin, nt, (size_t)M * K >= (size_t)8 << 20, [&](auto kernel, int lds) {
+      hipLaunchKernelGGL(kernel, dim3(M / (32 * p.thin), p.ks), dim3(256), lds, st, W, K, B, n, C, M);
+    });
+  else if (p.stream)
     hipLaunchKernelGGL(gemm_stream_kernel, dim3(p.grid), dim3(256), GM_LDS, st, W, M, K, B, nt, C, M, p.share,
                        p.slices);
   else

@@ -21,9 +21,8 @@ namespace vx {
 
 constexpr int PF_MAXT = 1024;          // tokens per chunk, at most
 constexpr int PF_NC = 2 * PF_MAXT;     // B columns (hi, lo), at most
-// A chunk of n tokens uses nt = n rounded up to 128 hi columns and as many
-// lo columns: N = 2 nt GEMM columns.
-__host__ __device__ constexpr int pf_nt(int n) { return (n + 127) / 128 * 128; }
+// A chunk of n tokens uses nt = gm_cols(n) hi columns (16, 32 or a multiple of
+// 64: the widths the GEMM grids come in) and as many lo columns.
 
 // value of output (token t, row m): the sum of the NS K-slice blocks, in order
 template <int NS>
