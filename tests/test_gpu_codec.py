@@ -76,6 +76,22 @@ def test_chunked_gemms(oracle_codec):
         g.destroy()
 
 
+def test_chunks_hand_on_their_last_keys(oracle_codec):
+    """33 frames in 128-token chunks: stage 2 runs 132 tokens in two chunks
+    (window 8) and stage 3 264 in three (window 16), so each of both layers'
+    halos is written and read in turn; every stage, the same bar."""
+    print("[codec] 33 frames in 128-token chunks", flush=True)
+    os.environ["VX_CODEC_CHUNK"] = "128"
+    try:
+        g = gpu_engine(n_layers=1, max_seq=64)
+    finally:
+        del os.environ["VX_CODEC_CHUNK"]
+    try:
+        check_all(g, oracle_codec, *random_codes(33, 33))
+    finally:
+        g.destroy()
+
+
 def test_codes_outside_the_tables(engine, oracle_codec):
     """Semantic codes 8192 and 8193 (which generate() can emit) and beyond
     read a zero codebook row; acoustic codes below 2 wrap as u32."""

@@ -8,14 +8,18 @@
 // products keep f32 accuracy. A GEMM may leave its sum in up to 8 K-slice
 // partials; the epilogue kernels below (template parameter NS) add them in
 // slice order, so every result is bit-reproducible.
-//   - the causal convs become GEMMs over an im2col B (k-major: column t holds
-//     x[t - (k_size-1) + kk][ci] at k = kk * c_in + ci) with the weights
+//   - the causal convs become GEMMs whose column t holds
+//     x[t - (k_size-1) + kk][ci] at k = kk * c_in + ci, with the weights
 //     reordered to match once after loading; their weight norm g/||w|| is
-//     one scale per output row, applied in the epilogue;
+//     one scale per output row, applied in the epilogue.  For the output conv
+//     (c_in = 1024) column t is the 7 consecutive packed rows t - 6 .. t, so
+//     each row is packed once and the columns overlap (packing one copy per
+//     tap took 18 us of a 250-frame decode and 57 MB); the input conv's 292
+//     channels are no multiple of 16 bytes and are packed per tap;
 //   - the stride-2 transposed conv (kernel 4) gives output step 2 tau + r
 //     from input steps tau (tap r) and tau - 1 (tap r + 2): one GEMM of
-//     2048 rows (both parities) over B = [x[tau]; x[tau - 1]] scaled by the
-//     per-input-channel weight norm;
+//     2048 rows (both parities) over the packed rows x[tau - 1], x[tau],
+//     scaled by the per-input-channel weight norm;
 //   - the input conv's B is gathered straight from the codes (vqLookup,
 //     fsqDequant and concatCodecInput fused into the packing).
 // Tokens are processed in column chunks of at most CX_MAXT; a chunk's B
@@ -104,16 +108,15 @@ __device__ __forceinline__ void cx_put(h8 *B, int nc, int kg, int kb, int t, con
 }
 
 // ------------------------------------------------------------- packing
-// B from rows t0 + t of X [*][K], optionally RMS-normalised with gains g
+// B from rows t0 + t of X [*][K], RMS-normalised with gains g
 // (batchedRmsNorm, src/shaders.ts:1646-1692).  Grid: nt blocks of 256.
-template <bool NORM>
 __global__ __launch_bounds__(256) void cx_pack_kernel(const float *X, int K, int t0, int n, int nc,
                                                       const uint16_t *g, float eps, h8 *B) {
   const int t = blockIdx.x, tid = threadIdx.x;
   const bool live = t < n;
   const float *x = X + (size_t)(t0 + t) * K;
   float r = 1.0f;
-  if (NORM && live) {
+  if (live) {
     __shared__ float red[4];
     float s = 0.f;
     for (int k = tid; k < K; k += 256) s = fmaf(x[k], x[k], s);
@@ -125,13 +128,11 @@ __global__ __launch_bounds__(256) void cx_pack_kernel(const float *X, int K, int
   for (int kb = tid; kb < K / 8; kb += 256) {
     float y[8];
     if (live) {
+      float gv[8];
       cx_load8(x + kb * 8, y);
-      if (NORM) {
-        float gv[8];
-        cx_load8h(g + kb * 8, gv);
+      cx_load8h(g + kb * 8, gv);
 #pragma unroll
-        for (int e = 0; e < 8; e++) y[e] = y[e] * r * gv[e];
-      }
+      for (int e = 0; e < 8; e++) y[e] = y[e] * r * gv[e];
     } else {
 #pragma unroll
       for (int e = 0; e < 8; e++) y[e] = 0.f;
@@ -172,46 +173,32 @@ __global__ __launch_bounds__(128) void cx_pack_in_kernel(const uint16_t *cbn, co
   }
 }
 
-// B of the transposed conv: k = j * CD + ci holds scale[ci] * x[tau - j][ci].
-// Grid: nt blocks of 256.
-__global__ __launch_bounds__(256) void cx_pack_up_kernel(const float *X, const float *scale, int t0,
-                                                         int n, int nc, h8 *B) {
-  const int t = blockIdx.x, tau = t0 + t;
-  for (int kb = threadIdx.x; kb < CKUP / 8; kb += 256) {
-    const int j = kb / (CD / 8), ci0 = (kb - j * (CD / 8)) * 8, src = tau - j;
-    const bool ok = t < n && src >= 0;
-    float y[8];
-    if (ok) {
+// Packed rows of the convs over CD channels: row i of B (hi; lo blo halves
+// further) is x[t0 - before + i], times scale[ci] if given; rows before the
+// first step and rows past step t0 + n - 1 are zero.  Grid: before + nt
+// blocks of 128.
+__global__ __launch_bounds__(128) void cx_pack_rows_kernel(const float *X, const float *scale, int before, int t0,
+                                                           int n, size_t blo, h8 *B) {
+  const int i = blockIdx.x, kb = threadIdx.x, src = t0 - before + i;
+  float y[8];
+  if (src >= 0 && src < t0 + n) {
+    cx_load8(X + (size_t)src * CD + kb * 8, y);
+    if (scale) {
       float sc[8];
-      cx_load8(X + (size_t)src * CD + ci0, y);
-      cx_load8(scale + ci0, sc);
+      cx_load8(scale + kb * 8, sc);
 #pragma unroll
       for (int e = 0; e < 8; e++) y[e] = sc[e] * y[e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; e++) y[e] = 0.f;
     }
-    cx_put(B, nc, CKUP / 8, kb, t, y);
-  }
-}
-
-// im2col B of the output conv (k = 7): k = kk * CD + ci holds
-// x[tau - 6 + kk][ci].  Grid: nt blocks of 256.
-__global__ __launch_bounds__(256) void cx_pack_out_kernel(const float *X, int t0, int n, int nc,
-                                                          h8 *B) {
-  const int t = blockIdx.x, tau = t0 + t;
-  for (int kb = threadIdx.x; kb < CKOUT / 8; kb += 256) {
-    const int kk = kb / (CD / 8), ci0 = (kb - kk * (CD / 8)) * 8, src = tau - (CK_OUT - 1) + kk;
-    float y[8];
-    if (t < n && src >= 0) {
-      cx_load8(X + (size_t)src * CD + ci0, y);
-    } else {
+  } else {
 #pragma unroll
-      for (int e = 0; e < 8; e++) y[e] = 0.f;
-    }
-    cx_put(B, nc, CKOUT / 8, kb, t, y);
+    for (int e = 0; e < 8; e++) y[e] = 0.f;
   }
+  h8 hi, lo;
+  split_n<8>(y, hi, lo);
+  B[(size_t)i * (CD / 8) + kb] = hi;
+  B[blo / 8 + (size_t)i * (CD / 8) + kb] = lo;
 }
+static_assert(CD == 128 * 8, "one 8-value group per thread");
 
 // ----------------------------------------------------------- epilogues
 // out[(t0 + t) * ldo + m] = rs[m] * y (conv weight norm g / ||w|| per
@@ -232,36 +219,48 @@ __global__ void cx_up_epi_kernel(const float *C, int nc, int t0, float *out) {
   out[(size_t)(2 * (t0 + t) + r) * CD + co] = cx_val<NS>(C, 2 * CD, nc, t, m);
 }
 
-// layer scale + residual (batchedLayerScale, src/shaders.ts:1755-1781):
-// X = y * scale + X.  Grid: (n, CD / 256).
-template <int NS>
-__global__ void cx_resid_epi_kernel(const float *C, int nc, int t0, const uint16_t *scale,
-                                    float *X) {
-  const int t = blockIdx.x, m = blockIdx.y * blockDim.x + threadIdx.x;
-  float *x = X + (size_t)(t0 + t) * CD + m;
-  *x = cx_val<NS>(C, CD, nc, t, m) * h2f(scale[m]) + *x;
-}
-
-// q, k, v from the stacked projection, q and k RMS-normalised per head
-// (qkNorm, src/shaders.ts:1787-1830: weight [CNH * CHDIM] read at h * CHDIM).
-// One wave per (token, part, head); grid (n, 3 * CNH / 4) of 256.
-template <int NS>
-__global__ __launch_bounds__(256) void cx_qkv_epi_kernel(const float *C, int nc, int t0,
-                                                         const uint16_t *qn, const uint16_t *kn,
-                                                         float *Q, float *K, float *V) {
-  const int t = blockIdx.x, gi = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int part = gi / CNH, h = gi - part * CNH, d = 2 * lane;
-  const int m = part * CD + h * CHDIM + d;
-  float y0 = cx_val<NS>(C, 3 * CD, nc, t, m), y1 = cx_val<NS>(C, 3 * CD, nc, t, m + 1);
-  if (part < 2) {
-    const float ss = wave_sum(y0 * y0 + y1 * y1);
-    const float r = 1.0f / sqrtf(ss / (float)CHDIM + CX_QK_EPS);
-    const uint16_t *w = (part == 0 ? qn : kn) + h * CHDIM + d;
-    y0 = y0 * r * h2f(w[0]);
-    y1 = y1 * r * h2f(w[1]);
+// layer scale + residual (batchedLayerScale, src/shaders.ts:1755-1781),
+// X = y * scale + X, and, with PACK, the next GEMM's B from the RMS-normalised
+// row (batchedRmsNorm, src/shaders.ts:1646-1692; zero for t >= n).  The sum
+// of squares needs the whole row, which the block holds: a pack kernel of its
+// own read X again (3.5-5.7 us and a launch per GEMM it fed).
+// Grid: nt blocks (n without PACK) of 128, one 8-value group per thread.
+template <bool PACK, int NS>
+__global__ __launch_bounds__(128) void cx_resid_pack_kernel(const float *C, int nc, int t0, int n,
+                                                            const uint16_t *scale, float *X, const uint16_t *g,
+                                                            float eps, h8 *B) {
+  const int t = blockIdx.x, kb = threadIdx.x;
+  float y[8];
+  if (t < n) {
+    float *x = X + (size_t)(t0 + t) * CD + kb * 8;
+    float xv[8], sc[8];
+    cx_load8(x, xv);
+    cx_load8h(scale + kb * 8, sc);
+    cx_val8<NS>(C, CD, nc, t, kb * 8, y);
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = y[e] * sc[e] + xv[e];
+    *(f32x4 *)x = f32x4{y[0], y[1], y[2], y[3]};
+    *(f32x4 *)(x + 4) = f32x4{y[4], y[5], y[6], y[7]};
   }
-  float *dst = part == 0 ? Q : part == 1 ? K : V;
-  *(float2 *)(dst + (size_t)(t0 + t) * CD + h * CHDIM + d) = make_float2(y0, y1);
+  if (!PACK) return;
+  if (t < n) {
+    __shared__ float red[2];
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) ss = fmaf(y[e], y[e], ss);
+    ss = wave_sum(ss);
+    if ((kb & 63) == 0) red[kb >> 6] = ss;
+    __syncthreads();
+    const float r = 1.0f / sqrtf((red[0] + red[1]) / (float)CD + eps);
+    float gv[8];
+    cx_load8h(g + kb * 8, gv);
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = y[e] * r * gv[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = 0.f;
+  }
+  cx_put(B, nc, CD / 8, kb, t, y);
 }
 
 // SwiGLU of the stacked gate/up projection (batchedSwiGLU,
@@ -285,52 +284,131 @@ __global__ __launch_bounds__(256) void cx_swiglu_epi_kernel(const float *C, int 
 }
 
 // ----------------------------------------------------------- attention
-// Windowed causal attention with ALiBi biases (alibiAttnScore, codecSoftmax,
-// codecAttnValue, src/shaders.ts:1432-1585): keys ki in
-// [max(0, qi - W + 1), qi], score q.k / sqrt(128) - 2^(-8(h+1)/8) (qi - ki).
-// One wave per (query, head), lane l holding dims 2l, 2l + 1.
-// Grid: (T, CNH / 4) of 256; W <= 16.
-constexpr int CX_MAXW = 16;
-__global__ __launch_bounds__(256) void cx_attn_kernel(const float *Q, const float *K,
-                                                      const float *V, int W, float *O) {
-  const int qi = blockIdx.x, h = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const size_t off = (size_t)h * CHDIM + 2 * lane;
-  const float2 q = *(const float2 *)(Q + (size_t)qi * CD + off);
-  const int k0 = qi + 1 > W ? qi - W + 1 : 0;
+// From the stacked q, k, v projection to the O projection's B in one kernel:
+// q and k RMS-normalised per head (qkNorm, src/shaders.ts:1787-1830: weight
+// [CNH * CHDIM] read at h * CHDIM), then windowed causal attention with ALiBi
+// biases (alibiAttnScore, codecSoftmax, codecAttnValue, src/shaders.ts:
+// 1432-1585): keys ki in [max(0, qi - W + 1), qi], score q.k / sqrt(128) -
+// 2^(-8(h+1)/8) (qi - ki), W <= 16.
+// Block = (CXA_T query tokens, head), one wave per query.  The keys of the block's
+// tokens, CXA_T + W - 1 rows at most, are summed over the K slices, normalised
+// and held in LDS (recomputed by the next block: at most 2x of an L2-resident
+// read, where q, k and v written and read again, one wave per query reading W
+// rows each, took 47.7 + 18 us a 2000-token layer, this 2 x 11.1; with four
+// waves a block, eight rows and four queries each in turn, it took 2 x 19).  A wave
+// stages two rows and takes one query: lane 4 j + p scores key k0 + j over the 16-byte
+// chunks 4 i + p of the row, the window's max and sum are 4 lane steps each, and
+// lane l sums dims 2 l, 2 l + 1 of P.V.  LDS rows are 144 floats apart, so
+// the 16 lanes of one read phase (4 keys x 4 chunks) touch distinct banks.
+// Keys before the chunk (t < t0) come from the previous chunk's `halo_in`
+// [CX_HALO][2][CD], normalised k and v; a chunk that has a successor leaves
+// its last CX_HALO rows in halo_out.
+// Grid: (nt / CXA_T, CNH) of 64 CXA_WAVES; B columns t >= n are zero.
+constexpr int CX_MAXW = 16, CX_HALO = CX_MAXW - 1;
+constexpr int CXA_T = 16, CXA_WAVES = CXA_T, CXA_ROWS = CXA_T + CX_HALO, CXA_LD = 144;
+static_assert(CXA_ROWS <= 2 * CXA_WAVES, "two rows per wave");
+template <int NS>
+__global__ __launch_bounds__(64 * CXA_WAVES) void cx_attn_kernel(const float *C, int nc, int t0, int n, int W,
+                                                      const uint16_t *qn, const uint16_t *kn, const float *halo_in,
+                                                      float *halo_out, h8 *B) {
+  __shared__ __attribute__((aligned(16))) float ks[CXA_ROWS * CXA_LD], vs[CXA_ROWS * CXA_LD], qs[CXA_T * CXA_LD];
+  const int tb = blockIdx.x * CXA_T, h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, d = 2 * lane;
+  const int nt = nc >> 1;
+  const int base = tb - (W - 1);  // token of K/V row 0, within the chunk (negative: the chunk before)
+  // q.k / sqrt(128) rows: RMS-normalise the pair (y0, y1) of a row over the wave
+  auto norm = [&](float2 y, const uint16_t *w) {
+    const float r = 1.0f / sqrtf(wave_sum_dpp(y.x * y.x + y.y * y.y) / (float)CHDIM + CX_QK_EPS);
+    return make_float2(y.x * r * h2f(w[h * CHDIM + d]), y.y * r * h2f(w[h * CHDIM + d + 1]));
+  };
+  auto row = [&](int t, int part) {
+    const int m = part * CD + h * CHDIM + d;
+    float2 v[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) v[s] = *(const float2 *)(C + ((size_t)s * nt + t) * (3 * CD) + m);
+    float2 y = v[0];
+#pragma unroll
+    for (int s = 1; s < NS; s++) {
+      y.x += v[s].x;
+      y.y += v[s].y;
+    }
+    return y;
+  };
+  // rows i and i + CXA_WAVES of every wave, all loads ahead of the first use;
+  // t past the chunk's tokens re-reads the last, t before it the halo
+  float2 k[2], v[2], q[2];
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int i = wave + CXA_WAVES * u, t = base + i;
+    if (t >= 0) {
+      const int tc = min(t, n - 1);
+      k[u] = row(tc, 1);
+      v[u] = row(tc, 2);
+      q[u] = row(tc, 0);
+    } else if (t0 + t >= 0 && i < W - 1) {
+      const float *p = halo_in + (size_t)(t + CX_HALO) * 2 * CD + h * CHDIM + d;
+      k[u] = *(const float2 *)p;
+      v[u] = *(const float2 *)(p + CD);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int i = wave + CXA_WAVES * u, t = base + i;
+    if (i >= CXA_T + W - 1 || t >= n || t0 + t < 0) continue;  // no such row, or never in a window
+    if (t >= 0) k[u] = norm(k[u], kn);
+    *(float2 *)(ks + i * CXA_LD + d) = k[u];
+    *(float2 *)(vs + i * CXA_LD + d) = v[u];
+    if (t < tb) continue;
+    *(float2 *)(qs + (t - tb) * CXA_LD + d) = norm(q[u], qn);
+    if (halo_out && t >= n - CX_HALO) {  // each row by the block that owns the token
+      float *o = halo_out + (size_t)(t - (n - CX_HALO)) * 2 * CD + h * CHDIM + d;
+      *(float2 *)o = k[u];
+      *(float2 *)(o + CD) = v[u];
+    }
+  }
+  __syncthreads();
   const float scale = 1.0f / sqrtf((float)CHDIM);
   const float slope = exp2f(-8.0f * (float)(h + 1) / (float)CNH);
-  float s[CX_MAXW];
-  float mx = -1e30f;
+  const int j = lane >> 2, p = lane & 3;
+  {
+    const int qi = wave, t = tb + qi;
+    if (t >= nt) return;
+    float2 o = make_float2(0.f, 0.f);
+    if (t < n) {
+      const int key = t - W + 1 + j;                    // this lane's key, LDS row qi + j
+      const bool in = j < W && t0 + key >= 0;
+      const float *kr = ks + (in ? qi + j : qi + W - 1) * CXA_LD + 4 * p, *qr = qs + qi * CXA_LD + 4 * p;
+      float dot = 0.f;
 #pragma unroll
-  for (int j = 0; j < CX_MAXW; j++) {
-    float sc = -1e30f;
-    const int ki = k0 + j;
-    if (j < W && ki <= qi) {
-      const float2 k = *(const float2 *)(K + (size_t)ki * CD + off);
-      const float dot = wave_sum(q.x * k.x + q.y * k.y);
-      sc = dot * scale + (-slope * (float)(qi - ki));
+      for (int i = 0; i < CHDIM / 16; i++) {
+        const f32x4 a = *(const f32x4 *)(qr + 16 * i), b = *(const f32x4 *)(kr + 16 * i);
+#pragma unroll
+        for (int e = 0; e < 4; e++) dot = fmaf(a[e], b[e], dot);
+      }
+      dot += __shfl_xor(dot, 1, 64);
+      dot += __shfl_xor(dot, 2, 64);
+      const float sc = in ? dot * scale - slope * (float)(t - key) : -INFINITY;
+      float mx = sc;
+#pragma unroll
+      for (int x = 4; x < 64; x <<= 1) mx = fmaxf(mx, __shfl_xor(mx, x, 64));
+      const float e = in ? expf(sc - mx) : 0.f;  // the query's own key is always in: mx is finite
+      float sum = e;
+#pragma unroll
+      for (int x = 4; x < 64; x <<= 1) sum += __shfl_xor(sum, x, 64);
+      const float pr = e / sum;
+      for (int jj = 0; jj < W; jj++) {
+        if (t0 + t - W + 1 + jj < 0) continue;
+        const float pj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pr), 4 * jj));
+        const float2 v = *(const float2 *)(vs + (qi + jj) * CXA_LD + d);
+        o.x = fmaf(pj, v.x, o.x);
+        o.y = fmaf(pj, v.y, o.y);
+      }
     }
-    s[j] = sc;
-    if (j < W) mx = fmaxf(mx, sc);
+    h2 hi, lo;
+    split2(o.x, o.y, hi, lo);
+    _Float16 *b = (_Float16 *)B + h * CHDIM + d;
+    *(h2 *)(b + (size_t)t * CD) = hi;
+    *(h2 *)(b + (size_t)(nt + t) * CD) = lo;
   }
-  float sum = 0.f;
-#pragma unroll
-  for (int j = 0; j < CX_MAXW; j++) {
-    s[j] = j < W ? expf(s[j] - mx) : 0.f;
-    sum += s[j];
-  }
-  float2 o = make_float2(0.f, 0.f);
-#pragma unroll
-  for (int j = 0; j < CX_MAXW; j++) {
-    const int ki = k0 + j;
-    if (j < W && ki <= qi) {
-      const float p = s[j] / sum;
-      const float2 v = *(const float2 *)(V + (size_t)ki * CD + off);
-      o.x += p * v.x;
-      o.y += p * v.y;
-    }
-  }
-  *(float2 *)(O + (size_t)qi * CD + off) = o;
 }
 
 // the concatenated input features [T][292] (debugCodecDecode's "concat")
@@ -418,13 +496,14 @@ __global__ void cx_reorder_out_kernel(const uint16_t *w, uint16_t *A) {
   }
 }
 
-// A of a transposed conv: [2 * CD][CKUP], A[r * CD + co][j * CD + ci] =
-// w[ci][co][r + 2 j] (w is [c_in][c_out][4])
+// A of a transposed conv: [2 * CD][CKUP], A[r * CD + co][(1 - j) * CD + ci] =
+// w[ci][co][r + 2 j] (w is [c_in][c_out][4]; j = 1 is the step before, whose
+// packed row comes first)
 __global__ void cx_reorder_up_kernel(const uint16_t *w, uint16_t *A) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < (size_t)2 * CD * CKUP;
        i += (size_t)gridDim.x * blockDim.x) {
     const int row = (int)(i / CKUP), k = (int)(i % CKUP);
-    const int r = row / CD, co = row - r * CD, j = k / CD, ci = k - j * CD;
+    const int r = row / CD, co = row - r * CD, j = 1 - k / CD, ci = k % CD;
     A[i] = w[((size_t)ci * CD + co) * CK_UP + r + 2 * j];
   }
 }

@@ -151,8 +151,7 @@ struct vx_engine {
   float *cx_rs_in = nullptr, *cx_rs_out = nullptr, *cx_s_up[CX_STAGES - 1] = {};
   void *cx_arena = nullptr;
   int cx_cap = 0;
-  float *cx_x = nullptr, *cx_x2 = nullptr, *cx_q = nullptr, *cx_k = nullptr, *cx_v = nullptr,
-        *cx_attn = nullptr, *cx_c = nullptr, *cx_audio = nullptr;
+  float *cx_x = nullptr, *cx_x2 = nullptr, *cx_halo = nullptr, *cx_c = nullptr, *cx_audio = nullptr;
   h8 *cx_b = nullptr;
   uint32_t *cx_sem = nullptr, *cx_ac = nullptr;
   int cx_chunk = CX_MAXT;  // tokens per codec GEMM chunk (multiple of 128)
@@ -1601,15 +1600,18 @@ static int pf_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nt, int n,
     return fail(e, VX_E_STATE, "prefill GEMM plan with %d slices", p.slices);
   if ((size_t)p.slices * nt * M > (size_t)PF_NC * 2 * HID)
     return fail(e, VX_E_STATE, "prefill GEMM output (%d slices of %d x %d) exceeds its buffer", p.slices, nt, M);
-  gemm_launch(p, e->st, W, M, K, (const uint16_t *)e->pf_b, nt, n, e->pf_c);
+  gemm_launch(p, e->st, W, M, K, (const uint16_t *)e->pf_b, K, (size_t)nt * K, nt, n, e->pf_c);
   *ns = p.slices;
   return VX_OK;
 }
 
 // cx_c[s][col][m] for s < *ns: the codec chunk's K-slice partial sums of
-// W[M][K] x cx_b (nc = 2 nt rows of K halves)
-static int cx_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nc, int n, int *ns) {
-  const int nt = nc / 2;
+// W[M][K] x cx_b: nc = 2 nt rows of K halves or, with `rows` > 0, columns that
+// overlap in packed rows of CD halves (column t starts at row t; rows hi, then
+// rows lo)
+static int cx_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nc, int n, int *ns, int rows = 0) {
+  const int nt = nc / 2, ldb = rows ? CD : K;
+  const size_t blo = (size_t)(rows ? rows : nt) * ldb;
   if (M % GM_BM || K % GM_BK || n < 1 || nt != gm_cols(n))
     return fail(e, VX_E_STATE, "codec GEMM shape M %d K %d nt %d", M, K, nt);
   const GemmPlan p = gemm_plan(M, K, nt, e->cus);
@@ -1617,7 +1619,7 @@ static int cx_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nc, int n,
     return fail(e, VX_E_STATE, "codec GEMM plan with %d slices", p.slices);
   if ((size_t)p.slices * nt * M > CX_CCAP)
     return fail(e, VX_E_STATE, "codec GEMM output (%d slices of %d x %d) exceeds its buffer", p.slices, nt, M);
-  gemm_launch(p, e->st, W, M, K, (const uint16_t *)e->cx_b, nt, n, e->cx_c);
+  gemm_launch(p, e->st, W, M, K, (const uint16_t *)e->cx_b, ldb, blo, nt, n, e->cx_c);
   *ns = p.slices;
   return VX_OK;
 }
@@ -1878,13 +1880,10 @@ static int codec_reserve(vx_engine *e, int T) {
   std::vector<std::pair<void **, size_t>> parts = {
       {(void **)&e->cx_x, TT * CD * 4},
       {(void **)&e->cx_x2, TT * CD * 4},
-      {(void **)&e->cx_q, TT * CD * 4},
-      {(void **)&e->cx_k, TT * CD * 4},
-      {(void **)&e->cx_v, TT * CD * 4},
-      {(void **)&e->cx_attn, TT * CD * 4},
+      {(void **)&e->cx_halo, (size_t)CX_LPS * 2 * CX_HALO * 2 * CD * 4},
       {(void **)&e->cx_audio, TT * CPATCH * 4},
       {(void **)&e->cx_c, CX_CCAP * 4},
-      {(void **)&e->cx_b, (size_t)CKOUT / 8 * CX_NC * 16},
+      {(void **)&e->cx_b, (size_t)CHID / 8 * CX_NC * 16},
       {(void **)&e->cx_sem, (size_t)T * 4},
       {(void **)&e->cx_ac, (size_t)T * NAC * 4}};
   size_t tot = 0;
@@ -1945,34 +1944,30 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
   float *x = e->cx_x, *x2 = e->cx_x2;
   static const int kWindow[CX_STAGES] = {2, 4, 8, 16};  // src/engine.ts:1507
   for (int s = 0; s < CX_STAGES && at < stop; s++) {
-    for (int l = 0; l < CX_LPS; l++) {
-      const CodecLayerW &L = w.L[s][l];
-      chunks(TT, [&](int t0, int n, int nc) {
-        hipLaunchKernelGGL(cx_pack_kernel<true>, dim3(nc / 2), blk, 0, st, x, CD, t0, n, nc,
-                           L.attn_norm, CX_NORM_EPS, e->cx_b);
+    // a chunk runs both layers before the next chunk starts: what a later
+    // chunk needs of it, the last keys and values of each layer, is its halo
+    // (two per layer, written and read in turn)
+    int parity = 0;
+    chunks(TT, [&](int t0, int n, int nc) {
+      hipLaunchKernelGGL(cx_pack_kernel, dim3(nc / 2), blk, 0, st, x, CD, t0, n, nc, w.L[s][0].attn_norm,
+                         CX_NORM_EPS, e->cx_b);
+      for (int l = 0; l < CX_LPS; l++) {
+        const CodecLayerW &L = w.L[s][l];
+        const size_t halo = (size_t)CX_HALO * 2 * CD;
+        const float *halo_in = e->cx_halo + (2 * l + (parity ^ 1)) * halo;
+        float *halo_out = t0 + n < TT ? e->cx_halo + (2 * l + parity) * halo : nullptr;
         int ns = 1;
         if (!rc) rc = cx_gemm(e, L.wqkv, 3 * CD, CD, nc, n, &ns);
         gm_with_slices(ns, [&](auto NS) {
-          hipLaunchKernelGGL(cx_qkv_epi_kernel<NS>, dim3(n, 3 * CNH / 4), blk, 0, st, e->cx_c, nc, t0,
-                             L.q_norm, L.k_norm, e->cx_q, e->cx_k, e->cx_v);
+          hipLaunchKernelGGL(cx_attn_kernel<NS>, dim3(nc / 2 / CXA_T, CNH), dim3(64 * CXA_WAVES), 0, st,
+                             e->cx_c, nc,
+                             t0, n, kWindow[s], L.q_norm, L.k_norm, halo_in, halo_out, e->cx_b);
         });
-      });
-      hipLaunchKernelGGL(cx_attn_kernel, dim3(TT, CNH / 4), blk, 0, st, e->cx_q, e->cx_k, e->cx_v,
-                         kWindow[s], e->cx_attn);
-      chunks(TT, [&](int t0, int n, int nc) {
-        hipLaunchKernelGGL(cx_pack_kernel<false>, dim3(nc / 2), blk, 0, st, e->cx_attn, CD, t0, n,
-                           nc, nullptr, 0.f, e->cx_b);
-        int ns = 1;
         if (!rc) rc = cx_gemm(e, L.wo, CD, CD, nc, n, &ns);
         gm_with_slices(ns, [&](auto NS) {
-          hipLaunchKernelGGL(cx_resid_epi_kernel<NS>, dim3(n, CD / 256), blk, 0, st, e->cx_c, nc, t0,
-                             L.attn_scale, x);
+          hipLaunchKernelGGL((cx_resid_pack_kernel<true, NS>), dim3(nc / 2), dim3(128), 0, st, e->cx_c, nc, t0, n,
+                             L.attn_scale, x, L.ffn_norm, CX_NORM_EPS, e->cx_b);
         });
-      });
-      chunks(TT, [&](int t0, int n, int nc) {
-        hipLaunchKernelGGL(cx_pack_kernel<true>, dim3(nc / 2), blk, 0, st, x, CD, t0, n, nc,
-                           L.ffn_norm, CX_NORM_EPS, e->cx_b);
-        int ns = 1;
         if (!rc) rc = cx_gemm(e, L.w13, 2 * CHID, CD, nc, n, &ns);
         // the gate/up GEMM has consumed B: the SwiGLU epilogue refills it
         gm_with_slices(ns, [&](auto NS) {
@@ -1981,19 +1976,25 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
         });
         if (!rc) rc = cx_gemm(e, L.w2, CD, CHID, nc, n, &ns);
         gm_with_slices(ns, [&](auto NS) {
-          hipLaunchKernelGGL(cx_resid_epi_kernel<NS>, dim3(n, CD / 256), blk, 0, st, e->cx_c, nc, t0,
-                             L.ffn_scale, x);
+          if (l + 1 < CX_LPS)
+            hipLaunchKernelGGL((cx_resid_pack_kernel<true, NS>), dim3(nc / 2), dim3(128), 0, st, e->cx_c, nc, t0,
+                               n, L.ffn_scale, x, w.L[s][l + 1].attn_norm, CX_NORM_EPS, e->cx_b);
+          else
+            hipLaunchKernelGGL((cx_resid_pack_kernel<false, NS>), dim3(n), dim3(128), 0, st, e->cx_c, nc, t0, n,
+                               L.ffn_scale, x, nullptr, 0.f, nullptr);
         });
-      });
-    }
+      }
+      parity ^= 1;
+    });
     at = VX_CODEC_STOP_STAGE0 + 2 * s;
     if (at == stop || s == CX_STAGES - 1) break;
     // ConvTranspose1d(1024 -> 1024, k = 4, stride 2), output trimmed to 2 TT
     chunks(TT, [&](int t0, int n, int nc) {
-      hipLaunchKernelGGL(cx_pack_up_kernel, dim3(nc / 2), blk, 0, st, x, e->cx_s_up[s], t0, n, nc,
-                         e->cx_b);
+      const int rows = nc / 2 + 1;
+      hipLaunchKernelGGL(cx_pack_rows_kernel, dim3(rows), dim3(128), 0, st, x, e->cx_s_up[s], 1, t0, n,
+                         (size_t)rows * CD, e->cx_b);
       int ns = 1;
-      if (!rc) rc = cx_gemm(e, e->cx_aup[s], 2 * CD, CKUP, nc, n, &ns);
+      if (!rc) rc = cx_gemm(e, e->cx_aup[s], 2 * CD, CKUP, nc, n, &ns, rows);
       gm_with_slices(ns, [&](auto NS) {
         hipLaunchKernelGGL(cx_up_epi_kernel<NS>, dim3(n, 2 * CD / 256), blk, 0, st, e->cx_c, nc, t0, x2);
       });
@@ -2011,9 +2012,11 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
   // output conv: CausalConv1d(1024 -> 240, k = 7); step t gives samples
   // [240 t, 240 t + 240)
   chunks(TT, [&](int t0, int n, int nc) {
-    hipLaunchKernelGGL(cx_pack_out_kernel, dim3(nc / 2), blk, 0, st, x, t0, n, nc, e->cx_b);
+    const int rows = nc / 2 + CK_OUT - 1;
+    hipLaunchKernelGGL(cx_pack_rows_kernel, dim3(rows), dim3(128), 0, st, x, (const float *)nullptr, CK_OUT - 1, t0,
+                       n, (size_t)rows * CD, e->cx_b);
     int ns = 1;
-    if (!rc) rc = cx_gemm(e, e->cx_aout, CPATCH_ROWS, CKOUT, nc, n, &ns);
+    if (!rc) rc = cx_gemm(e, e->cx_aout, CPATCH_ROWS, CKOUT, nc, n, &ns, rows);
     gm_with_slices(ns, [&](auto NS) {
       hipLaunchKernelGGL(cx_scale_rows_epi_kernel<NS>, dim3(n, 1), blk, 0, st, e->cx_c, CPATCH_ROWS, nc,
                          t0, e->cx_rs_out, CPATCH, e->cx_audio, CPATCH);

@@ -1,9 +1,11 @@
 // vx_gemm.h -- the prefill's projections as hand-written gfx950 MFMA GEMMs:
 //   C[s][col][m] = sum_{k in slice s} W[m][k] * (Bhi[col][k] + Blo[col][k])
 // W: f16 weights, row-major M x K as loaded (the decode GEMVs read the same
-// copy).  B: 2 nt rows of K halves, the hi half of each activation column in
-// row col and its f16 residual (lo) in row nt + col, as the prefill's
-// producer kernels write them.  Hi and lo go through the same MFMA
+// copy).  B: the hi half of activation column col is K halves from
+// B + col ldb, its f16 residual (lo) from B + blo + col ldb (16-byte
+// aligned), as the producer kernels write them.  ldb = K for packed
+// columns; a causal convolution's columns overlap (ldb = channels, K = taps x
+// channels), so its input is packed once and not once per tap.  Hi and lo go through the same MFMA
 // accumulator, so the product keeps f32 accuracy.  The K range is split
 // into S_out slices whose partial sums land in S_out consecutive [nt][M]
 // blocks of C; the consumer adds them (fixed order, so results are
@@ -204,8 +206,8 @@ __device__ __forceinline__ void gm_iteration(const GmLane &L, unsigned char *sme
 // slice s of KS = gridDim.y (K / 64 k-tiles in KS near-equal runs) and writes
 // C block s.  Needs M % 256 == 0, nt % 64 == 0, K % 64 == 0, KS <= K / 64.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_split_kernel(
-    const uint16_t *__restrict__ W, int M, int K, const uint16_t *__restrict__ B, int nt, float *__restrict__ C,
-    int ldc) {
+    const uint16_t *__restrict__ W, int M, int K, const uint16_t *__restrict__ B, int ldb, size_t blo, int nt,
+    float *__restrict__ C, int ldc) {
   extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
   const GmLane L(threadIdx.x);
   const int n_tiles = nt / GM_BN, m_tiles = M / GM_BM;
@@ -232,7 +234,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       base[i] = W + (size_t)(mt * GM_BM + row) * K + kb + chunk * 8;
     } else {
       const int br = row - GM_BM, hl = br / GM_BN, col = br % GM_BN;
-      base[i] = B + (size_t)(hl * nt + ntl * GM_BN + col) * K + kb + chunk * 8;
+      base[i] = B + hl * blo + (size_t)(ntl * GM_BN + col) * ldb + kb + chunk * 8;
     }
   }
   gm_f32x16 acc[2][2];
@@ -270,8 +272,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // b % 8 (one XCD, as workgroups are dealt to the XCDs round-robin) hold
 // whole shares, so one L2 serves them.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_stream_kernel(
-    const uint16_t *__restrict__ W, int M, int K, const uint16_t *__restrict__ B, int nt, float *__restrict__ C,
-    int ldc, int Lshare, int ns) {
+    const uint16_t *__restrict__ W, int M, int K, const uint16_t *__restrict__ B, int ldb, size_t blo, int nt,
+    float *__restrict__ C, int ldc, int Lshare, int ns) {
   extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
   const GmLane L(threadIdx.x);
   const int n_tiles = nt / GM_BN, m_tiles = M / GM_BM, nk = K / GM_BK;
@@ -292,7 +294,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       off[i] = (size_t)row * K + chunk * 8;
     } else {
       const int br = row - GM_BM, hl = br / GM_BN, col = br % GM_BN;
-      off[i] = (size_t)(hl * nt + c * GM_BN + col) * K + chunk * 8;
+      off[i] = hl * blo + (size_t)(c * GM_BN + col) * ldb + chunk * 8;
     }
   }
   gm_f32x16 acc[2][2];
@@ -419,8 +421,8 @@ __device__ __forceinline__ void gt_direct(const uint16_t *src, unsigned char *ld
 
 template <int RT, int NT, bool NTW>
 __global__ __launch_bounds__(256) void gemm_thin_kernel(const uint16_t *__restrict__ W, int K,
-                                                        const uint16_t *__restrict__ B, int n,
-                                                        float *__restrict__ C, int ldc) {
+                                                        const uint16_t *__restrict__ B, int ldb, size_t blo,
+                                                        int n, float *__restrict__ C, int ldc) {
   using G = GtShape<RT, NT>;
   constexpr int S = G::S;
   extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
@@ -433,7 +435,8 @@ __global__ __launch_bounds__(256) void gemm_thin_kernel(const uint16_t *__restri
 #pragma unroll
   for (int i = 0; i < G::LOADS; i++) {
     const int row = 8 * (4 * i + wave) + (lane >> 3), chunk = (lane & 7) ^ gm_key(row);
-    src[i] = (i < RT ? W + (size_t)(m0 + row) * K : B + (size_t)(row - G::BM) * K) + k0 * GM_BK + chunk * 8;
+    const int br = row - G::BM, hl = br >= NT ? 1 : 0;  // i >= RT
+    src[i] = (i < RT ? W + (size_t)(m0 + row) * K : B + hl * blo + (size_t)(br - hl * NT) * ldb) + k0 * GM_BK + chunk * 8;
   }
   auto issue = [&](int stage) {
 #pragma unroll
@@ -645,17 +648,17 @@ inline hipError_t gemm_setup() {
 // codec's matrices (2-17 MB, 298 MB in all) stay allocating, so that a
 // decode of a few frames finds part of them in the 256 MB last-level cache.
 inline void gemm_launch(const GemmPlan &p, hipStream_t st, const uint16_t *W, int M, int K, const uint16_t *B,
-                        int nt, int n, float *C) {
+                        int ldb, size_t blo, int nt, int n, float *C) {
   if (p.thin)
     gm_with_thin(p.thin, nt, (size_t)M * K >= (size_t)8 << 20, [&](auto kernel, int lds) {
-      hipLaunchKernelGGL(kernel, dim3(M / (32 * p.thin), p.ks), dim3(256), lds, st, W, K, B, n, C, M);
+      hipLaunchKernelGGL(kernel, dim3(M / (32 * p.thin), p.ks), dim3(256), lds, st, W, K, B, ldb, blo, n, C, M);
     });
   else if (p.stream)
-    hipLaunchKernelGGL(gemm_stream_kernel, dim3(p.grid), dim3(256), GM_LDS, st, W, M, K, B, nt, C, M, p.share,
-                       p.slices);
+    hipLaunchKernelGGL(gemm_stream_kernel, dim3(p.grid), dim3(256), GM_LDS, st, W, M, K, B, ldb, blo, nt, C, M,
+                       p.share, p.slices);
   else
     hipLaunchKernelGGL(gemm_split_kernel, dim3((M / GM_BM) * (nt / GM_BN), p.ks), dim3(256), GM_LDS, st, W, M, K,
-                       B, nt, C, M);
+                       B, ldb, blo, nt, C, M);
 }
 
 }  // namespace vx
