@@ -1595,7 +1595,7 @@ static int pf_gemm_setup(vx_engine *e) {
 static int pf_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nt, int n, int *ns) {
   if (M % GM_BM || K % GM_BK || n < 1 || nt != gm_cols(n))
     return fail(e, VX_E_STATE, "prefill GEMM shape M %d K %d nt %d", M, K, nt);
-  const GemmPlan p = gemm_plan(M, K, nt, e->cus);
+  const GemmPlan p = gemm_plan(M, K, nt, e->cus, (size_t)PF_NC * 2 * HID);
   if (p.slices < 1 || p.slices > 8)
     return fail(e, VX_E_STATE, "prefill GEMM plan with %d slices", p.slices);
   if ((size_t)p.slices * nt * M > (size_t)PF_NC * 2 * HID)
@@ -1614,7 +1614,7 @@ static int cx_gemm(vx_engine *e, const uint16_t *W, int M, int K, int nc, int n,
   const size_t blo = (size_t)(rows ? rows : nt) * ldb;
   if (M % GM_BM || K % GM_BK || n < 1 || nt != gm_cols(n))
     return fail(e, VX_E_STATE, "codec GEMM shape M %d K %d nt %d", M, K, nt);
-  const GemmPlan p = gemm_plan(M, K, nt, e->cus);
+  const GemmPlan p = gemm_plan(M, K, nt, e->cus, CX_CCAP);
   if (p.slices < 1 || p.slices > 8)
     return fail(e, VX_E_STATE, "codec GEMM plan with %d slices", p.slices);
   if ((size_t)p.slices * nt * M > CX_CCAP)

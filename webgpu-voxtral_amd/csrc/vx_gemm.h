@@ -11,27 +11,35 @@
 // blocks of C; the consumer adds them (fixed order, so results are
 // deterministic).
 //
-// Tile: 256 weight rows x 64 columns (128 B rows: 64 hi + 64 lo) per block
-// of 4 waves; wave w owns weight rows 64 w .. + 64 and all 128 B rows, as
-// 2 x 2 tiles of v_mfma_f32_32x32x16_f16 (hi and lo accumulate into the
-// same tile).  A k-tile is 64 halves: 256 + 128 rows of 128 B = 48 KB of
-// LDS, filled by direct global->LDS loads (global_load_lds_dwordx4, 1 KB per
-// instruction = 8 rows) into a ring of 3 stages (144 KB).  Per k-tile a wave
-// issues 32 MFMAs, 24 ds_read_b128 and 12 direct loads; the schedule
-// interleaves them (MFMA, read, load, MFMA, read ...) so that neither the
-// LDS reads nor the loads' issue stall the matrix pipe, reads of step q + 1
-// run under the MFMAs of step q, and the stage barrier sits before the last
-// step so the next stage's first fragments are read under it.
+// Tiles: 256 weight rows x CN columns (2 CN B rows: hi and lo) per block of
+// eight waves.  Four compute: wave w owns 32 RT weight rows and 64 columns, as
+// RT x 2 tiles of v_mfma_f32_32x32x16_f16 (hi and lo accumulate into the same
+// tile).  Four load: a k-tile is 64 halves, 128 bytes of each of the 256 + 2 CN
+// rows, brought to LDS by direct loads (global_load_lds_dwordx4, 1 KB per
+// instruction = 8 rows) into a ring of DA weight stages and DB stages of B.
 //
-// Two grids:
-//  - gemm_split_kernel: one tile per block, K split in KS = gridDim.y
-//    slices (S_out = KS); for shapes with at most one block per CU.
-//  - gemm_stream_kernel: one block per CU, each doing an equal share of the
-//    column tile's (row tile, k-tile) sequence; S_out = the most blocks a
-//    tile is split over (rounded up to 1, 2, 4 or 8); for shapes with more
-//    tiles than CUs, which would otherwise run in uneven rounds.
+// What bounds it is the operands' way to the matrix cores, and power.  The
+// 256 x 64 tile's 48 KB of direct loads per k-tile alone take 1180 clocks (41
+// bytes a clock and CU) against 1024 of MFMA; issued by the computing waves
+// (an earlier form) each also held up its wave's MFMAs by 35-41 clocks: 1500
+// clocks a k-tile, 2970 for the 256 x 128 tile, whose MFMAs take 2048.  Hence
+// loaders of their own: four, as one wave issues a direct load only every 60
+// clocks (a single loader took 1.69 us per 256 x 128 k-tile, four 1.25, the
+// computing waves 1.32).  Under full load the clock falls to 1.5 GHz, so bytes
+// moved count twice: the 256 x 128 tile moves 64 KB for twice the MFMAs of the
+// 256 x 64 tile's 48 KB and reads 8 fragments for 16 MFMAs, not 6 for 8.
+// Issued rates at 1024 columns: gate/up (18432 x 3072) 0.91 PFLOP/s, QKV 0.89,
+// where one 8192^3 f16 product of the vendor library reaches 1.18 on this card.
+//
+// A block works through k-tiles g0 .. g1 - 1 of one column tile's sequence
+// g = mt nk + kt.  Two ways to cut it:
+//  - K slices: one tile per block, K split in KS slices (S_out = KS);
+//  - shares: every block an equal share of its column tile's sequence; S_out =
+//    the most blocks a tile is split over (1 .. 8); for shapes with more tiles
+//    than CUs, which would otherwise run in uneven rounds.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 
@@ -41,14 +49,10 @@ typedef _Float16 gm_h8 __attribute__((ext_vector_type(8)));
 typedef float gm_f32x4 __attribute__((ext_vector_type(4)));
 typedef float gm_f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int GM_BM = 256;                 // weight rows per tile
-constexpr int GM_BN = 64;                  // activation columns per tile
-constexpr int GM_BK = 64;                  // halves per k-tile
-constexpr int GM_ROWB = 128;               // bytes per LDS row (one k-tile of one row)
-constexpr int GM_STAGE = (GM_BM + 2 * GM_BN) * GM_ROWB;  // 48 KB
-constexpr int GM_S = 3;                    // stages in the LDS ring
-constexpr int GM_LDS = GM_S * GM_STAGE;    // 144 KB
-constexpr int GM_LOADS = 12;               // direct loads per wave per k-tile
+constexpr int GM_BM = 256;   // weight rows per tile
+constexpr int GM_BN = 64;    // columns of the narrow tile, and of a compute wave
+constexpr int GM_BK = 64;    // halves per k-tile
+constexpr int GM_ROWB = 128; // bytes per LDS row (one k-tile of one row)
 
 // s_waitcnt immediate for vmcnt(vm) with the other counters left open
 constexpr int gm_vmcnt(int vm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (15 << 8); }
@@ -58,81 +62,43 @@ constexpr int GM_LGKM0 = 0xC07F;  // lgkmcnt(0)
 // 32 rows one fragment read touches spread over the banks
 __device__ __forceinline__ int gm_key(int row) { return (row >> 1) & 7; }
 
-// The k-tile pipeline shared by both grids.  State: fragment registers,
-// accumulators, per-lane LDS offsets; the caller supplies the source of each
-// k-tile's loads.
-struct GmLane {
-  int lane, wave, r, h;
-  int roff[6], rkey[6];  // LDS row offset and key of fragment f (A: f < 2, B: 2 + 2 hl + j)
-  __device__ __forceinline__ GmLane(int tid) {
-    lane = tid & 63;
-    wave = tid >> 6;
-    r = lane & 31;
-    h = lane >> 5;
-#pragma unroll
-    for (int f = 0; f < 6; f++) {
-      const int row = f < 2 ? wave * 64 + f * 32 + r : GM_BM + ((f - 2) >> 1) * GM_BN + ((f - 2) & 1) * 32 + r;
-      roff[f] = row * GM_ROWB;
-      rkey[f] = gm_key(row);
-    }
-  }
-  // direct load i of this wave fills stage row 8 (4 i + w) + lane / 8
-  // (i < 8: weight rows, else B rows), position lane % 8, which holds chunk
-  // (lane % 8) ^ key(row)
-  __device__ __forceinline__ int load_row(int i) const { return 8 * (4 * i + wave) + (lane >> 3); }
-  __device__ __forceinline__ int load_chunk(int i) const { return (lane & 7) ^ gm_key(load_row(i)); }
-};
-
 __device__ __forceinline__ void gm_direct(const uint16_t *src, unsigned char *lds_row_block) {
   __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)lds_row_block, 16,
                                    0, 0);
 }
 
-__device__ __forceinline__ void gm_read(const GmLane &L, const unsigned char *stage, int q, gm_h8 (&fr)[6]) {
-  const int c = 2 * q + L.h;
-#pragma unroll
-  for (int f = 0; f < 6; f++) fr[f] = *(const gm_h8 *)(stage + L.roff[f] + ((c ^ L.rkey[f]) << 4));
-}
+// One tile shape: RT 32-row tiles and one of WC 64-column groups per compute
+// wave, rings of DA weight stages and DB stages of B.
+template <int RT_, int WC_, int DA_, int DB_>
+struct GmShape {
+  static constexpr int RT = RT_, WC = WC_, DA = DA_, DB = DB_;
+  static constexpr int CN = GM_BN * WC;               // columns per tile
+  static constexpr int ASTAGE = GM_BM * GM_ROWB;      // 32 KB
+  static constexpr int BSTAGE = 2 * CN * GM_ROWB;     // 16 KB per 64 columns
+  static constexpr int NA = GM_BM / 32, NB = 2 * CN / 32;  // direct loads per loader wave and stage
+  static constexpr int LDS = DA * ASTAGE + DB * BSTAGE;
+  static_assert(32 * RT * 4 / WC == GM_BM && DA == 3 && (DB == 2 || DB == 3), "tile");
+};
+using GmNarrow = GmShape<2, 1, 3, 3>;  // 256 x 64, 144 KB
+using GmWide = GmShape<4, 2, 3, 2>;    // 256 x 128, 160 KB: the weights, which come from HBM, two k-tiles ahead
 
-__device__ __forceinline__ void gm_mfma(gm_f32x16 (&acc)[2][2], const gm_h8 (&fr)[6]) {
+template <int RT>
+__device__ __forceinline__ void gm_mfma(gm_f32x16 (&acc)[RT][2], const gm_h8 (&fr)[RT + 4]) {
 #pragma unroll
   for (int hl = 0; hl < 2; hl++)
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < RT; i++)
 #pragma unroll
       for (int j = 0; j < 2; j++)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[i], fr[2 + 2 * hl + j], acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[i], fr[RT + 2 * hl + j], acc[i][j], 0, 0, 0);
 }
 
-// 8 MFMAs, 6 LDS reads, 3 direct loads: M R L M R  M R L M R  M R L M R  M M
-__device__ __forceinline__ void gm_interleave() {
+// acc[i][j][e] is weight row 32 i + 8 (e / 4) + 4 h + e % 4 of the wave's,
+// column 32 j + r: written as C[col][m] with float4 stores
+template <int RT>
+__device__ __forceinline__ void gm_store(const gm_f32x16 (&acc)[RT][2], float *cp, int ldc, bool zero) {
 #pragma unroll
-  for (int k = 0; k < 3; k++) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-  }
-  __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-}
-
-__device__ __forceinline__ void gm_zero(gm_f32x16 (&acc)[2][2]) {
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
-}
-
-// acc[i][j][e] is weight row 64 w + 32 i + 8 (e / 4) + 4 h + e % 4 of the
-// tile, column 32 j + r: written as C[col][m] with float4 stores
-__device__ __forceinline__ void gm_store(const GmLane &L, const gm_f32x16 (&acc)[2][2], float *C, int ldc, int col0,
-                                         int m0, bool zero) {
-  float *cp = C + (size_t)(col0 + L.r) * ldc + m0 + L.wave * 64 + 4 * L.h;
-#pragma unroll
-  for (int i = 0; i < 2; i++)
+  for (int i = 0; i < RT; i++)
 #pragma unroll
     for (int j = 0; j < 2; j++)
 #pragma unroll
@@ -142,230 +108,172 @@ __device__ __forceinline__ void gm_store(const GmLane &L, const gm_f32x16 (&acc)
                  : gm_f32x4{acc[i][j][4 * g4], acc[i][j][4 * g4 + 1], acc[i][j][4 * g4 + 2], acc[i][j][4 * g4 + 3]};
 }
 
-// One k-tile iteration t of the pipeline.  Stage `stage` holds k-tile t,
-// stage nxt k-tile t + 1 (in flight); f0 holds step 0's fragments.  The 12
-// direct loads of the pending k-tile (the one the previous iteration's
-// barrier freed a stage for) are finished in steps 0-2 (loads 3-11, unless
-// FIRST: none pending yet), then after this iteration's barrier a new
-// k-tile's loads 0-2 go out in step 3 (`next_src` switches the source).
-// Each k-tile's 12 loads stay contiguous in issue order, so at the barrier
-// k-tile t + 1 is in once at most 12 (S - 2) younger loads, plus `extra`
-// stores issued since, are outstanding.
-template <bool FIRST, typename Src, typename Next>
-__device__ __forceinline__ void gm_iteration(const GmLane &L, unsigned char *smem, gm_f32x16 (&acc)[2][2],
-                                             gm_h8 (&f0)[6], gm_h8 (&f1)[6], int &stage, int &pend_stage,
-                                             int extra, const Src &src, const Next &next_src) {
-  const int nxt = stage + 1 == GM_S ? 0 : stage + 1;
-  const unsigned char *cur = smem + stage * GM_STAGE;
-  // step q's reads with loads i0 .. i0 + 2 between them in program order
-  // (the compiler keeps LDS reads and direct loads, which may alias, in
-  // that order; the schedule then interleaves both with the MFMAs)
-  auto read_load = [&](const unsigned char *rs, int q, gm_h8 (&fr)[6], int i0) {
-    const int c = 2 * q + L.h;
-    unsigned char *ls = smem + pend_stage * GM_STAGE;
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      fr[2 * k] = *(const gm_h8 *)(rs + L.roff[2 * k] + ((c ^ L.rkey[2 * k]) << 4));
-      gm_direct(src(i0 + k), ls + (4 * (i0 + k) + L.wave) * 1024);
-      fr[2 * k + 1] = *(const gm_h8 *)(rs + L.roff[2 * k + 1] + ((c ^ L.rkey[2 * k + 1]) << 4));
-    }
-  };
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (!FIRST) read_load(cur, 1, f1, 3);
-  else gm_read(L, cur, 1, f1);
-  gm_mfma(acc, f0);
-  gm_interleave();
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (!FIRST) read_load(cur, 2, f0, 6);
-  else gm_read(L, cur, 2, f0);
-  gm_mfma(acc, f1);
-  gm_interleave();
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (!FIRST) read_load(cur, 3, f1, 9);
-  else gm_read(L, cur, 3, f1);
-  gm_mfma(acc, f0);
-  gm_interleave();
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt(GM_LGKM0);
-  if (extra == 0) __builtin_amdgcn_s_waitcnt(gm_vmcnt(12 * (GM_S - 2)));
-  else if (extra == 16) __builtin_amdgcn_s_waitcnt(gm_vmcnt(12 * (GM_S - 2) + 16));
-  else __builtin_amdgcn_s_waitcnt(gm_vmcnt(12 * (GM_S - 2) + 32));
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  // every wave is done with stage `stage`: it takes the new k-tile
-  next_src();
-  pend_stage = stage;
-  read_load(smem + nxt * GM_STAGE, 0, f0, 0);
-  gm_mfma(acc, f1);
-  gm_interleave();
-  __builtin_amdgcn_sched_barrier(0);
-  stage = nxt;
-}
-
-// Split-K grid: block (x, s) computes tile x (XCD-grouped, m-major) over K
-// slice s of KS = gridDim.y (K / 64 k-tiles in KS near-equal runs) and writes
-// C block s.  Needs M % 256 == 0, nt % 64 == 0, K % 64 == 0, KS <= K / 64.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_split_kernel(
+// KS > 0: block = K slice of one tile (K / 64 k-tiles in KS near-equal runs),
+// C block = slice.  KS = 0: shares.  Block lb works on column tile
+// c = lb % n_tiles, share j = lb / n_tiles: g in [j L, (j + 1) L).  A tile is
+// split into the segments of the blocks whose shares overlap it; the segment
+// of block j goes to C block j - j0(mt), j0(mt) = mt nk / L (its first block),
+// and the block holding a tile's last segment writes zeros to the C blocks
+// after it, up to the ns blocks the consumer reads.
+// Needs M % 256 == 0, nt % 64 == 0, K % 64 == 0, KS <= K / 64.  Columns past nt
+// (the last 256 x 128 tile of an odd multiple of 64) are computed from the
+// rows that follow in B, which the caller's buffer holds, and not stored.
+template <typename S>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_kernel(
     const uint16_t *__restrict__ W, int M, int K, const uint16_t *__restrict__ B, int ldb, size_t blo, int nt,
-    float *__restrict__ C, int ldc) {
+    float *__restrict__ C, int ldc, int Lshare, int ns, int ks) {
+  constexpr int RT = S::RT, WC = S::WC;
   extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
-  const GmLane L(threadIdx.x);
-  const int n_tiles = nt / GM_BN, m_tiles = M / GM_BM;
-  // tiles m-major; the blocks b with b % 8 == x take the x-th eighth (the
-  // first tiles % 8 eighths hold one more).  Workgroups are dealt to the 8
-  // XCDs round-robin (from a starting XCD that varies between launches), so
-  // blocks with equal b % 8 share an XCD: the column tiles sharing a weight
-  // tile run together and one L2 serves the re-reads.  (Without the grouping
-  // O at 320 columns, 60 tiles in 4 slices, took 28.5 us against 23.)
-  int mt, ntl;
-  {
-    const int x = blockIdx.x & 7, tiles = m_tiles * n_tiles;
-    const int tile = x * (tiles >> 3) + min(x, tiles & 7) + (blockIdx.x >> 3);
-    mt = tile / n_tiles;
-    ntl = tile - mt * n_tiles;
+  unsigned char *const a_ring = gm_smem, *const b_ring = gm_smem + S::DA * S::ASTAGE;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n_tiles = (nt + S::CN - 1) / S::CN, m_tiles = M / GM_BM, nk = K / GM_BK, total = m_tiles * nk;
+  // this block's place in the list of work: the blocks b with b % 8 == x take
+  // the x-th eighth (the first G % 8 eighths hold one more).  Workgroups are
+  // dealt to the 8 XCDs round-robin (from a starting XCD that varies between
+  // launches), so blocks with equal b % 8 share an XCD: the column tiles
+  // sharing a weight tile run together and one L2 serves the re-reads.
+  // (Without the grouping O at 320 columns, 60 tiles in 4 slices, took 28.5 us
+  // against 23.)
+  const int x = blockIdx.x & 7, G = gridDim.x;
+  const int lb = x * (G >> 3) + min(x, G & 7) + (blockIdx.x >> 3);
+  int c, j, g0, g1;
+  if (ks > 0) {  // K slice j of tile (g0 / nk, c)
+    const int tiles = m_tiles * n_tiles, tile = lb % tiles, mt = tile / n_tiles;
+    j = lb / tiles;
+    c = tile - mt * n_tiles;
+    g0 = mt * nk + j * nk / ks;
+    g1 = mt * nk + (j + 1) * nk / ks;
+  } else {
+    c = lb % n_tiles;
+    j = lb / n_tiles;
+    g0 = min(j * Lshare, total);
+    g1 = min(g0 + Lshare, total);
+    if (g0 >= g1) return;
   }
-  const int kt0 = (int)(blockIdx.y * (K / GM_BK) / gridDim.y), kb = kt0 * GM_BK;
-  const int nk = (int)((blockIdx.y + 1) * (K / GM_BK) / gridDim.y) - kt0, last = nk - 1;
-  const uint16_t *base[GM_LOADS];
-#pragma unroll
-  for (int i = 0; i < GM_LOADS; i++) {
-    const int row = L.load_row(i), chunk = L.load_chunk(i);
-    if (i < 8) {
-      base[i] = W + (size_t)(mt * GM_BM + row) * K + kb + chunk * 8;
-    } else {
-      const int br = row - GM_BM, hl = br / GM_BN, col = br % GM_BN;
-      base[i] = B + hl * blo + (size_t)(ntl * GM_BN + col) * ldb + kb + chunk * 8;
-    }
-  }
-  gm_f32x16 acc[2][2];
-  gm_zero(acc);
-  gm_h8 f0[6], f1[6];
-  // prologue: k-tiles 0 .. S-1 fill the ring (indices past the last k-tile
-  // reload it, so every iteration issues the same number of loads)
-#pragma unroll
-  for (int s = 0; s < GM_S; s++)
-#pragma unroll
-    for (int i = 0; i < GM_LOADS; i++)
-      gm_direct(base[i] + min(s, last) * GM_BK, gm_smem + s * GM_STAGE + (4 * i + L.wave) * 1024);
-  __builtin_amdgcn_s_waitcnt(gm_vmcnt(12 * (GM_S - 1)));
-  __builtin_amdgcn_s_barrier();
-  gm_read(L, gm_smem, 0, f0);
-  int stage = 0, pend_stage = 0, pend_kt = min(GM_S, last);
-  auto src = [&](int i) { return base[i] + pend_kt * GM_BK; };
-  int t = 0;
-  auto next = [&]() { pend_kt = min(t + GM_S, last); };
-  gm_iteration<true>(L, gm_smem, acc, f0, f1, stage, pend_stage, 0, src, next);
-  for (t = 1; t < nk; t++) gm_iteration<false>(L, gm_smem, acc, f0, f1, stage, pend_stage, 0, src, next);
-  // the ring's last loads (re-reads) must land before this block's LDS is released
-  __builtin_amdgcn_s_waitcnt(gm_vmcnt(0));
-  gm_store(L, acc, C + (size_t)blockIdx.y * nt * ldc, ldc, ntl * GM_BN, mt * GM_BM, false);
-}
-
-// Balanced grid: G blocks (G / 8 a multiple of n_tiles).  Block lb works on
-// column tile c = lb % n_tiles, share j = lb / n_tiles of that column's
-// sequence g = mt * nk + kt, g in [j L, (j + 1) L).  A tile is split into
-// the segments of the blocks whose shares overlap it; the segment of block j
-// goes to C block j - j0(mt), j0(mt) = mt nk / L (its first block), and the
-// block holding a tile's last segment writes zeros to the C blocks after it,
-// up to the ns blocks the consumer reads.  The n_tiles blocks of a share
-// read the same weight k-tiles at the same time; the blocks b with equal
-// b % 8 (one XCD, as workgroups are dealt to the XCDs round-robin) hold
-// whole shares, so one L2 serves them.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_stream_kernel(
-    const uint16_t *__restrict__ W, int M, int K, const uint16_t *__restrict__ B, int ldb, size_t blo, int nt,
-    float *__restrict__ C, int ldc, int Lshare, int ns) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
-  const GmLane L(threadIdx.x);
-  const int n_tiles = nt / GM_BN, m_tiles = M / GM_BM, nk = K / GM_BK;
-  const int G = gridDim.x;
-  const int lb = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int c = lb % n_tiles, j = lb / n_tiles;
-  const int total = m_tiles * nk;
-  const int g0 = min(j * Lshare, total), g1 = min(g0 + Lshare, total);
-  if (g0 >= g1) return;
   const int last = g1 - 1;
-  const size_t slot_stride = (size_t)nt * ldc;
-  // per-lane offsets of the direct loads from the k-tile's weight / B origin
-  size_t off[GM_LOADS];
+  // Every wave passes one barrier before the first k-tile and one in each.  At
+  // k-tile g's, k-tile g + 1 is in LDS and no wave reads k-tile g again.
+  if (wave >= 4) {
+    // loader wave l: its load k fills rows 32 k + 8 l + lane / 8 of a stage, at
+    // position lane % 8, which holds chunk (lane % 8) ^ key(row)
+    const int l = wave - 4, lrow = 8 * l + (lane >> 3), chunk = (lane & 7) ^ gm_key(lrow);
+    const uint32_t aoff = (uint32_t)lrow * K + chunk * 8, boff = (uint32_t)lrow * ldb + chunk * 8;
+    int a_mt = g0 / nk, a_kt = g0 - a_mt * nk, b_kt = a_kt, sa = 0, sb = 0;
+    auto load_a = [&]() {  // the next weight stage
+      const uint16_t *src = W + (size_t)a_mt * GM_BM * K + a_kt * GM_BK;
 #pragma unroll
-  for (int i = 0; i < GM_LOADS; i++) {
-    const int row = L.load_row(i), chunk = L.load_chunk(i);
-    if (i < 8) {
-      off[i] = (size_t)row * K + chunk * 8;
-    } else {
-      const int br = row - GM_BM, hl = br / GM_BN, col = br % GM_BN;
-      off[i] = hl * blo + (size_t)(c * GM_BN + col) * ldb + chunk * 8;
-    }
-  }
-  gm_f32x16 acc[2][2];
-  gm_zero(acc);
-  // zeros for the C blocks past each tile whose last segment is this
-  // block's (issued before the ring's first loads, so the stores are older
-  // than every load the pipeline counts)
-  for (int mt = g0 / nk; mt <= last / nk; mt++) {
-    if ((mt + 1) * nk - 1 > last) break;  // the tile goes on in the next block
-    for (int sl = j - mt * nk / Lshare + 1; sl < ns; sl++)
-      gm_store(L, acc, C + sl * slot_stride, ldc, c * GM_BN, mt * GM_BM, true);
-  }
-  gm_h8 f0[6], f1[6];
-#pragma unroll
-  for (int s = 0; s < GM_S; s++) {
-    const int g = min(g0 + s, last), mt = g / nk, kt = g - mt * nk;
-    const uint16_t *wa = W + (size_t)mt * GM_BM * K + kt * GM_BK, *ba = B + kt * GM_BK;
-#pragma unroll
-    for (int i = 0; i < GM_LOADS; i++)
-      gm_direct((i < 8 ? wa : ba) + off[i], gm_smem + s * GM_STAGE + (4 * i + L.wave) * 1024);
-  }
-  __builtin_amdgcn_s_waitcnt(gm_vmcnt(12 * (GM_S - 1)));
-  __builtin_amdgcn_s_barrier();
-  gm_read(L, gm_smem, 0, f0);
-  // pending loads' position (iteration min(g + S, last)), advanced one k-tile
-  // per iteration without divisions
-  int p_mt, p_kt;
-  {
-    const int pg = min(g0 + GM_S, last);
-    p_mt = pg / nk;
-    p_kt = pg - p_mt * nk;
-  }
-  const uint16_t *wa = W + (size_t)p_mt * GM_BM * K + p_kt * GM_BK, *ba = B + p_kt * GM_BK;
-  auto src = [&](int i) { return (i < 8 ? wa : ba) + off[i]; };
-  int g = g0;
-  bool first = true;
-  auto next = [&]() {
-    if (!first && g + GM_S <= last) {
-      if (++p_kt == nk) {
-        p_kt = 0;
-        ++p_mt;
+      for (int k = 0; k < S::NA; k++)
+        gm_direct(src + (size_t)k * 32 * K + aoff, a_ring + sa * S::ASTAGE + (4 * k + l) * 1024);
+      sa = sa + 1 == S::DA ? 0 : sa + 1;
+      if (++a_kt == nk) {
+        a_kt = 0;
+        ++a_mt;
       }
-      wa = W + (size_t)p_mt * GM_BM * K + p_kt * GM_BK;
-      ba = B + p_kt * GM_BK;
+    };
+    auto load_b = [&]() {  // rows 0 .. CN - 1 hi, then lo
+      const uint16_t *src = B + (size_t)c * S::CN * ldb + b_kt * GM_BK;
+#pragma unroll
+      for (int k = 0; k < S::NB; k++)
+        gm_direct(src + (size_t)(k % (S::NB / 2)) * 32 * ldb + (k / (S::NB / 2)) * blo + boff,
+                  b_ring + sb * S::BSTAGE + (4 * k + l) * 1024);
+      sb = sb + 1 == S::DB ? 0 : sb + 1;
+      if (++b_kt == nk) b_kt = 0;
+    };
+    constexpr int YOUNG = S::NA + (S::DB > 2 ? S::NB : 0);  // loads of k-tile g + 2 that may be in flight
+    load_a();
+    load_b();
+    if (g0 + 1 <= last) {
+      load_a();
+      load_b();
     }
+    if (g0 + 2 <= last) {
+      load_a();
+      if (S::DB > 2) load_b();
+    }
+    if (g0 + 2 <= last) __builtin_amdgcn_s_waitcnt(gm_vmcnt(S::NA + S::NB + YOUNG));
+    else if (g0 + 1 <= last) __builtin_amdgcn_s_waitcnt(gm_vmcnt(S::NA + S::NB));
+    else __builtin_amdgcn_s_waitcnt(gm_vmcnt(0));
+    __builtin_amdgcn_s_barrier();
+    for (int g = g0; g < g1; g++) {
+      if (g + 2 <= last) __builtin_amdgcn_s_waitcnt(gm_vmcnt(YOUNG));
+      else __builtin_amdgcn_s_waitcnt(gm_vmcnt(0));
+      __builtin_amdgcn_s_barrier();
+      if (g + S::DB <= last) load_b();
+      if (g + S::DA <= last) load_a();
+    }
+    return;
+  }
+  const int r = lane & 31, h = lane >> 5, wr = wave / WC, wc = wave % WC;
+  const size_t slot_stride = (size_t)nt * ldc;
+  const int col0 = c * S::CN + wc * 64;
+  const bool live = col0 < nt;
+  float *cw = C + (size_t)(col0 + r) * ldc + wr * 32 * RT + 4 * h;
+  gm_f32x16 acc[RT][2];
+  auto zero_acc = [&]() {
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+      for (int jj = 0; jj < 2; jj++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[i][jj][e] = 0.f;
   };
-  int stage = 0, pend_stage = 0;
-  int c_mt = g0 / nk, c_kt = g0 - c_mt * nk;  // tile and k-tile of iteration g
-  int stored = 0;                              // stores issued at the end of the last iteration
-  auto tail = [&]() {
-    stored = 0;
+  zero_acc();
+  // zeros for the C blocks past each tile whose last segment is this block's
+  if (ks == 0 && live)
+    for (int mt = g0 / nk; mt <= last / nk; mt++) {
+      if ((mt + 1) * nk - 1 > last) break;  // the tile goes on in the next block
+      for (int sl = j - mt * nk / Lshare + 1; sl < ns; sl++)
+        gm_store<RT>(acc, cw + sl * slot_stride + mt * GM_BM, ldc, true);
+    }
+  // fragment f of step q: weight rows 32 RT wr + 32 f + r, B rows hi / lo
+  // 64 wc + 32 j + r; every row's key is (r >> 1) & 7
+  const int key = (r >> 1) & 7;
+  const int ra = (wr * 32 * RT + r) * GM_ROWB, rb = (wc * 64 + r) * GM_ROWB;
+  auto frag = [&](const unsigned char *pa, const unsigned char *pb, int q, int f) {
+    const int pos = ((2 * q + h) ^ key) << 4;
+    return f < RT ? *(const gm_h8 *)(pa + ra + f * 32 * GM_ROWB + pos)
+                  : *(const gm_h8 *)(pb + rb + ((f - RT) >> 1) * S::CN * GM_ROWB + ((f - RT) & 1) * 32 * GM_ROWB + pos);
+  };
+  __builtin_amdgcn_s_barrier();
+  gm_h8 f0[RT + 4], f1[RT + 4];
+#pragma unroll
+  for (int f = 0; f < RT + 4; f++) f0[f] = frag(a_ring, b_ring, 0, f);
+  int c_mt = g0 / nk, c_kt = g0 - c_mt * nk;  // k-tile of iteration g
+  int sa = 0, sb = 0;                         // its stages
+  // MFMAs of `fr` with the reads of step q into `to`
+  auto step = [&](const gm_h8 (&fr)[RT + 4], gm_h8 (&to)[RT + 4], int q) {
+    const unsigned char *pa = a_ring + sa * S::ASTAGE, *pb = b_ring + sb * S::BSTAGE;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int f = 0; f < RT + 4; f++) to[f] = frag(pa, pb, q, f);
+    gm_mfma<RT>(acc, fr);
+#pragma unroll
+    for (int k = 0; k < RT + 4; k++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 4 * RT - (RT + 4), 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int g = g0; g < g1; g++) {
+    step(f0, f1, 1);
+    step(f1, f0, 2);
+    step(f0, f1, 3);
+    __builtin_amdgcn_s_waitcnt(GM_LGKM0);
+    __builtin_amdgcn_s_barrier();
+    sa = sa + 1 == S::DA ? 0 : sa + 1;
+    sb = sb + 1 == S::DB ? 0 : sb + 1;
+    step(f1, f0, 0);  // the next k-tile's first fragments (past the last: unused)
     if (c_kt == nk - 1 || g == last) {
-      const int slot = j - c_mt * nk / Lshare;  // this segment's C block
-      gm_store(L, acc, C + slot * slot_stride, ldc, c * GM_BN, c_mt * GM_BM, false);
-      stored = 16;
-      gm_zero(acc);
+      const int slot = ks > 0 ? j : j - c_mt * nk / Lshare;  // this segment's C block
+      if (live) gm_store<RT>(acc, cw + slot * slot_stride + c_mt * GM_BM, ldc, false);
+      zero_acc();
     }
     if (++c_kt == nk) {
       c_kt = 0;
       ++c_mt;
     }
-  };
-  gm_iteration<true>(L, gm_smem, acc, f0, f1, stage, pend_stage, stored, src, next);
-  tail();
-  first = false;
-  for (g = g0 + 1; g < g1; g++) {
-    gm_iteration<false>(L, gm_smem, acc, f0, f1, stage, pend_stage, stored, src, next);
-    tail();
   }
-  // direct loads and stores in flight must finish before the block ends
-  __builtin_amdgcn_s_waitcnt(gm_vmcnt(0));
 }
 
 // Thin grid, for chunks of at most GT_MAXN columns: the product is then bound
@@ -518,12 +426,12 @@ __global__ __launch_bounds__(256) void gemm_thin_kernel(const uint16_t *__restri
 inline int gm_cols(int n) { return n <= 16 ? 16 : n <= 32 ? 32 : (n + GM_BN - 1) / GM_BN * GM_BN; }
 
 struct GemmPlan {
-  int thin = 0;    // thin grid: 32-row tiles per block (0: another grid)
-  bool stream = false;
-  int ks = 1;      // split and thin grids: K slices
-  int grid = 0;    // stream grid: blocks
-  int share = 0;   // stream grid: k-tiles per block
-  int slices = 1;  // C blocks the consumer sums
+  int thin = 0;       // thin grid: 32-row tiles per block (0: the tiled grid)
+  bool wide = false;  // 256 x 128 tiles, else 256 x 64
+  int ks = 1;         // K slices (0: shares)
+  int grid = 0;       // tiled grid: blocks
+  int share = 0;      // k-tiles per block
+  int slices = 1;     // C blocks the consumer sums
 };
 
 // Calls f(std::integral_constant<int, NS>) for the slice counts a plan can
@@ -544,16 +452,15 @@ inline bool gm_with_slices(int ns, F &&f) {
   }
 }
 
-// Consumer slice count of a balanced grid with per_col shares of L k-tiles
-// per column: the most segments any tile is cut into, rounded up to 1, 2, 4
-// or 8 (0: more than 8)
-inline int gemm_stream_slices(int m_tiles, int nk, int L) {
+// Consumer slice count of shares of L k-tiles: the most segments any tile is
+// cut into (0: more than 8)
+inline int gemm_share_slices(int m_tiles, int nk, int L) {
   int most = 1;
   for (int mt = 0; mt < m_tiles; mt++) {
     const int segs = (mt * nk + nk - 1) / L - mt * nk / L + 1;
     if (segs > most) most = segs;
   }
-  return most == 1 ? 1 : most == 2 ? 2 : most <= 4 ? 4 : most <= 8 ? 8 : 0;
+  return most <= 8 ? most : 0;
 }
 
 // Thin grid: 64-row blocks where M has enough of them for KS <= 8 slices to
@@ -574,41 +481,55 @@ inline GemmPlan gemm_thin_plan(int M, int K, int nt, int cus) {
   return p;
 }
 
+// The tiled grid's plan, by estimated time.  A block spends 0.8 us on a k-tile
+// of 256 x 64 and 1.2 us on one of 256 x 128, or the device does 300 or 180 of
+// them per us (power), whichever takes longer; a slice of C is written and
+// read again at 5 TB/s.  Candidates, for both tiles: one tile per block with K
+// in 1 .. 8 slices while that is at most one block per CU; with more tiles
+// than CUs, equal shares, or shares of whole tiles (no tile is cut: one
+// slice).  c_cap: floats that C holds.
+// The figures are a fit to 560 timed plans (88 shapes of K 896 .. 9216, M 256
+// .. 18432 and 64 .. 1024 columns, GEMM plus a reader of C, a copy of 200 MB
+// before each, as other kernels run between a prompt's products): the plan
+// picked is 0.3% slower than the best of them on average and 8% at most.
+inline GemmPlan gemm_tiled_plan(int M, int K, int nt, int cus, size_t c_cap) {
+  GemmPlan best;
+  double best_us = -1;
+  const int m_tiles = M / GM_BM, nk = K / GM_BK;
+  for (int wide = 0; wide < 2; wide++) {
+    const int n_tiles = (nt + (wide ? 127 : 63)) / (wide ? 128 : 64), tiles = m_tiles * n_tiles;
+    auto consider = [&](int ks, int grid, int share, int slices) {
+      if (slices < 1 || slices > 8 || (size_t)slices * nt * M > c_cap) return;
+      const int per_block = ks ? (nk + ks - 1) / ks : share;
+      const double us = std::max(per_block * (wide ? 1.2 : 0.8), (double)tiles * nk / (wide ? 180 : 300)) +
+                        slices * (8.0 * nt * M / 5e6);
+      if (best_us < 0 || us < best_us) {
+        best_us = us;
+        best.wide = wide;
+        best.ks = ks;
+        best.grid = grid;
+        best.share = share;
+        best.slices = slices;
+      }
+    };
+    if (tiles <= cus) {
+      for (int ks = 1; ks <= 8 && tiles * ks <= cus && (ks == 1 || nk / ks >= 2); ks++)
+        consider(ks, tiles * ks, 0, ks);
+    } else if (n_tiles <= cus) {
+      const int per_col = cus / n_tiles, even = (m_tiles * nk + per_col - 1) / per_col;
+      const int whole = (m_tiles + per_col - 1) / per_col;  // tiles
+      consider(0, per_col * n_tiles, even, gemm_share_slices(m_tiles, nk, even));
+      consider(0, (m_tiles + whole - 1) / whole * n_tiles, whole * nk, 1);
+    }
+  }
+  return best;
+}
+
 // cus: the device's compute units (8 XCDs).  Shapes must satisfy
 // M % 256 == 0, K % 64 == 0, nt = gm_cols(n).
-inline GemmPlan gemm_plan(int M, int K, int nt, int cus) {
+inline GemmPlan gemm_plan(int M, int K, int nt, int cus, size_t c_cap) {
   if (nt < GT_MAXN || (nt == GT_MAXN && M <= 2048)) return gemm_thin_plan(M, K, nt, cus);
-  GemmPlan p;
-  const int m_tiles = M / GM_BM, n_tiles = nt / GM_BN, tiles = m_tiles * n_tiles, nk = K / GM_BK;
-  if (tiles > cus) {
-    const int per_col = 8 * ((cus / 8) / n_tiles);  // balanced grid: shares per column tile
-    if (per_col >= 8 && m_tiles >= per_col) {
-      p.stream = true;
-      p.grid = per_col * n_tiles;
-      p.share = (m_tiles * nk + per_col - 1) / per_col;
-      p.slices = gemm_stream_slices(m_tiles, nk, p.share);
-      return p;
-    }
-    return p;  // split grid, K whole, several rounds
-  }
-  // At most one block per CU: K split in KS slices, as many as pay: a k-tile
-  // takes a block about 0.65 us, and a slice of C is written and read again
-  // at about 3 TB/s.  (Powers of two that fill the CUs, without the second
-  // term, took 33.0 us for gate/up at 64 columns, KS 2, where KS 3 takes 27.2,
-  // and 18.0 us with the reader of C for 1024 x 1024 at 512 columns, KS 8.
-  // The balanced grid on all CUs, with a tile cut into up to 8 segments,
-  // measured slower for these shapes: QKV, O and down of the 256-token prompt
-  // took 2-5 us more each.)
-  double best = 0;
-  for (int ks = 1; ks <= 8 && tiles * ks <= cus && (ks == 1 || nk / ks >= 2); ks++) {
-    const double us = 0.65 * ((nk + ks - 1) / ks) + ks * (8.0 * nt * M / 3e6);
-    if (ks == 1 || us < best) {
-      best = us;
-      p.ks = ks;
-    }
-  }
-  p.slices = p.ks;
-  return p;
+  return gemm_tiled_plan(M, K, nt, cus, c_cap);
 }
 
 // f(kernel, LDS bytes) for every thin kernel a plan can name
@@ -626,13 +547,14 @@ inline void gm_with_thin(int rt, int nt, bool ntw, F &&f) {
   else if (nt == 64) pick(two, std::integral_constant<int, 64>{});
 }
 
-// the kernels' dynamic LDS: 144 KB for the tiles of 256 x 64, 48 or 72 KB for
-// the thin ones
+// the kernels' dynamic LDS: 144 and 160 KB for the tiled grid, 48 or 72 KB
+// for the thin one
 inline hipError_t gemm_setup() {
-  hipError_t e = hipFuncSetAttribute((const void *)gemm_split_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     GM_LDS);
+  hipError_t e = hipFuncSetAttribute((const void *)gemm_kernel<GmNarrow>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     GmNarrow::LDS);
   if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void *)gemm_stream_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, GM_LDS);
+    e = hipFuncSetAttribute((const void *)gemm_kernel<GmWide>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            GmWide::LDS);
   for (int rt = 1; rt <= 2; rt++)
     for (int nt : {16, 32, 64})
       for (bool ntw : {false, true})
@@ -653,12 +575,12 @@ inline void gemm_launch(const GemmPlan &p, hipStream_t st, const uint16_t *W, in
     gm_with_thin(p.thin, nt, (size_t)M * K >= (size_t)8 << 20, [&](auto kernel, int lds) {
       hipLaunchKernelGGL(kernel, dim3(M / (32 * p.thin), p.ks), dim3(256), lds, st, W, K, B, ldb, blo, n, C, M);
     });
-  else if (p.stream)
-    hipLaunchKernelGGL(gemm_stream_kernel, dim3(p.grid), dim3(256), GM_LDS, st, W, M, K, B, ldb, blo, nt, C, M,
-                       p.share, p.slices);
+  else if (p.wide)
+    hipLaunchKernelGGL(gemm_kernel<GmWide>, dim3(p.grid), dim3(512), GmWide::LDS, st, W, M, K, B, ldb, blo, nt, C, M,
+                       p.share, p.slices, p.ks);
   else
-    hipLaunchKernelGGL(gemm_split_kernel, dim3((M / GM_BM) * (nt / GM_BN), p.ks), dim3(256), GM_LDS, st, W, M, K,
-                       B, ldb, blo, nt, C, M);
+    hipLaunchKernelGGL(gemm_kernel<GmNarrow>, dim3(p.grid), dim3(512), GmNarrow::LDS, st, W, M, K, B, ldb, blo, nt, C,
+                       M, p.share, p.slices, p.ks);
 }
 
 }  // namespace vx
