@@ -183,6 +183,38 @@ def test_prefill_after_long_context(kv_f16):
         o.close()
 
 
+@pytest.mark.parametrize("pos0,n", [(1, 3), (31, 1), (32, 33), (45, 20)])
+@pytest.mark.parametrize("kv_f16", [False, True])
+def test_prefill_context_ends_inside_a_key_tile(pos0, n, kv_f16):
+    """The attention's 32-key tiles where old and new positions meet: a tile
+    with one old key, one that the prompt only fills up, one that starts with
+    it, one that holds both.  New K/V rows (f16 cache to 1e-2, as above), the
+    old ones untouched, and the last W.normed."""
+    print(f"[prefill] 1 layer, {pos0} cached + {n} tokens, f16 KV {kv_f16}", flush=True)
+    from vxtest import fill_oracle_kv
+    g = gpu_engine(n_layers=1, max_seq=96, kv_f16=kv_f16)
+    o = oracle_engine(n_layers=1, max_seq=96)
+    try:
+        if kv_f16:
+            o.set_kv_f16(True)
+        g.fill_kv_synthetic(SEED, pos0)
+        fill_oracle_kv(o, SEED, pos0)
+        g.position = pos0
+        o.position = pos0
+        old = [g.read_kv(0, w, 0, pos0) for w in (0, 1)]
+        tokens = np.random.default_rng(pos0).integers(0, 131072, n)
+        g.prefill(tokens)
+        oracle_prefill(o, tokens, 0, 0, None)
+        bar = 1e-2 if kv_f16 else 1e-3
+        for w in (0, 1):
+            assert np.array_equal(g.read_kv(0, w, 0, pos0), old[w])
+            assert max_rel_err(g.read_kv(0, w, pos0, n), o.kv(0, w)[pos0:pos0 + n]) < bar
+        assert max_rel_err(g.debug_read("normed", 3072), o.buffer("normed")) < bar
+    finally:
+        g.destroy()
+        o.close()
+
+
 def test_prefill_argument_errors():
     import voxtral_amd as V
     g = gpu_engine(n_layers=1, max_seq=64)

@@ -123,6 +123,7 @@ struct vx_engine {
         *pf_voice = nullptr;
   h8 *pf_b = nullptr;
   int32_t *pf_tok = nullptr;
+  unsigned char *pf_kv = nullptr;  // one layer's keys and values as the prompt attention's operands
   int pf_chunk = PF_MAXT;  // tokens per prefill chunk (multiple of 128)
 
   int host_pos = 0;
@@ -670,6 +671,20 @@ static char *noalloc_scratch(int *dev_out) {
 }
 
 // ================================================================ C ABI
+// from the QKV product (ns K slices in pf_c) of layer l's chunk to the O
+// projection's input: the cache rows, then the attention over [0, pos0 + n)
+template <typename KVT>
+static void enqueue_pf_attn(vx_engine *e, int l, int pos0, int n, int nt, int ns) {
+  hipStream_t st = e->st;
+  const int tiles = (pos0 + n + PFA_K - 1) / PFA_K;
+  gm_with_slices(ns, [&](auto NS) {
+    hipLaunchKernelGGL((pf_qkv_epi_kernel<NS, KVT>), dim3(tiles * NKV + 4 * n), dim3(512), 0, st, e->pf_c, nt,
+                       e->pf_q, (KVT *)e->kc(l), (KVT *)e->vc(l), e->max_seq, pos0, n, e->inv_freq, e->pf_kv);
+  });
+  hipLaunchKernelGGL(pf_attn_mfma_kernel<KVT>, dim3(NKV * (nt / PFA_T)), dim3(256 * PFA_KG), pfa_lds<KVT>(), st,
+                     e->pf_q, e->pf_kv, pos0, n, nt, e->pf_b);
+}
+
 extern "C" {
 
 int vx_config_default(vx_config *c) {
@@ -952,7 +967,9 @@ int vx_create(const vx_config *cfg_in, int32_t max_seq, vx_engine **out) {
         {(void **)&e->pf_c, (size_t)PF_NC * 2 * HID * 4},
         {(void **)&e->pf_b, (size_t)HID / 8 * PF_NC * 16},
         {(void **)&e->pf_voice, (size_t)PF_MAXT * DIM * 4},
-        {(void **)&e->pf_tok, (size_t)PF_MAXT * 4}};
+        {(void **)&e->pf_tok, (size_t)PF_MAXT * 4},
+        {(void **)&e->pf_kv, (size_t)((max_seq + PFA_K - 1) / PFA_K) * NKV *
+                                 (e->kv_f32 ? pfa_tile_bytes<float>() : pfa_tile_bytes<uint16_t>())}};
     size_t tot = 0;
     for (auto &q : parts) tot += align256(q.second);
     if (hipMalloc(&e->pf_arena, tot) != hipSuccess) {
@@ -1573,15 +1590,16 @@ int vx_fill_kv_synthetic(vx_engine *e, uint64_t seed, int32_t npos) {
 // rows are already on the device.  Afterwards the residual stream and
 // W.normed hold the last token's values and the position is advanced, as
 // after n single steps.
-// The prefill GEMMs (vx_gemm.h): 144 KB of dynamic LDS per block and the
-// device's compute-unit count for the grids; the prompt attention's 71 KB.
+// The prefill GEMMs (vx_gemm.h): up to 160 KB of dynamic LDS per block and the
+// device's compute-unit count for the grids; the prompt attention's 128 KB
+// (64 KB with the f16 cache).
 static int pf_gemm_setup(vx_engine *e) {
   if (e->gemm_ready) return VX_OK;
   HIPCHK(e, gemm_setup());
   HIPCHK(e, hipFuncSetAttribute((const void *)pf_attn_mfma_kernel<float>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, PFA_LDS));
+                                hipFuncAttributeMaxDynamicSharedMemorySize, pfa_lds<float>()));
   HIPCHK(e, hipFuncSetAttribute((const void *)pf_attn_mfma_kernel<uint16_t>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, PFA_LDS));
+                                hipFuncAttributeMaxDynamicSharedMemorySize, pfa_lds<uint16_t>()));
   int dev = 0;
   HIPCHK(e, hipGetDevice(&dev));
   HIPCHK(e, hipDeviceGetAttribute(&e->cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1640,18 +1658,8 @@ static int enqueue_prefill_chunk(vx_engine *e, int n, int tok0, int vstart, int 
     const LayerW &W = e->L[l];
     const bool next = l + 1 < e->cfg.n_layers;
     if ((rc = pf_gemm(e, W.wqkv, QKV_ROWS, DIM, nt, n, &ns))) return rc;
-    gm_with_slices(ns, [&](auto NS) {
-      hipLaunchKernelGGL(pf_qkv_epi_kernel<NS>, dim3(n, QKV_ROWS / 2 / 256), blk, 0, st, e->pf_c, nt,
-                         e->pf_q, e->kc(l), e->vc(l), e->kv_f32, e->max_seq, pos0, e->inv_freq);
-    });
-    if (e->kv_f32)
-      hipLaunchKernelGGL(pf_attn_mfma_kernel<float>, dim3(nt / PFA_T, NKV), dim3(256 * PFA_KG), PFA_LDS,
-                         st, e->pf_q, (const float *)e->kc(l), (const float *)e->vc(l), e->max_seq, pos0,
-                         n, nt, e->pf_b);
-    else
-      hipLaunchKernelGGL(pf_attn_mfma_kernel<uint16_t>, dim3(nt / PFA_T, NKV), dim3(256 * PFA_KG),
-                         PFA_LDS, st, e->pf_q, (const uint16_t *)e->kc(l), (const uint16_t *)e->vc(l),
-                         e->max_seq, pos0, n, nt, e->pf_b);
+    if (e->kv_f32) enqueue_pf_attn<float>(e, l, pos0, n, nt, ns);
+    else enqueue_pf_attn<uint16_t>(e, l, pos0, n, nt, ns);
     if ((rc = pf_gemm(e, W.wo, DIM, QD, nt, n, &ns))) return rc;
     gm_with_slices(ns, [&](auto NS) {
       hipLaunchKernelGGL((pf_resid_pack_kernel<true, NS>), dim3(nt), blk, 0, st, e->pf_c, n, nt, e->pf_x,

@@ -94,30 +94,6 @@ __global__ __launch_bounds__(256) void pf_pack_kernel(const float *X, int K, int
   }
 }
 
-// QKV outputs: interleaved rope of q and k at position pos0 + t
-// (src/shaders.ts:224-256), q -> Q[t][QD], k and v -> cache rows pos0 + t.
-// Grid: (n, QKV_ROWS / 2 / 256), one row pair per thread.
-template <int NS>
-__global__ void pf_qkv_epi_kernel(const float *C, int nt, float *Q, void *kc, void *vc, int kv_f32,
-                                  int max_seq, int pos0, const float *inv_freq) {
-  const int t = blockIdx.x, row = 2 * (blockIdx.y * blockDim.x + threadIdx.x);
-  const float y0 = pf_c<NS>(C, QKV_ROWS, nt, t, row), y1 = pf_c<NS>(C, QKV_ROWS, nt, t, row + 1);
-  const int pos = pos0 + t;
-  if (row < QD + KVD) {
-    const float ang = (float)pos * inv_freq[(row & (HD - 1)) >> 1];
-    const float cs = cosf(ang), sn = sinf(ang);
-    const float r0 = y0 * cs - y1 * sn, r1 = y0 * sn + y1 * cs;
-    if (row < QD) {
-      Q[(size_t)t * QD + row] = r0;
-      Q[(size_t)t * QD + row + 1] = r1;
-    } else {
-      kv_store2(kc, kv_f32, max_seq, row - QD, pos, r0, r1);
-    }
-  } else {
-    kv_store2(vc, kv_f32, max_seq, row - QD - KVD, pos, y0, y1);
-  }
-}
-
 // hi/lo halves of y into B columns t and nt + t at k (8 consecutive k)
 __device__ __forceinline__ void pf_put8(h8 *B, int K, int nt, int t, int kb, const float (&y)[8]) {
   h8 hi, lo;
@@ -204,35 +180,34 @@ static_assert(DIM % 8 == 0 && (HID / 8) % 128 == 0, "prefill packing groups");
 // ------------------------------------------------ causal attention on MFMA
 // Causal attention of the chunk (attnScore + softmax + attnValue per prompt
 // token over keys 0..pos0+t, src/shaders.ts:306-447) with the products on the
-// matrix cores; blocks of tokens t >= n write zero columns of the O GEMM's B.
-// Block = (16-token tile, KV head) of PFA_KG groups of 4 waves; wave w of a
-// group is query head 4*kv_head + w.  The tile's keys are taken 32 at a
-// time: group g stages tiles g, g + PFA_KG, ... in its own LDS area, K rows
-// and transposed V rows already split into f16 hi and lo (once per group,
-// not once per wave), shared by its 4 waves, and keeps its own online
-// softmax; the groups' (max, sum, O) are merged through LDS at the end.
-// Per 32-key tile and wave, in the transposed form (the token is the MFMA
-// column, so every lane holds one token's values):
-//   S^T[16 keys][16 tokens] = K[16][128] . Q^T[128][16]     16x16x32 f16
-//   O^T[16 dims][16 tokens] += V^T[16][16 keys] . P^T[16 keys][16]   16x16x16 f16
-// The D layout of S^T (lane l: keys 4(l/16)..+3 of token l%16) is exactly
-// the B operand of the 16x16x16 product, so P needs no shuffle; the online
-// softmax rescale of O^T is per lane.  Every f32 operand is split into f16
-// hi + lo and a product is hi.hi + hi.lo + lo.hi, about 2^-20 relative (the
-// dropped lo.lo term), where the prefill GEMMs, with exact f16 weights, are
-// at the split's 2^-21.  An f16 cache is exact in f16: its lo halves are
-// zero, so they are neither stored nor multiplied.  Output: hi/lo
-// rows of the O projection's B (rows t and nt + t), zero for t >= n.
+// matrix cores, in the transposed form (the token is the MFMA column, so every
+// lane holds one token's values).  Per 32-key tile, wave and 16 tokens:
+//   S^T[32 keys][16 tokens] = K[32][128] . Q^T[128][16]        16x16x32 f16
+//   O^T[128 dims][16 tokens] += V^T[128][32 keys] . P^T[32][16]  16x16x32 f16
+// Every f32 operand is split into f16 hi + lo and a product is hi.hi + hi.lo +
+// lo.hi, about 2^-20 relative (the dropped lo.lo term), where the prefill
+// GEMMs, with exact f16 weights, are at the split's 2^-21.  An f16 cache is
+// exact in f16: its lo halves are zero, so they are neither stored nor
+// multiplied.
+//
+// The D layout of S^T (lane l: keys 16 kt + 4 (l / 16) .. + 3 of token l % 16)
+// becomes the B operand of the second product, which wants 8 consecutive
+// contraction slots per lane, by numbering the slots to suit: slot 8 g + 4 kt
+// + q is key 16 kt + 4 g + q, so P needs no shuffle.
+//
+// pf_qkv_epi_kernel writes the keys and values of the whole context as the
+// operands of both products, a lane's 16 bytes together, hi and lo split:
+// per KV head and 32-key tile, K hi [2 kt][4 chunks of 32 dims][64 lanes][8],
+// K lo, V^T hi [8 tiles of 16 dims][64 lanes][8 slots], V^T lo (f16 cache: K
+// and V^T hi only), 32 or 16 KB in all; keys past the last are zero.  So the
+// attention's tiles go from memory to LDS by direct loads and from there to
+// the MFMAs as they are.  Splitting and transposing in each attention block
+// instead (16 tokens each, every block its own copy) took 2.2 us per pair of
+// tiles, 0.5 of it in two barriers: 19 us at 256 tokens (13 now), 98 us at 1024
+// tokens on 500 of context, f16 cache (51 now).
 typedef _Float16 hf4 __attribute__((ext_vector_type(4)));
-constexpr int PFA_T = 16;          // tokens per block
-constexpr int PFA_K = 32;          // keys per staged tile
-constexpr int PFA_KW = HD + 8;     // LDS row of K, halves (272 B)
-constexpr int PFA_VW = PFA_K + 4;  // LDS row of V^T, halves (72 B: 16 rows start on 16 distinct even banks)
-constexpr int PFA_KG = 2;          // key groups per block
-constexpr int PFA_GROUP = 2 * (PFA_K * PFA_KW + HD * PFA_VW);  // halves of one group's area (hi + lo)
-constexpr int PFA_LDS = PFA_KG * PFA_GROUP * 2;                // dynamic LDS bytes (70 KB)
-constexpr int PFA_RED = 2 + 4 * (HD / 16);                     // merged values per lane: m, l, O^T
-static_assert((PFA_KG - 1) * 4 * PFA_RED * 64 * 4 <= PFA_LDS, "merge area");
+constexpr int PFA_K = 32;      // keys per tile
+constexpr int PFA_PART = 8192; // bytes of K or V^T of one tile, hi or lo
 
 // hi/lo operand halves (split2) of 8 or 4 f32 values
 __device__ __forceinline__ void split8(const f32x4 a, const f32x4 b, h8 &hi, h8 &lo) {
@@ -244,85 +219,215 @@ __device__ __forceinline__ void split4(const f32x4 a, hf4 &hi, hf4 &lo) {
   split_n<4>(x, hi, lo);
 }
 
-// 4 consecutive K/V values as held between load and staging: f32 as loaded,
-// f16 as raw halves (widened only when staged, so the prefetch's wait stays
-// at the staging point)
-__device__ __forceinline__ f32x4 pfa_ld4(const float *p) { return *(const f32x4 *)p; }
-__device__ __forceinline__ uint2 pfa_ld4(const uint16_t *p) { return *(const uint2 *)p; }
-__device__ __forceinline__ f32x4 pfa_widen(f32x4 v) { return v; }
-__device__ __forceinline__ f32x4 pfa_widen(uint2 v) {
-  const h2 a = __builtin_bit_cast(h2, v.x), b = __builtin_bit_cast(h2, v.y);
-  return f32x4{(float)a.x, (float)a.y, (float)b.x, (float)b.y};
+template <typename KVT>
+__host__ __device__ constexpr int pfa_tile_bytes() {
+  return sizeof(KVT) == 2 ? 2 * PFA_PART : 4 * PFA_PART;
+}
+// 8 consecutive cached values, and a value as the cache holds it
+__device__ __forceinline__ void kv_load8(const float *p, float (&y)[8]) {
+  const f32x4 a = *(const f32x4 *)p, b = *(const f32x4 *)(p + 4);
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    y[e] = a[e];
+    y[4 + e] = b[e];
+  }
+}
+__device__ __forceinline__ void kv_load8(const uint16_t *p, float (&y)[8]) {
+  const h8 a = *(const h8 *)p;
+#pragma unroll
+  for (int e = 0; e < 8; e++) y[e] = (float)a[e];
+}
+__device__ __forceinline__ float kv_load(const float *p) { return *p; }
+__device__ __forceinline__ float kv_load(const uint16_t *p) { return h2f(*p); }
+__device__ __forceinline__ float kv_store(float *p, float v) { return *p = v; }
+__device__ __forceinline__ float kv_store(uint16_t *p, float v) {
+  const uint16_t b = f2h(v);
+  *p = b;
+  return h2f(b);
 }
 
+// QKV outputs, two kinds of block in one launch of 512 threads:
+//  - block b < tiles * NKV (tiles = ceil((pos0 + n) / 32)): KV head b % NKV of
+//    the 32 positions of tile b / NKV.  New keys and values (positions pos0 ..
+//    pos0 + n - 1) come from the GEMM's K slices, the keys with interleaved
+//    rope (src/shaders.ts:224-256), and go to the cache; older ones come from
+//    the cache; both are written as the attention's operands (above), as the
+//    cache holds them.  Thread i is fragment i / 64's lane i % 64 of both K
+//    and V^T.
+//  - the blocks after them: q of token (b - tiles * NKV) / 4, rope, one row
+//    pair per thread.
+// 6 us at 256 tokens: the epilogue alone took 5.6 and a second kernel that
+// packed the operands from the cache 5.
 // KVT = float (f32 cache) or uint16_t (f16 cache).
-// Launch: grid (nt / PFA_T, NKV), 256 * PFA_KG threads, PFA_LDS dynamic LDS.
+template <int NS, typename KVT>
+__global__ __launch_bounds__(512) void pf_qkv_epi_kernel(const float *C, int nt, float *Q, KVT *kc, KVT *vc,
+                                                         int max_seq, int pos0, int n, const float *inv_freq,
+                                                         unsigned char *kv) {
+  constexpr bool EXACT = sizeof(KVT) == 2;
+  const int kend = pos0 + n, tiles = (kend + PFA_K - 1) / PFA_K;
+  if ((int)blockIdx.x >= tiles * NKV) {
+    const int b = blockIdx.x - tiles * NKV, t = b >> 2, row = 2 * ((b & 3) * 512 + threadIdx.x);
+    const float y0 = pf_c<NS>(C, QKV_ROWS, nt, t, row), y1 = pf_c<NS>(C, QKV_ROWS, nt, t, row + 1);
+    const float ang = (float)(pos0 + t) * inv_freq[(row & (HD - 1)) >> 1];
+    const float cs = cosf(ang), sn = sinf(ang);
+    *(float2 *)(Q + (size_t)t * QD + row) = make_float2(y0 * cs - y1 * sn, y0 * sn + y1 * cs);
+    return;
+  }
+  const int it = blockIdx.x / NKV, kvh = blockIdx.x % NKV, f = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int r = lane & 15, g = lane >> 4;
+  KVT *Kb = kc + (size_t)kvh * max_seq * HD, *Vb = vc + (size_t)kvh * max_seq * HD;
+  h8 *o = (h8 *)(kv + ((size_t)it * NKV + kvh) * pfa_tile_bytes<KVT>());
+  // K: position key, dims d .. d + 7; V^T: dim dv of 8 positions.  Every load is
+  // issued before the first use, from a clamped row where there is none; only
+  // a tile that holds older positions (uniform) reads the cache as well.
+  const int key = it * PFA_K + 16 * (f >> 2) + r, d = 32 * (f & 3) + 8 * g, dv = 16 * f + r;
+  auto vpos = [&](int e) { return it * PFA_K + 16 * (e >> 2) + 4 * g + (e & 3); };
+  auto row = [&](int pos) { return max(min(pos, kend - 1) - pos0, 0); };
+  float k[8], v[8], fr[4];
+  const f32x4 ka = pf_c4<NS>(C, QKV_ROWS, nt, row(key), QD + kvh * HD + d);
+  const f32x4 kb = pf_c4<NS>(C, QKV_ROWS, nt, row(key), QD + kvh * HD + d + 4);
+#pragma unroll
+  for (int e = 0; e < 4; e++) fr[e] = inv_freq[(d >> 1) + e];
+#pragma unroll
+  for (int e = 0; e < 8; e++) v[e] = pf_c<NS>(C, QKV_ROWS, nt, row(vpos(e)), QD + KVD + kvh * HD + dv);
+  float ko[8], vo[8];
+  if (it * PFA_K < pos0) {
+    kv_load8(Kb + (size_t)min(key, pos0 - 1) * HD + d, ko);
+#pragma unroll
+    for (int e = 0; e < 8; e++) vo[e] = kv_load(Vb + (size_t)min(vpos(e), pos0 - 1) * HD + dv);
+  }
+  const float y[8] = {ka[0], ka[1], ka[2], ka[3], kb[0], kb[1], kb[2], kb[3]};
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    const float ang = (float)key * fr[e >> 1];
+    const float cs = cosf(ang), sn = sinf(ang);
+    k[e] = y[e] * cs - y[e + 1] * sn;
+    k[e + 1] = y[e] * sn + y[e + 1] * cs;
+  }
+  if (key >= pos0 && key < kend) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) k[e] = kv_store(Kb + (size_t)key * HD + d + e, k[e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; e++) k[e] = key < pos0 ? ko[e] : 0.f;
+  }
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const int pos = vpos(e);
+    if (pos >= pos0 && pos < kend) v[e] = kv_store(Vb + (size_t)pos * HD + dv, v[e]);
+    else v[e] = pos < pos0 ? vo[e] : 0.f;
+  }
+  h8 hi, lo;
+  h8 *ov = o + (EXACT ? 1 : 2) * (PFA_PART / 16);
+  split_n<8>(k, hi, lo);
+  o[f * 64 + lane] = hi;
+  if (!EXACT) o[PFA_PART / 16 + f * 64 + lane] = lo;
+  split_n<8>(v, hi, lo);
+  ov[f * 64 + lane] = hi;
+  if (!EXACT) ov[PFA_PART / 16 + f * 64 + lane] = lo;
+}
+
+// maximum / sum of a value over the four lane groups that hold one token, by
+// two lane swaps of the value with a copy of itself (an LDS permute, __shfl_xor,
+// is about 100 clocks on each of the tile's four steps).  In asm, with the
+// two wait states that a swap needs after a VALU write: for the builtins this
+// compiler uses the first of the two results twice.  The results only feed
+// VALU instructions.
+__device__ __forceinline__ void pfa_swap16(float &a, float &b) {
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ void pfa_swap32(float &a, float &b) {
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ float pfa_max4(float a) {
+  float b = a;
+  pfa_swap16(a, b);
+  a = b = fmaxf(a, b);
+  pfa_swap32(a, b);
+  return fmaxf(a, b);
+}
+__device__ __forceinline__ float pfa_sum4(float a) {
+  float b = a;
+  pfa_swap16(a, b);
+  a = b = a + b;
+  pfa_swap32(a, b);
+  return a + b;
+}
+
+// Block = (16 tokens, KV head): two key groups of 4 waves, wave w of a group
+// query head 4 kv_head + w.  Group g walks tiles g, g + 2, ... in two LDS
+// stages of its own, one tile loading while the last is used, with its own
+// online softmax; the groups' (max, sum, O) are merged through LDS at the end,
+// in group order.  Writes hi/lo rows of the O projection's B (rows t and
+// nt + t), zero for t >= n.
+// 32 tokens per wave (half the LDS reads per MFMA, half the blocks) and four
+// groups (f16 cache) were slower at every size: 1024 tokens, f32 cache, 56
+// against 44 us; 512 tokens 31 against 21; 1024 tokens on 500 of context, f16
+// cache, 62 and 64 against 49-50; 276 more on those 42 and 41 against 38.
+// Launch: grid NKV * nt / 16, 512 threads, pfa_lds dynamic LDS.  Block b takes
+// KV head b % 8 (blocks with equal b % 8 share an XCD, so its L2 holds that
+// head's tiles) and the later, longer token tiles first.
+constexpr int PFA_T = 16;            // tokens per block
+constexpr int PFA_KG = 2;            // key groups per block
+constexpr int PFA_RED = 2 + HD / 4;  // merged values per lane: m, l, O^T
 template <typename KVT>
-__global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float *Q, const KVT *kc,
-                                                                    const KVT *vc, int max_seq, int pos0,
+__host__ __device__ constexpr int pfa_lds() {
+  static_assert((PFA_KG - 1) * 4 * PFA_RED * 256 <= PFA_KG * 2 * 2 * PFA_PART, "merge area");
+  return PFA_KG * 2 * pfa_tile_bytes<KVT>();
+}
+template <typename KVT>
+__global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float *Q, const unsigned char *kv, int pos0,
                                                                     int n, int nt, h8 *B) {
   constexpr bool EXACT = std::is_same<KVT, uint16_t>::value;  // f16 cache: no lo halves
-  extern __shared__ __attribute__((aligned(16))) _Float16 pfa_smem[];
-  const int t0 = blockIdx.x * PFA_T, kvh = blockIdx.y;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  constexpr int TILE = pfa_tile_bytes<KVT>(), NL = TILE / 4096;  // bytes; direct loads per wave
+  extern __shared__ __attribute__((aligned(16))) unsigned char pfa_smem[];
+  const int kvh = blockIdx.x % NKV, t0 = (gridDim.x / NKV - 1 - blockIdx.x / NKV) * PFA_T;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int grp_k = wave >> 2, hw = wave & 3;  // key group, head within the KV group
   const int h = kvh * (NH / NKV) + hw;
   const int col = lane & 15, grp = lane >> 4;  // MFMA column (token) and row group
   const int t = t0 + col;                      // this lane's token
-  _Float16 *khs = pfa_smem + grp_k * PFA_GROUP, *kls = khs + PFA_K * PFA_KW;
-  _Float16 *vhs = kls + PFA_K * PFA_KW, *vls = vhs + HD * PFA_VW;
+  _Float16 *const out = (_Float16 *)B + (size_t)t * QD + h * HD + 4 * grp;  // its hi row; lo: nt rows on
   if (t0 >= n) {  // padding columns of the GEMM: zero hi and lo (group 0 writes)
     if (grp_k == 0) {
-      _Float16 *p = (_Float16 *)B;
 #pragma unroll
       for (int dt = 0; dt < HD / 16; dt++) {
-        const size_t c = (size_t)h * HD + dt * 16 + 4 * grp;
-        *(hf4 *)(p + (size_t)t * QD + c) = hf4{0, 0, 0, 0};
-        *(hf4 *)(p + (size_t)(nt + t) * QD + c) = hf4{0, 0, 0, 0};
+        *(hf4 *)(out + dt * 16) = hf4{0, 0, 0, 0};
+        *(hf4 *)(out + (size_t)nt * QD + dt * 16) = hf4{0, 0, 0, 0};
       }
     }
     return;
   }
-  const KVT *Kb = kc + (size_t)kvh * max_seq * HD;
-  const KVT *Vb = vc + (size_t)kvh * max_seq * HD;
-  const int last = pos0 + min(t, n - 1);         // last key of this lane's token
-  const int kend = pos0 + min(t0 + PFA_T, n);    // keys of the tile: [0, kend)
+  const int last = pos0 + min(t, n - 1);            // last key of this lane's token
+  const int kend = pos0 + min(t0 + PFA_T, n);       // keys of the block: [0, kend)
   const int ntile = (kend + PFA_K - 1) / PFA_K;
   const int iters = (ntile + PFA_KG - 1) / PFA_KG;  // the same count in every group
-
-  // staging, thread i of its group: K rows (i / 32) + 8j, dims 4 (i % 32)
-  // (row-major LDS writes); V keys 2 (i % 16) and 2 (i % 16) + 1, dims
-  // 4 (i / 16) and 64 + 4 (i / 16), so each transposed LDS write holds the
-  // pair of keys as one dword
-  const int gtid = tid & 255, srow = gtid >> 5, sdim = (gtid & 31) * 4;
-  const int vkey = 2 * (gtid & 15), vdim = 4 * (gtid >> 4);
-  decltype(pfa_ld4(Kb)) kr[4], vr[4];
-  auto load_tile = [&](int kb) {
+  unsigned char *const ring = pfa_smem + grp_k * 2 * TILE;
+  // tile it into stage s: wave w of the group brings the KBs w, w + 4, ...
+  auto load_tile = [&](int it, int s) {
+    const unsigned char *src = kv + ((size_t)it * NKV + kvh) * TILE + hw * 1024 + lane * 16;
+    unsigned char *dst = ring + s * TILE + hw * 1024;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int key = min(kb + srow + 8 * j, kend - 1);  // rows past the keys re-read the last
-      kr[j] = pfa_ld4(Kb + (size_t)key * HD + sdim);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {  // vr[j]: key vkey + (j >> 1), dims vdim + 64 (j & 1)
-      const int key = min(kb + vkey + (j >> 1), kend - 1);
-      vr[j] = pfa_ld4(Vb + (size_t)key * HD + vdim + 64 * (j & 1));
-    }
+    for (int i = 0; i < NL; i++)
+      __builtin_amdgcn_global_load_lds((const void *)(src + i * 4096),
+                                       (__attribute__((address_space(3))) void *)(dst + i * 4096), 16, 0, 0);
   };
-  if (grp_k < ntile) load_tile(grp_k * PFA_K);
+  if (grp_k < ntile) load_tile(grp_k, 0);
 
-  // Q^T operand of S^T (token t, dims 32c + 8grp..+8), hi and lo; padding tokens zero
+  // Q^T operand of S^T (token t, dims 32c + 8grp..+8), hi and lo, in units
+  // that make a score log2(e) / sqrt(128) q.k (the softmax is of powers of
+  // two); padding tokens zero
   h8 qh[HD / 32], ql[HD / 32];
   {
+    const float scale = 1.44269504f / sqrtf((float)HD);
     const float *qp = Q + (size_t)min(t, n - 1) * QD + h * HD + 8 * grp;
 #pragma unroll
     for (int c = 0; c < HD / 32; c++) {
       f32x4 a = *(const f32x4 *)(qp + 32 * c), b = *(const f32x4 *)(qp + 32 * c + 4);
       if (t >= n) a = b = f32x4{0.f, 0.f, 0.f, 0.f};
-      split8(a, b, qh[c], ql[c]);
+      split8(a * scale, b * scale, qh[c], ql[c]);
     }
   }
-  const float scale = 1.0f / sqrtf((float)HD);
   float m = -INFINITY, l = 0.f;
   f32x4 o[HD / 16];
 #pragma unroll
@@ -330,150 +435,112 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
 
   for (int i = 0; i < iters; i++) {
     const int it = grp_k + PFA_KG * i, kb = it * PFA_K;
-    const bool live = it < ntile;  // uniform over the group
-    __syncthreads();  // the previous tile's LDS reads are done
-    if (live) {
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        hf4 hi, lo;
-        split4(pfa_widen(kr[j]), hi, lo);
-        *(hf4 *)(khs + (srow + 8 * j) * PFA_KW + sdim) = hi;
-        if (!EXACT) *(hf4 *)(kls + (srow + 8 * j) * PFA_KW + sdim) = lo;
-      }
-#pragma unroll
-      for (int hd = 0; hd < 2; hd++) {
-        const f32x4 va = pfa_widen(vr[hd]), vb = pfa_widen(vr[2 + hd]);  // keys vkey, vkey + 1
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          h2 hi, lo;
-          split2(va[q], vb[q], hi, lo);
-          const int d = vdim + 64 * hd + q;
-          *(h2 *)(vhs + d * PFA_VW + vkey) = hi;
-          if (!EXACT) *(h2 *)(vls + d * PFA_VW + vkey) = lo;
-        }
-      }
-      if (it + PFA_KG < ntile) load_tile(kb + PFA_KG * PFA_K);
-    }
-    __syncthreads();
-    if (!live) continue;
+    // this wave's share of tile it is in (every load is: the next tile's go
+    // out below), and past the barrier every wave's is, and no wave reads the
+    // other stage any more
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (it + PFA_KG < ntile) load_tile(it + PFA_KG, (i + 1) & 1);
+    if (it >= ntile) continue;  // uniform over the group
+    const h8 *kh = (const h8 *)(ring + (i & 1) * TILE) + lane, *kl = kh + PFA_PART / 16;
+    const h8 *vh = kh + (EXACT ? 1 : 2) * (PFA_PART / 16), *vl = vh + PFA_PART / 16;
 
-    // S^T for keys kb + 16kt + (4grp..+3), token col
-    f32x4 s[2];
+    // S^T of keys kb + 16kt + (4grp..+3), token t; the lo products in an
+    // accumulator of their own, so no chain of dependent MFMAs is longer than 8
+    f32x4 s[2], sl[2];
 #pragma unroll
-    for (int kt = 0; kt < 2; kt++) {
-      f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-      const int ro = (16 * kt + col) * PFA_KW + 8 * grp;
+    for (int kt = 0; kt < 2; kt++) s[kt] = sl[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int c = 0; c < HD / 32; c++) {
-        const h8 kh = *(const h8 *)(khs + ro + 32 * c);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[c], acc, 0, 0, 0);
-        if (!EXACT) {
-          const h8 kl = *(const h8 *)(kls + ro + 32 * c);
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[c], acc, 0, 0, 0);
-        }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[c], acc, 0, 0, 0);
-      }
-      s[kt] = acc;
-    }
-    // online softmax of token col over this tile's keys (8 per lane, 4 lanes per token)
-    float mx = -INFINITY;
-#pragma unroll
-    for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int key = kb + 16 * kt + 4 * grp + q;
-        const float v = key <= last ? s[kt][q] * scale : -INFINITY;
-        s[kt][q] = v;
-        mx = fmaxf(mx, v);
-      }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    // a token whose keys all lie past this tile's start keeps m = -inf
-    // (only in groups other than 0: key 0 <= last is in tile 0)
-    const float mnew = fmaxf(m, mx);
-    const float corr = mnew == -INFINITY ? 1.0f : expf(m - mnew);
-    float ps = 0.f;
-#pragma unroll
-    for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const float e = s[kt][q] == -INFINITY ? 0.f : expf(s[kt][q] - mnew);
-        s[kt][q] = e;
-        ps += e;
-      }
-    ps += __shfl_xor(ps, 16, 64);
-    ps += __shfl_xor(ps, 32, 64);
-    l = l * corr + ps;
-    m = mnew;
-    // O^T += V^T . P^T
-    hf4 ph[2], pl[2];
-#pragma unroll
-    for (int kt = 0; kt < 2; kt++) split4(s[kt], ph[kt], pl[kt]);
-#pragma unroll
-    for (int dt = 0; dt < HD / 16; dt++) {
-      f32x4 acc = o[dt] * corr;
+    for (int c = 0; c < HD / 32; c++)
 #pragma unroll
       for (int kt = 0; kt < 2; kt++) {
-        const int ro = (16 * dt + col) * PFA_VW + 16 * kt + 4 * grp;
-        const hf4 vh = *(const hf4 *)(vhs + ro);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(vh, ph[kt], acc, 0, 0, 0);
-        if (!EXACT) {
-          const hf4 vl = *(const hf4 *)(vls + ro);
-          acc = __builtin_amdgcn_mfma_f32_16x16x16f16(vl, ph[kt], acc, 0, 0, 0);
-        }
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(vh, pl[kt], acc, 0, 0, 0);
+        const h8 a = kh[(4 * kt + c) * 64];
+        s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[c], s[kt], 0, 0, 0);
+        sl[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[c], sl[kt], 0, 0, 0);
+        if (!EXACT) sl[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[(4 * kt + c) * 64], qh[c], sl[kt], 0, 0, 0);
       }
-      o[dt] = acc;
+    // online softmax over this tile's keys (8 per lane, 4 lanes per token);
+    // only a tile that reaches past the block's first token has keys to hide
+    float p[8], mx = -INFINITY;
+    const bool edge = kb + PFA_K - 1 > pos0 + t0;
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      p[q] = s[q >> 2][q & 3] + sl[q >> 2][q & 3];
+      if (edge && kb + 16 * (q >> 2) + 4 * grp + (q & 3) > last) p[q] = -INFINITY;
+      mx = fmaxf(mx, p[q]);
+    }
+    mx = pfa_max4(mx);
+    if (__builtin_amdgcn_ballot_w64(mx > m)) {  // some token's maximum grows
+      // a token whose keys all lie before this tile's start keeps m = -inf
+      // (only in groups other than 0: key 0 <= last is in tile 0)
+      const float mnew = fmaxf(m, mx);
+      const float corr = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mnew);
+      m = mnew;
+      l *= corr;
+#pragma unroll
+      for (int dt = 0; dt < HD / 16; dt++) o[dt] = o[dt] * corr;
+    }
+    const float base = m == -INFINITY ? 0.f : m;
+    float ps = 0.f;
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      p[q] = __builtin_amdgcn_exp2f(p[q] - base);  // hidden keys: 0
+      ps += p[q];
+    }
+    l += pfa_sum4(ps);
+    h8 ph, pl;
+    split_n<8>(p, ph, pl);
+    // O^T += V^T . P^T
+#pragma unroll
+    for (int dt = 0; dt < HD / 16; dt++) {
+      const h8 a = vh[dt * 64];
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ph, o[dt], 0, 0, 0);
+      if (!EXACT) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl[dt * 64], ph, o[dt], 0, 0, 0);
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pl, o[dt], 0, 0, 0);
     }
   }
   // merge the groups' (m, l, O^T) in group order: groups 1.. write theirs
   // to LDS (lane-minor), group 0 combines them
-  if (PFA_KG > 1) {
-    float *red = (float *)pfa_smem;
-    __syncthreads();  // every group is done with its staging area
-    if (grp_k > 0) {
-      float *r = red + ((grp_k - 1) * 4 + hw) * PFA_RED * 64 + lane;
-      r[0] = m;
-      r[64] = l;
+  float *red = (float *)pfa_smem;
+  __syncthreads();  // every group is done with its stages
+  if (grp_k > 0) {
+    float *r = red + ((grp_k - 1) * 4 + hw) * PFA_RED * 64 + lane;
+    r[0] = m;
+    r[64] = l;
 #pragma unroll
-      for (int dt = 0; dt < HD / 16; dt++)
+    for (int dt = 0; dt < HD / 16; dt++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) r[(2 + 4 * dt + q) * 64] = o[dt][q];
-    }
-    __syncthreads();
-    if (grp_k > 0) return;
-    float mg[PFA_KG];
-    mg[0] = m;
+      for (int q = 0; q < 4; q++) r[(2 + 4 * dt + q) * 64] = o[dt][q];
+  }
+  __syncthreads();
+  if (grp_k > 0) return;
+  float mm = m;
 #pragma unroll
-    for (int g = 1; g < PFA_KG; g++) mg[g] = red[((g - 1) * 4 + hw) * PFA_RED * 64 + lane];
-    float mm = mg[0];
+  for (int g = 1; g < PFA_KG; g++) mm = fmaxf(mm, red[((g - 1) * 4 + hw) * PFA_RED * 64 + lane]);
+  const float c0 = __builtin_amdgcn_exp2f(m - mm);  // m is finite in group 0
+  l *= c0;
 #pragma unroll
-    for (int g = 1; g < PFA_KG; g++) mm = fmaxf(mm, mg[g]);
-    const float c0 = expf(m - mm);  // m is finite in group 0
-    l *= c0;
+  for (int dt = 0; dt < HD / 16; dt++) o[dt] = o[dt] * c0;
 #pragma unroll
-    for (int dt = 0; dt < HD / 16; dt++) o[dt] = o[dt] * c0;
+  for (int g = 1; g < PFA_KG; g++) {
+    const float *rg = red + ((g - 1) * 4 + hw) * PFA_RED * 64 + lane;
+    const float cg = __builtin_amdgcn_exp2f(rg[0] - mm);  // m = -inf: 0
+    l += rg[64] * cg;
 #pragma unroll
-    for (int g = 1; g < PFA_KG; g++) {
-      const float *rg = red + ((g - 1) * 4 + hw) * PFA_RED * 64 + lane;
-      const float cg = mg[g] == -INFINITY ? 0.f : expf(mg[g] - mm);
-      l += rg[64] * cg;
+    for (int dt = 0; dt < HD / 16; dt++)
 #pragma unroll
-      for (int dt = 0; dt < HD / 16; dt++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) o[dt][q] += rg[(2 + 4 * dt + q) * 64] * cg;
-    }
+      for (int q = 0; q < 4; q++) o[dt][q] += rg[(2 + 4 * dt + q) * 64] * cg;
   }
   // out[t][dims] = O^T / l, as hi and lo f16 rows of B (zero past n)
-  _Float16 *p = (_Float16 *)B;
   const float inv = 1.0f / l;
 #pragma unroll
   for (int dt = 0; dt < HD / 16; dt++) {
     hf4 hi = hf4{0, 0, 0, 0}, lo = hf4{0, 0, 0, 0};
     if (t < n) split4(o[dt] * inv, hi, lo);
-    const size_t c = (size_t)h * HD + dt * 16 + 4 * grp;
-    *(hf4 *)(p + (size_t)t * QD + c) = hi;
-    *(hf4 *)(p + (size_t)(nt + t) * QD + c) = lo;
+    *(hf4 *)(out + dt * 16) = hi;
+    *(hf4 *)(out + (size_t)nt * QD + dt * 16) = lo;
   }
 }
 
