@@ -466,3 +466,29 @@ def test_long_context_decode_26_layers_f16_kv():
     finally:
         g.destroy()
         o.close()
+
+
+def test_lm_head_argmax_ties():
+    """The LM head's argmax over equal largest logits: embedding rows made
+    equal (and parallel to the step's W.normed, so theirs are the largest) at
+    indices whose lanes (i % 256) the reference's tree orders differently than
+    their numbers; the oracle's argmax of the logits read back."""
+    name = "mm_audio_embeddings.tok_embeddings.weight"
+    print("[lm head] argmax ties", flush=True)
+    g = gpu_engine(n_layers=1, max_seq=64)
+    try:
+        x = O.gen_f32(3, "input.hidden", 3072)
+        _, h = g.backbone_step(precomputed=x)
+        bits = g.read_tensor(name, 131072 * 3072).reshape(131072, 3072)
+        row = (h / np.linalg.norm(h) * 40).astype(np.float16).view(np.uint16)
+        for ties in ([1, 128], [5, 261], [255, 254, 1795], [131071, 65536 + 3, 70], [64, 2, 32 + 256 * 400]):
+            b = bits.copy()
+            b[ties] = row
+            g.load_tensor(name, b)
+            g.position = 0
+            top, _ = g.backbone_step(precomputed=x, lm_head=True)
+            logits = g.debug_read("logits", 131072)
+            assert len(set(logits[ties])) == 1 and logits.max() == logits[ties[0]]
+            assert top in ties and top == O.argmax(logits), (ties, top)
+    finally:
+        g.destroy()

@@ -101,6 +101,7 @@ struct vx_engine {
   unsigned long long *timeline = nullptr;
   int *pos = nullptr, *frame = nullptr;
   uint32_t *sem_code = nullptr, *codes = nullptr, *argmax_res = nullptr;
+  ArgmaxBest *argmax_part = nullptr;  // LM head argmax, best of each block
   uint64_t *noise_seed = nullptr;
   float *inv_freq = nullptr;  // rope inverse frequencies [HD/2]
   float *fm_seq = nullptr, *fm_q = nullptr, *fm_k = nullptr, *fm_v = nullptr, *fm_attn = nullptr,
@@ -354,8 +355,9 @@ static void enqueue_backbone_feedback(vx_engine *e) {
 static void enqueue_lm_head(vx_engine *e) {
   GemvArgs a = gargs(e->tok_emb, e->normed, DIM, e->logits, 0, e->cfg.vocab_size);
   launch_gemv<1, W4, 2, EPI_PLAIN, false, DIM, DIM>(e->st, a);
-  hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(256), 0, e->st, e->logits, e->cfg.vocab_size, 0,
-                     e->argmax_res);
+  hipLaunchKernelGGL(argmax_part_kernel, dim3(AM_BLOCKS), dim3(256), 0, e->st, e->logits, e->cfg.vocab_size,
+                     e->argmax_part);
+  hipLaunchKernelGGL(argmax_merge_kernel, dim3(1), dim3(256), 0, e->st, e->argmax_part, e->argmax_res);
 }
 
 // Before an FM pass: the time-projection table of the nfe-1 timesteps and
@@ -476,7 +478,7 @@ static void enqueue_fm_kernel(vx_engine *e, int l, int k, int nssq_attn) {
 // The input kernel of Euler step s.  noise_src: x_0 (step 0), or null for
 // the device generator (seed, kNoiseStream, frame counter).  sem_mask >= 0:
 // step 0 also takes the argmax of the semantic logits into sem_code, with
-// argmax_kernel's mask (8194: the greedy code's valid range; 0: unmasked).
+// argmax_block's mask (8194: the greedy code's valid range; 0: unmasked).
 static void enqueue_fm_step_in(vx_engine *e, int s, const float *noise_src, int sem_mask = -1) {
   const float alpha = e->cfg.cfg_alpha;
   const float dt = (float)(1.0 / (double)(e->cfg.nfe - 1));
@@ -1035,6 +1037,7 @@ int vx_create(const vx_config *cfg_in, int32_t max_seq, vx_engine **out) {
   aplace((void **)&e->sem_code, 4);
   aplace((void **)&e->codes, 64 * 4);
   aplace((void **)&e->argmax_res, 4);
+  aplace((void **)&e->argmax_part, AM_BLOCKS * sizeof(ArgmaxBest));
   aplace((void **)&e->noise_seed, 8);
   aplace((void **)&e->rng_state, 8);
   aplace((void **)&e->tp_params, 16);

@@ -17,7 +17,8 @@
 //                    flash decoding with a last-block log-sum-exp combine.
 //   fm_* kernels     biAttn* (:684-807), timeEmbedding (:579-602),
 //                    cfgCombine/eulerStep (:611-648), fsqQuantize (:653-673).
-//   argmax_kernel    argmax (:1154-1211), same 256-lane tree tie rule.
+//   argmax_block     argmax (:1154-1211), same 256-lane tree tie rule;
+//                    argmax_part_kernel, argmax_merge_kernel over many blocks.
 //   embed kernels    embeddingLookup (:193-213), multiCodebookEmbed
 //                    (:1878-1917).
 #pragma once
@@ -909,9 +910,54 @@ __device__ __forceinline__ void argmax_block(const float *x, int n, int mask_val
   }
   if (t == 0) result[0] = bi[0];
 }
-__global__ __launch_bounds__(256) void argmax_kernel(const float *x, int n, int mask_valid,
-                                                     uint32_t *result) {
-  argmax_block(x, n, mask_valid, result);
+
+// The same argmax over many blocks, for the LM head's 131072 logits (one block
+// took 23 us, these two launches 5).  The 256-lane rule above, as an order: of
+// the entries with the largest value (above -1e30; else entry 0) the tree
+// keeps the lane with the smallest bit-reversed number (its last step decides
+// on bit 0, the step before on bit 1, ...), and in the lane i % 256 the first.
+// So each block finds the best of its run under that order, and the second
+// kernel the best of the blocks.
+constexpr int AM_BLOCKS = 128;
+struct ArgmaxBest {
+  float v;
+  uint32_t i;
+};
+__device__ __forceinline__ bool argmax_before(float v, uint32_t i, float w, uint32_t j) {
+  if (v != w) return v > w;
+  const uint32_t a = __brev(i & 255u), b = __brev(j & 255u);
+  return a != b ? a < b : i < j;
+}
+// best of the block's 256 threads, in thread 0
+__device__ __forceinline__ ArgmaxBest argmax_reduce(ArgmaxBest b) {
+  __shared__ ArgmaxBest w[4];
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const float v = __shfl_xor(b.v, o, 64);
+    const uint32_t i = __shfl_xor(b.i, o, 64);
+    if (argmax_before(v, i, b.v, b.i)) b = {v, i};
+  }
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = b;
+  __syncthreads();
+  for (int q = 1; q < 4; q++)
+    if (argmax_before(w[q].v, w[q].i, b.v, b.i)) b = w[q];
+  return b;
+}
+// Grid: AM_BLOCKS of 256; an entry that no value beats is {-1e30, 0}
+__global__ __launch_bounds__(256) void argmax_part_kernel(const float *x, int n, ArgmaxBest *part) {
+  const int per = (n + AM_BLOCKS - 1) / AM_BLOCKS, i0 = blockIdx.x * per, i1 = min(n, i0 + per);
+  ArgmaxBest b = {-1e30f, 0};
+#pragma unroll 4
+  for (int i = i0 + threadIdx.x; i < i1; i += 256) {
+    const float v = x[i];
+    if (v > -1e30f && argmax_before(v, (uint32_t)i, b.v, b.i)) b = {v, (uint32_t)i};
+  }
+  b = argmax_reduce(b);
+  if (threadIdx.x == 0) part[blockIdx.x] = b;
+}
+__global__ __launch_bounds__(256) void argmax_merge_kernel(const ArgmaxBest *part, uint32_t *result) {
+  const ArgmaxBest b = argmax_reduce(threadIdx.x < AM_BLOCKS ? part[threadIdx.x] : ArgmaxBest{-1e30f, 0});
+  if (threadIdx.x == 0) *result = b.i;
 }
 
 // ------------------------------------------------------------- generator
@@ -1568,7 +1614,7 @@ struct FmStepArgs {
   const uint16_t *gn;    //   times its attention-norm gains,
   float *ssq_out;        //   and sums of squares, vector-major [FMV][SSQ_MAX]
   // step 0: a block past the grid's DIM / 256 takes the (masked) argmax of
-  // the semantic logits (argmax_kernel's work, off the FM's critical path)
+  // the semantic logits (off the FM's critical path)
   const float *sem_logits;
   int sem_mask;
   uint32_t *sem_code;
