@@ -133,13 +133,15 @@ struct vx_engine {
                  fm_greedy_exec = nullptr, fm_plain_exec = nullptr;
   bool use_graphs = true;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  // device top-p: its uniform stream and (top_p, temperature); a logits
-  // buffer for vx_sample_top_p; pinned per-frame readback slots
+  // device top-p: its uniform stream and (top_p, temperature); pinned
+  // per-frame readback slots
   uint64_t *rng_state = nullptr;
   double *tp_params = nullptr;
-  float *tp_logits = nullptr;
   uint32_t *h_frame = nullptr;  // [2][1 + NAC], pinned, written by the frame's last kernels
   uint32_t *d_frame = nullptr;  // h_frame's device address
+  // pinned staging of the calls' host operands and results (struct Stage):
+  // [0, STAGE_BYTES) in, then as much out
+  unsigned char *h_stage = nullptr, *d_stage = nullptr;
   hipEvent_t ev_frame[2] = {nullptr, nullptr};
   hipGraphExec_t fm_topp_exec = nullptr, frame_topp_exec = nullptr;
 
@@ -584,6 +586,72 @@ static int run_step_hold(vx_engine *e) {
   return run_seq(e, &e->hold_exec, enqueue_backbone_hold);
 }
 
+// ---------------------------------------------------------------- staging
+// A call's host operands and results cross the bus through pinned memory that
+// a small kernel on the engine's stream reads or writes.  hipMemcpyAsync on
+// the caller's pageable memory costs the host 10-20 us a copy (its own
+// staging, and a wait for each copy back), which a small call pays two to five
+// times: a two-layer step at 3900 positions took 144 us for 110 us of
+// kernels.  Every call that stages waits for the stream before it returns, so
+// the buffer is free at the next.
+constexpr size_t STAGE_BYTES = (size_t)1 << 20;  // each way; larger operands are copied as before
+
+// bytes: a multiple of 4; both addresses are 16-byte aligned
+__global__ __launch_bounds__(256) void stage_copy_kernel(const uint32_t *src, uint32_t *dst, int bytes) {
+  const int i = 4 * (blockIdx.x * 256 + threadIdx.x), left = bytes / 4 - i;
+  if (left >= 4) *(u32x4 *)(dst + i) = *(const u32x4 *)(src + i);
+  else
+    for (int q = 0; q < left; q++) dst[i + q] = src[i + q];
+}
+
+// One call's operands and results.  finish() waits for the stream and hands
+// the results over.
+struct Stage {
+  vx_engine *e;
+  size_t in_at = 0, out_at = 0;
+  int n = 0;
+  struct {
+    void *dst;
+    size_t at, bytes;
+  } outs[4];
+  explicit Stage(vx_engine *e_) : e(e_) {}
+  void copy(void *dst, const void *src, size_t bytes) {
+    hipLaunchKernelGGL(stage_copy_kernel, dim3((bytes + 4095) / 4096), dim3(256), 0, e->st, (const uint32_t *)src,
+                       (uint32_t *)dst, (int)bytes);
+  }
+  int in(void *dev, const void *src, size_t bytes) {
+    if (bytes == 0) return VX_OK;
+    if (bytes % 4 || in_at + bytes > STAGE_BYTES) {
+      HIPCHK(e, hipMemcpyAsync(dev, src, bytes, hipMemcpyHostToDevice, e->st));
+      return VX_OK;
+    }
+    memcpy(e->h_stage + in_at, src, bytes);
+    copy(dev, e->d_stage + in_at, bytes);
+    in_at += align256(bytes);
+    return VX_OK;
+  }
+  int out(void *dst, const void *dev, size_t bytes) {
+    if (bytes == 0) return VX_OK;
+    if (n == 4 || bytes % 4 || ((uintptr_t)dev & 15) || out_at + bytes > STAGE_BYTES) {
+      HIPCHK(e, hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, e->st));
+      return VX_OK;
+    }
+    const size_t at = STAGE_BYTES + out_at;
+    copy(e->d_stage + at, dev, bytes);
+    outs[n].dst = dst;
+    outs[n].at = at;
+    outs[n++].bytes = bytes;
+    out_at += align256(bytes);
+    return VX_OK;
+  }
+  int finish() {
+    LAUNCHCHK(e);
+    HIPCHK(e, hipStreamSynchronize(e->st));
+    for (int i = 0; i < n; i++) memcpy(outs[i].dst, e->h_stage + outs[i].at, outs[i].bytes);
+    return VX_OK;
+  }
+};
+
 // ---------------------------------------------------------------- helpers
 __global__ void set_int_kernel(int *p, int v) { *p = v; }
 __global__ void set_u32_kernel(uint32_t *p, const uint32_t v0) { *p = v0; }
@@ -612,7 +680,7 @@ static int prepare_input(vx_engine *e, int32_t token, int32_t mode, const float 
       break;
     case VX_EMBED_PRECOMPUTED:
       if (!pre) return fail(e, VX_E_INVALID, "precomputed embedding is NULL");
-      HIPCHK(e, hipMemcpyAsync(e->x, pre, DIM * sizeof(float), hipMemcpyHostToDevice, e->st));
+      if (int rc = Stage(e).in(e->x, pre, DIM * sizeof(float))) return rc;
       break;
     case VX_EMBED_CODES:
       hipLaunchKernelGGL(multi_codebook_kernel, dim3(DIM / 256), dim3(256), 0, e->st, e->audio_emb,
@@ -777,6 +845,12 @@ int vx_create(const vx_config *cfg_in, int32_t max_seq, vx_engine **out) {
       hipHostGetDevicePointer((void **)&e->d_frame, e->h_frame, 0) != hipSuccess) {
     vx_destroy(e);
     return fail(nullptr, VX_E_NOMEM, "hipHostMalloc of readback slots failed");
+  }
+  if (hipHostMalloc((void **)&e->h_stage, 2 * STAGE_BYTES, hipHostMallocMapped | hipHostMallocCoherent) !=
+          hipSuccess ||
+      hipHostGetDevicePointer((void **)&e->d_stage, e->h_stage, 0) != hipSuccess) {
+    vx_destroy(e);
+    return fail(nullptr, VX_E_NOMEM, "hipHostMalloc of the staging buffer failed");
   }
 
   // ---- weight table (names: src/engine.ts:659-743)
@@ -1041,7 +1115,6 @@ int vx_create(const vx_config *cfg_in, int32_t max_seq, vx_engine **out) {
   aplace((void **)&e->noise_seed, 8);
   aplace((void **)&e->rng_state, 8);
   aplace((void **)&e->tp_params, 16);
-  aplace((void **)&e->tp_logits, (size_t)TP_MAXN * 4);
   aplace((void **)&e->fm_seq, 6 * DIM * 4);
   aplace((void **)&e->fm_q, 6 * QD * 4);
   aplace((void **)&e->fm_k, 6 * KVD * 4);
@@ -1106,6 +1179,7 @@ void vx_destroy(vx_engine *e) {
   for (auto &ev : e->ev_frame)
     if (ev) (void)hipEventDestroy(ev);
   if (e->h_frame) (void)hipHostFree(e->h_frame);
+  if (e->h_stage) (void)hipHostFree(e->h_stage);
   if (e->fm_plain_exec) (void)hipGraphExecDestroy(e->fm_plain_exec);
   if (e->frame_exec) (void)hipGraphExecDestroy(e->frame_exec);
   if (e->warena) (void)hipFree(e->warena);
@@ -1335,12 +1409,10 @@ int vx_backbone_step(vx_engine *e, int32_t token, int32_t mode, const float *pre
     enqueue_lm_head(e);
     LAUNCHCHK(e);
   }
-  if (argmax_out && lm_head)
-    HIPCHK(e, hipMemcpyAsync(argmax_out, e->argmax_res, 4, hipMemcpyDeviceToHost, e->st));
-  if (normed_out)
-    HIPCHK(e, hipMemcpyAsync(normed_out, e->normed, DIM * 4, hipMemcpyDeviceToHost, e->st));
-  HIPCHK(e, hipStreamSynchronize(e->st));
-  return VX_OK;
+  Stage io(e);
+  if (argmax_out && lm_head && (rc = io.out(argmax_out, e->argmax_res, 4))) return rc;
+  if (normed_out && (rc = io.out(normed_out, e->normed, DIM * 4))) return rc;
+  return io.finish();
 }
 
 // One eager step that stages the reference's per-layer read points
@@ -1411,17 +1483,14 @@ int vx_fm_forward(vx_engine *e, const float *noise, float *sem_logits, uint32_t 
   int rc = check_ready(e);
   if (rc) return rc;
   if ((rc = ensure_tproj(e))) return rc;
-  if (noise) HIPCHK(e, hipMemcpyAsync(e->noise, noise, NAC * 4, hipMemcpyHostToDevice, e->st));
+  Stage io(e);
+  if (noise && (rc = io.in(e->noise, noise, NAC * 4))) return rc;
   enqueue_fm(e, noise ? e->noise : nullptr, false);
   LAUNCHCHK(e);
-  if (sem_logits)
-    HIPCHK(e, hipMemcpyAsync(sem_logits, e->sem_logits, SEMV * 4, hipMemcpyDeviceToHost, e->st));
-  if (codes) HIPCHK(e, hipMemcpyAsync(codes, e->codes, NAC * 4, hipMemcpyDeviceToHost, e->st));
-  if (x_final)
-    HIPCHK(e, hipMemcpyAsync(x_final, e->xh + (size_t)e->nsteps() * NAC, NAC * 4,
-                             hipMemcpyDeviceToHost, e->st));
-  HIPCHK(e, hipStreamSynchronize(e->st));
-  return VX_OK;
+  if (sem_logits && (rc = io.out(sem_logits, e->sem_logits, SEMV * 4))) return rc;
+  if (codes && (rc = io.out(codes, e->codes, NAC * 4))) return rc;
+  if (x_final && (rc = io.out(x_final, e->xh + (size_t)e->nsteps() * NAC, NAC * 4))) return rc;
+  return io.finish();
 }
 
 int vx_set_semantic_code(vx_engine *e, uint32_t code) {
@@ -1477,9 +1546,9 @@ int vx_read(vx_engine *e, const char *name, float *dst, size_t count) {
   for (auto &b : t)
     if (!strcmp(b.n, name)) {
       if (count > b.cnt) return fail(e, VX_E_INVALID, "%s holds %zu values", name, b.cnt);
-      HIPCHK(e, hipMemcpyAsync(dst, b.p, count * 4, hipMemcpyDeviceToHost, e->st));
-      HIPCHK(e, hipStreamSynchronize(e->st));
-      return VX_OK;
+      Stage io(e);
+      if (int rc = io.out(dst, b.p, count * 4)) return rc;
+      return io.finish();
     }
   return fail(e, VX_E_INVALID, "Unknown buffer: %s", name);
 }
@@ -1491,9 +1560,9 @@ int vx_write(vx_engine *e, const char *name, const float *src, size_t count) {
   else if (!strcmp(name, "hidden")) dst = e->x;
   else return fail(e, VX_E_INVALID, "Unknown writable buffer: %s", name);
   if (count > (size_t)DIM) return fail(e, VX_E_INVALID, "%s holds %d values", name, DIM);
-  HIPCHK(e, hipMemcpyAsync(dst, src, count * 4, hipMemcpyHostToDevice, e->st));
-  HIPCHK(e, hipStreamSynchronize(e->st));
-  return VX_OK;
+  Stage io(e);
+  if (int rc = io.in(dst, src, count * 4)) return rc;
+  return io.finish();
 }
 
 static uint16_t host_f2h(float f) {  // IEEE round-to-nearest-even
@@ -1684,7 +1753,7 @@ static int enqueue_prefill_chunk(vx_engine *e, int n, int tok0, int vstart, int 
                            nullptr, 0.f, nullptr);
     });
   }
-  (void)hipMemcpyAsync(e->x, e->pf_x + (size_t)(n - 1) * DIM, DIM * 4, hipMemcpyDeviceToDevice, st);
+  hipLaunchKernelGGL(copy_dim_kernel, dim3(DIM / 256), dim3(256), 0, st, e->pf_x + (size_t)(n - 1) * DIM, e->x);
   hipLaunchKernelGGL(final_norm_kernel, dim3(1), dim3(1024), 0, st, e->x, e->final_norm,
                      e->cfg.norm_eps, e->normed, nullptr, nullptr);
   hipLaunchKernelGGL(set_int_kernel, dim3(1), dim3(1), 0, st, e->pos, pos0 + n);
@@ -1711,21 +1780,20 @@ int vx_prefill(vx_engine *e, const int32_t *tokens, int32_t n_tokens, int32_t au
   const bool has_voice = voice && audio_count > 0;
   for (int c0 = 0; c0 < n_tokens; c0 += e->pf_chunk) {
     const int n = std::min(e->pf_chunk, n_tokens - c0);
-    HIPCHK(e, hipMemcpyAsync(e->pf_tok, tokens + c0, (size_t)n * 4, hipMemcpyHostToDevice, e->st));
+    Stage io(e);
+    if ((rc = io.in(e->pf_tok, tokens + c0, (size_t)n * 4))) return rc;
     // voice rows of this chunk, at chunk-local offsets
     int vs = 0, vc = 0;
     if (has_voice) {
       const int a = std::max(c0, audio_start), b = std::min(c0 + n, audio_start + audio_count);
       if (a < b) {
-        HIPCHK(e, hipMemcpyAsync(e->pf_voice, voice + (size_t)(a - audio_start) * DIM,
-                                 (size_t)(b - a) * DIM * 4, hipMemcpyHostToDevice, e->st));
+        if ((rc = io.in(e->pf_voice, voice + (size_t)(a - audio_start) * DIM, (size_t)(b - a) * DIM * 4))) return rc;
         vs = a;
         vc = b - a;
       }
     }
     if ((rc = enqueue_prefill_chunk(e, n, c0, vs, vc, vc > 0))) return rc;
-    LAUNCHCHK(e);
-    HIPCHK(e, hipStreamSynchronize(e->st));  // the host buffers above are reused per chunk
+    if ((rc = io.finish())) return rc;  // the host buffers above are reused per chunk
   }
   return VX_OK;
 }
@@ -1787,16 +1855,22 @@ int vx_sample_top_p(vx_engine *e, const float *logits, int32_t n, int32_t valid,
     *code = sample_top_p(l.data(), n, top_p, temperature, state);
     return VX_OK;
   }
+  // the kernel reads its operands from the pinned in half (33 KB, once) and
+  // leaves the code and the advanced generator state in the out half
+  constexpr size_t kParams = (size_t)TP_MAXN * 4, kState = kParams + 16;
+  static_assert(kParams % 16 == 0 && kState + 8 <= STAGE_BYTES, "staging layout");
   const double params[2] = {top_p, temperature};
-  HIPCHK(e, hipMemcpyAsync(e->tp_logits, logits, (size_t)n * 4, hipMemcpyHostToDevice, e->st));
-  HIPCHK(e, hipMemcpyAsync(e->tp_params, params, 16, hipMemcpyHostToDevice, e->st));
-  HIPCHK(e, hipMemcpyAsync(e->rng_state, state, 8, hipMemcpyHostToDevice, e->st));
-  hipLaunchKernelGGL(topp_sample_kernel, dim3(1), dim3(TP_NT), 0, e->st, e->tp_logits, n, valid,
-                     e->tp_params, e->rng_state, e->argmax_res, (const int *)nullptr, (uint32_t *)nullptr);
+  unsigned char *h = e->h_stage, *d = e->d_stage;
+  memcpy(h, logits, (size_t)n * 4);
+  memcpy(h + kParams, params, 16);
+  memcpy(h + kState, state, 8);
+  hipLaunchKernelGGL(topp_sample_kernel, dim3(1), dim3(TP_NT), 0, e->st, (const float *)d, n, valid,
+                     (const double *)(d + kParams), (uint64_t *)(d + kState), (uint32_t *)(d + STAGE_BYTES),
+                     (const int *)nullptr, (uint32_t *)nullptr);
   LAUNCHCHK(e);
-  HIPCHK(e, hipMemcpyAsync(code, e->argmax_res, 4, hipMemcpyDeviceToHost, e->st));
-  HIPCHK(e, hipMemcpyAsync(state, e->rng_state, 8, hipMemcpyDeviceToHost, e->st));
   HIPCHK(e, hipStreamSynchronize(e->st));
+  memcpy(code, h + STAGE_BYTES, 4);
+  memcpy(state, h + kState, 8);
   return VX_OK;
 }
 
@@ -2053,16 +2127,16 @@ static int codec_decode_impl(vx_engine *e, const uint32_t *semantic, const uint3
                 vx_codec_stop_count(n_frames, stop));
   if ((rc = codec_prepare(e)) || (rc = codec_reserve(e, n_frames)) || (rc = pf_gemm_setup(e)))
     return rc;
-  HIPCHK(e, hipMemcpyAsync(e->cx_sem, semantic, (size_t)n_frames * 4, hipMemcpyHostToDevice, e->st));
-  HIPCHK(e, hipMemcpyAsync(e->cx_ac, acoustic, (size_t)n_frames * NAC * 4, hipMemcpyHostToDevice,
-                           e->st));
+  Stage io(e);
+  if ((rc = io.in(e->cx_sem, semantic, (size_t)n_frames * 4)) ||
+      (rc = io.in(e->cx_ac, acoustic, (size_t)n_frames * NAC * 4)))
+    return rc;
   const float *res = nullptr;
   size_t count = 0;
   if ((rc = codec_run(e, n_frames, stop, &res, &count))) return rc;
   LAUNCHCHK(e);
-  HIPCHK(e, hipMemcpyAsync(out, res, count * 4, hipMemcpyDeviceToHost, e->st));
-  HIPCHK(e, hipStreamSynchronize(e->st));
-  return VX_OK;
+  if ((rc = io.out(out, res, count * 4))) return rc;
+  return io.finish();
 }
 
 size_t vx_codec_stop_count(int32_t n_frames, int32_t stop) {
