@@ -1720,12 +1720,11 @@ static int enqueue_prefill_chunk(vx_engine *e, int n, int tok0, int vstart, int 
   const int nt = gm_cols(n);
   hipStream_t st = e->st;
   const int pos0 = e->host_pos;
-  hipLaunchKernelGGL(pf_embed_kernel, dim3(n, DIM / 256), dim3(256), 0, st, e->tok_emb, e->pf_tok,
-                     has_voice ? e->pf_voice : nullptr, vstart, vcount, tok0, e->pf_x);
-  const dim3 blk(256);
-  // layer 0's B; every later B is written by the kernel producing its input
-  hipLaunchKernelGGL(pf_pack_kernel<true>, dim3(nt), blk, 0, st, e->pf_x, DIM, n, nt,
-                     e->L[0].attn_norm, e->cfg.norm_eps, e->pf_b);
+  // layer 0's B too; every later B is written by the kernel producing its input
+  hipLaunchKernelGGL(pf_embed_pack_kernel, dim3(nt), dim3(PF_ROW), 0, st, e->tok_emb, e->pf_tok,
+                     has_voice ? e->pf_voice : nullptr, vstart, vcount, tok0, n, nt, e->pf_x, e->L[0].attn_norm,
+                     e->cfg.norm_eps, e->pf_b);
+  const dim3 row(PF_ROW);
   for (int l = 0; l < e->cfg.n_layers; l++) {
     const LayerW &W = e->L[l];
     const bool next = l + 1 < e->cfg.n_layers;
@@ -1734,7 +1733,7 @@ static int enqueue_prefill_chunk(vx_engine *e, int n, int tok0, int vstart, int 
     else enqueue_pf_attn<uint16_t>(e, l, pos0, n, nt, ns);
     if ((rc = pf_gemm(e, W.wo, DIM, QD, nt, n, &ns))) return rc;
     gm_with_slices(ns, [&](auto NS) {
-      hipLaunchKernelGGL((pf_resid_pack_kernel<true, NS>), dim3(nt), blk, 0, st, e->pf_c, n, nt, e->pf_x,
+      hipLaunchKernelGGL((pf_resid_pack_kernel<true, NS>), dim3(nt), row, 0, st, e->pf_c, n, nt, e->pf_x,
                          W.ffn_norm, e->cfg.norm_eps, e->pf_b);
     });
     // W1 and W3 are adjacent in the arena: one GEMM over the stacked rows
@@ -1746,10 +1745,10 @@ static int enqueue_prefill_chunk(vx_engine *e, int n, int tok0, int vstart, int 
     if ((rc = pf_gemm(e, W.w2, DIM, HID, nt, n, &ns))) return rc;
     gm_with_slices(ns, [&](auto NS) {
       if (next)
-        hipLaunchKernelGGL((pf_resid_pack_kernel<true, NS>), dim3(nt), blk, 0, st, e->pf_c, n, nt, e->pf_x,
+        hipLaunchKernelGGL((pf_resid_pack_kernel<true, NS>), dim3(nt), row, 0, st, e->pf_c, n, nt, e->pf_x,
                            e->L[l + 1].attn_norm, e->cfg.norm_eps, e->pf_b);
       else
-        hipLaunchKernelGGL((pf_resid_pack_kernel<false, NS>), dim3(n), blk, 0, st, e->pf_c, n, nt, e->pf_x,
+        hipLaunchKernelGGL((pf_resid_pack_kernel<false, NS>), dim3(n), row, 0, st, e->pf_c, n, nt, e->pf_x,
                            nullptr, 0.f, nullptr);
     });
   }

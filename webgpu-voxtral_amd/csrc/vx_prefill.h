@@ -48,52 +48,6 @@ __device__ __forceinline__ f32x4 pf_c4(const float *C, int ldc, int nt, int t, i
 }
 
 // ------------------------------------------------------- per-token kernels
-// X[t] = token embedding row, or voice row v = t + tok0 - vstart for the
-// tokens inside [vstart, vstart + vcount) (src/engine.ts:2457-2472)
-__global__ void pf_embed_kernel(const uint16_t *table, const int32_t *tokens, const float *voice,
-                                int vstart, int vcount, int tok0, float *X) {
-  const int t = blockIdx.x, i = blockIdx.y * blockDim.x + threadIdx.x;
-  const int gi = tok0 + t;
-  float v;
-  if (voice && gi >= vstart && gi < vstart + vcount)
-    v = voice[(size_t)(gi - vstart) * DIM + i];
-  else
-    v = h2f(table[(size_t)tokens[t] * DIM + i]);
-  X[(size_t)t * DIM + i] = v;
-}
-
-// B columns t and nt + t (K halves each) from row t of X, optionally
-// RMS-normalised with gains g (rmsNorm, src/shaders.ts:137-183); columns of
-// tokens t >= n are zero.  Grid: nt blocks of 256.
-template <bool NORM>
-__global__ __launch_bounds__(256) void pf_pack_kernel(const float *X, int K, int n, int nt,
-                                                      const uint16_t *g, float eps, h8 *B) {
-  const int t = blockIdx.x, tid = threadIdx.x;
-  const float *x = X + (size_t)t * K;
-  float r = 1.0f;
-  if (NORM && t < n) {
-    __shared__ float red[4];
-    float s = 0.f;
-    for (int k = tid; k < K; k += 256) s = fmaf(x[k], x[k], s);
-    s = wave_sum(s);
-    if ((tid & 63) == 0) red[tid >> 6] = s;
-    __syncthreads();
-    r = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)K + eps);
-  }
-  for (int kb = tid; kb < K / 8; kb += 256) {
-    h8 hi, lo;
-    float y[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const int k = kb * 8 + e;
-      y[e] = t < n ? (NORM ? x[k] * r * h2f(g[k]) : x[k]) : 0.f;
-    }
-    split_n<8>(y, hi, lo);
-    B[(size_t)t * (K / 8) + kb] = hi;
-    B[(size_t)(nt + t) * (K / 8) + kb] = lo;
-  }
-}
-
 // hi/lo halves of y into B columns t and nt + t at k (8 consecutive k)
 __device__ __forceinline__ void pf_put8(h8 *B, int K, int nt, int t, int kb, const float (&y)[8]) {
   h8 hi, lo;
@@ -102,55 +56,95 @@ __device__ __forceinline__ void pf_put8(h8 *B, int K, int nt, int t, int kb, con
   B[(size_t)(nt + t) * (K / 8) + kb] = lo;
 }
 
+// The rows of a prompt are DIM = 384 groups of 8 values: a block of 384 threads
+// holds one row, so every load of it is in flight at once and its sum of
+// squares costs one barrier.  (256 threads, half of them with a second group
+// behind the first: 7 us at 256 tokens for the residual, 8 us for the packing
+// of the embeddings in a kernel of its own.)
+constexpr int PF_ROW = DIM / 8;
+static_assert(PF_ROW == 6 * 64, "one 8-value group per thread");
+
+// B columns t and nt + t from rmsNorm(v) * g (src/shaders.ts:137-183), v the
+// row's 8 values of this thread
+__device__ __forceinline__ void pf_norm_pack(const float (&v)[8], const uint16_t *g, float eps, int nt, int t, h8 *B) {
+  __shared__ float red[6];
+  const int kb = threadIdx.x;
+  const h8 gv = *(const h8 *)(g + kb * 8);
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e++) ss = fmaf(v[e], v[e], ss);
+  ss = wave_sum_dpp(ss);
+  if ((kb & 63) == 0) red[kb >> 6] = ss;
+  __syncthreads();
+  const float r =
+      1.0f / sqrtf((((red[0] + red[1]) + (red[2] + red[3])) + (red[4] + red[5])) / (float)DIM + eps);
+  float y[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) y[e] = v[e] * r * (float)gv[e];
+  pf_put8(B, DIM, nt, t, kb, y);
+}
+__device__ __forceinline__ void pf_zero_pack(int nt, int t, h8 *B) {
+  const float y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  pf_put8(B, DIM, nt, t, threadIdx.x, y);
+}
+
+// X[t] = token embedding row, or voice row v = t + tok0 - vstart for the
+// tokens inside [vstart, vstart + vcount) (src/engine.ts:2457-2472), and the
+// first layer's B from it; columns of tokens t >= n are zero.
+// Grid: nt blocks of PF_ROW.
+__global__ __launch_bounds__(PF_ROW) void pf_embed_pack_kernel(const uint16_t *table, const int32_t *tokens,
+                                                               const float *voice, int vstart, int vcount, int tok0,
+                                                               int n, int nt, float *X, const uint16_t *g, float eps,
+                                                               h8 *B) {
+  const int t = blockIdx.x, i = 8 * threadIdx.x, gi = tok0 + t;
+  if (t >= n) {
+    pf_zero_pack(nt, t, B);
+    return;
+  }
+  float v[8];
+  if (voice && gi >= vstart && gi < vstart + vcount) {
+    const float *p = voice + (size_t)(gi - vstart) * DIM + i;
+    const f32x4 a = *(const f32x4 *)p, b = *(const f32x4 *)(p + 4);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      v[e] = a[e];
+      v[4 + e] = b[e];
+    }
+  } else {
+    const h8 w = *(const h8 *)(table + (size_t)tokens[t] * DIM + i);
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = (float)w[e];
+  }
+  float *x = X + (size_t)t * DIM + i;
+  *(f32x4 *)x = f32x4{v[0], v[1], v[2], v[3]};
+  *(f32x4 *)(x + 4) = f32x4{v[4], v[5], v[6], v[7]};
+  pf_norm_pack(v, g, eps, nt, t, B);
+}
+
 // Residual add of a DIM-row GEMM output, X[t] += y (addInPlace,
 // src/shaders.ts:532-547), then, with PACK, the next GEMM's B from
-// rmsNorm(X[t]) * g (src/shaders.ts:137-183); columns of tokens t >= n are
-// zero.  Grid: nt blocks (n without PACK) of 256; thread i owns the 8-value
-// groups i and i + 256 (DIM / 8 = 384 groups).
+// rmsNorm(X[t]) * g; columns of tokens t >= n are zero.
+// Grid: nt blocks (n without PACK) of PF_ROW.
 template <bool PACK, int NS>
-__global__ __launch_bounds__(256) void pf_resid_pack_kernel(const float *C, int n, int nt, float *X,
-                                                            const uint16_t *g, float eps, h8 *B) {
-  constexpr int NG = DIM / 8, GPT = (NG + 255) / 256;
-  const int t = blockIdx.x, tid = threadIdx.x;
-  float v[GPT][8];
-  float ss = 0.f;
-  if (t < n) {
-#pragma unroll
-    for (int i = 0; i < GPT; i++) {
-      const int kb = tid + 256 * i;
-      if (kb < NG) {
-        float *x = X + (size_t)t * DIM + kb * 8;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-          const f32x4 xv = *(const f32x4 *)(x + 4 * h), a = pf_c4<NS>(C, DIM, nt, t, kb * 8 + 4 * h);
-#pragma unroll
-          for (int e = 0; e < 4; e++) v[i][4 * h + e] = xv[e] + a[e];
-          *(f32x4 *)(x + 4 * h) = f32x4{v[i][4 * h], v[i][4 * h + 1], v[i][4 * h + 2], v[i][4 * h + 3]};
-        }
-#pragma unroll
-        for (int e = 0; e < 8; e++) ss = fmaf(v[i][e], v[i][e], ss);
-      }
-    }
+__global__ __launch_bounds__(PF_ROW) void pf_resid_pack_kernel(const float *C, int n, int nt, float *X,
+                                                               const uint16_t *g, float eps, h8 *B) {
+  const int t = blockIdx.x, i = 8 * threadIdx.x;
+  if (t >= n) {
+    if (PACK) pf_zero_pack(nt, t, B);
+    return;
   }
-  if (!PACK) return;
-  float r = 0.f;
-  if (t < n) {
-    __shared__ float red[4];
-    ss = wave_sum(ss);
-    if ((tid & 63) == 0) red[tid >> 6] = ss;
-    __syncthreads();
-    r = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)DIM + eps);
-  }
+  float *x = X + (size_t)t * DIM + i;
+  const f32x4 xa = *(const f32x4 *)x, xb = *(const f32x4 *)(x + 4);
+  const f32x4 a = pf_c4<NS>(C, DIM, nt, t, i), b = pf_c4<NS>(C, DIM, nt, t, i + 4);
+  float v[8];
 #pragma unroll
-  for (int i = 0; i < GPT; i++) {
-    const int kb = tid + 256 * i;
-    if (kb < NG) {
-      float y[8];
-#pragma unroll
-      for (int e = 0; e < 8; e++) y[e] = t < n ? v[i][e] * r * h2f(g[kb * 8 + e]) : 0.f;
-      pf_put8(B, DIM, nt, t, kb, y);
-    }
+  for (int e = 0; e < 4; e++) {
+    v[e] = xa[e] + a[e];
+    v[4 + e] = xb[e] + b[e];
   }
+  *(f32x4 *)x = f32x4{v[0], v[1], v[2], v[3]};
+  *(f32x4 *)(x + 4) = f32x4{v[4], v[5], v[6], v[7]};
+  if (PACK) pf_norm_pack(v, g, eps, nt, t, B);
 }
 
 // SwiGLU of the stacked [W1; W3] output (ldc = 2 HID; swiGLU,
