@@ -1403,62 +1403,71 @@ __device__ __forceinline__ uint64_t tp_mass(uint64_t key) {
 // pub (or null): the frame's host-visible code slots [2][1 + NAC] (pinned
 // host memory); the code also goes to slot (*frame - 1) & 1, the slot
 // fm_finish_kernel filled for this frame before it advanced *frame.
+// The thread's entries i = tid + 1024 j stay in registers from the load to the
+// picked key, so all nine loads are in flight at once (they may come from
+// host memory) and the passes read no keys from LDS.  A call on 8320 host
+// logits takes 39 us, the kernel 27.6 of them; with the entries in LDS, one
+// load after the other and two f64 divisions an entry it took 48 us.
+
+// x / d, correctly rounded, for rd = 1 / d: one Newton step on the quotient
+// with its exact remainder (Markstein); x / d itself where that could leave
+// the normal range
+__device__ __forceinline__ double tp_div(double x, double d, double rd, bool plain) {
+  const double q = x * rd, y = fma(fma(-q, d, x), rd, q);
+  return plain || !(fabs(q) < 1e300) ? x / d : y;
+}
+
 __global__ __launch_bounds__(TP_NT) void topp_sample_kernel(const float *logits, int n, int valid,
                                                             const double *params, uint64_t *rng,
                                                             uint32_t *out, const int *frame, uint32_t *pub) {
-  const double top_p = params[0], temp = params[1];  // in device memory: graphs stay valid
-  __shared__ uint64_t key[TP_MAXN];       // first holds s_i, then p_i, as floats
-  __shared__ uint64_t bmass[TP_BINS];     // also the f64 tree of the p sum
+  constexpr int PER = TP_MAXN / TP_NT;
+  __shared__ uint64_t bmass[TP_BINS];
   __shared__ uint32_t bcnt[TP_BINS];
   __shared__ uint64_t wsum[TP_WAVES];
-  __shared__ double red[TP_WAVES];
+  __shared__ double red[TP_WAVES], red2[TP_WAVES];
   __shared__ uint64_t sel_base, sel_incl, sel_key, target;
   __shared__ int sel;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  float *sv = reinterpret_cast<float *>(key);
+  const double top_p = params[0], temp = params[1];  // in device memory: graphs stay valid
+  const uint64_t rng0 = tid == 0 ? *rng : 0;
+  float pv[PER];
+#pragma unroll
+  for (int j = 0; j < PER; j++) pv[j] = logits[min(tid + j * TP_NT, n - 1)];
   // s_i and the max
+  const double rtemp = 1.0 / temp;
+  const bool odd_temp = !(temp > 1e-200 && temp < 1e200);
   double mx = -INFINITY;
-  for (int i = tid; i < n; i += TP_NT) {
-    const float si = (i > 0 && i < valid) ? (float)((double)logits[i] / temp) : -INFINITY;
-    sv[i] = si;
-    mx = fmax(mx, (double)si);
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const int i = tid + j * TP_NT;
+    pv[j] = i > 0 && i < valid && i < n ? (float)tp_div((double)pv[j], temp, rtemp, odd_temp) : -INFINITY;
+    mx = fmax(mx, (double)pv[j]);
   }
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
   if (lane == 0) red[wave] = mx;
   __syncthreads();
   mx = red[0];
   for (int w = 1; w < TP_WAVES; w++) mx = fmax(mx, red[w]);
-  // p_i and their sum in f64: per thread, then a tree
-  double *part = reinterpret_cast<double *>(bmass);
+  // p_i and their sum in f64: per thread, per wave, then the waves in order
   double s = 0.0;
-  for (int i = tid; i < n; i += TP_NT) {
-    const float pi = (float)exp((double)sv[i] - mx);
-    sv[i] = pi;
-    s += (double)pi;
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    pv[j] = tid + j * TP_NT < n ? (float)exp((double)pv[j] - mx) : 0.f;
+    s += (double)pv[j];
   }
-  part[tid] = s;
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (lane == 0) red2[wave] = s;
   __syncthreads();
-  for (int o = TP_NT / 2; o > 0; o >>= 1) {
-    if (tid < o) part[tid] += part[tid + o];
-    __syncthreads();
-  }
-  const double sum = part[0];
-  // keys (each thread first reads its p_i: keys overwrite the floats)
-  constexpr int PER = TP_MAXN / TP_NT;
-  float pv[PER];
+  double sum = red2[0];
+  for (int w = 1; w < TP_WAVES; w++) sum += red2[w];
+  const double rsum = 1.0 / sum;
+  const bool odd_sum = !(sum > 1e-200 && sum < 1e200);
+  uint64_t key[PER];  // ~0: no such entry (its mass and every digit are never looked at)
 #pragma unroll
   for (int j = 0; j < PER; j++) {
     const int i = tid + j * TP_NT;
-    pv[j] = i < n ? sv[i] : 0.f;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < PER; j++) {
-    const int i = tid + j * TP_NT;
-    if (i < n) {
-      const float q = (float)((double)pv[j] / sum);
-      key[i] = ((uint64_t)(0x7FFFFFFFu - __builtin_bit_cast(uint32_t, q)) << 14) | (uint32_t)i;
-    }
+    const float q = (float)tp_div((double)pv[j], sum, rsum, odd_sum);
+    key[j] = i < n ? ((uint64_t)(0x7FFFFFFFu - __builtin_bit_cast(uint32_t, q)) << 14) | (uint32_t)i : ~0ull;
   }
   // smallest key K with mass(keys <= K) >= t; returns K and that mass, or
   // found = false when the total mass stays below t
@@ -1473,8 +1482,9 @@ __global__ __launch_bounds__(TP_NT) void topp_sample_kernel(const float *logits,
       }
       if (tid == 0) sel = TP_BINS;
       __syncthreads();
-      for (int i = tid; i < n; i += TP_NT) {
-        const uint64_t k = key[i];
+#pragma unroll
+      for (int j = 0; j < PER; j++) {
+        const uint64_t k = key[j];
         if ((k >> hi) == prefix) {
           const int d = (int)((k >> shift) & (uint64_t)(nb - 1));
           atomicAdd((unsigned long long *)&bmass[d], (unsigned long long)tp_mass(k));
@@ -1525,8 +1535,9 @@ __global__ __launch_bounds__(TP_NT) void topp_sample_kernel(const float *logits,
       if (bcnt[ds] == 1) {
         // one key carries this prefix: the later passes would select its
         // digits with the same inclusive mass, so it is the answer
-        for (int i = tid; i < n; i += TP_NT)
-          if ((key[i] >> shift) == prefix) sel_key = key[i];
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+          if ((key[j] >> shift) == prefix) sel_key = key[j];
         __syncthreads();
         kout = sel_key;
         __syncthreads();  // every thread has read sel_key
@@ -1549,7 +1560,9 @@ __global__ __launch_bounds__(TP_NT) void topp_sample_kernel(const float *logits,
     for (int b = tid; b < TP_BINS; b += TP_NT) bmass[b] = 0;
     __syncthreads();
     uint64_t m = 0;
-    for (int i = tid; i < n; i += TP_NT) m += tp_mass(key[i]);
+#pragma unroll
+    for (int j = 0; j < PER; j++)
+      if (key[j] != ~0ull) m += tp_mass(key[j]);
     atomicAdd((unsigned long long *)&bmass[0], (unsigned long long)m);
     __syncthreads();
     resum = bmass[0];
@@ -1557,7 +1570,8 @@ __global__ __launch_bounds__(TP_NT) void topp_sample_kernel(const float *logits,
   }
   // draw: t = ceil(u * resum) with u = u53 * 2^-53, exactly
   if (tid == 0) {
-    uint64_t z = (*rng += 0x9E3779B97F4A7C15ull);
+    uint64_t z = rng0 + 0x9E3779B97F4A7C15ull;
+    *rng = z;
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     z ^= z >> 31;
