@@ -263,6 +263,82 @@ __global__ __launch_bounds__(128) void cx_resid_pack_kernel(const float *C, int 
   cx_put(B, nc, CD / 8, kb, t, y);
 }
 
+// The same residual at the end of a stage, and the next conv's packed rows
+// (cx_pack_rows_kernel) from the row while the block holds it: row before + t
+// of B is X[t], times conv_scale if given; the rows before the first step and
+// past the last are zero.  For a stage of one chunk.  Grid: before + nt blocks
+// of 128.
+template <int NS>
+__global__ __launch_bounds__(128) void cx_resid_rows_kernel(const float *C, int nc, int n, const uint16_t *scale,
+                                                            float *X, const float *conv_scale, int before, size_t blo,
+                                                            h8 *B) {
+  const int t = (int)blockIdx.x - before, kb = threadIdx.x;
+  float y[8];
+  if (t >= 0 && t < n) {
+    float *x = X + (size_t)t * CD + kb * 8;
+    float xv[8], sc[8];
+    cx_load8(x, xv);
+    cx_load8h(scale + kb * 8, sc);
+    cx_val8<NS>(C, CD, nc, t, kb * 8, y);
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = y[e] * sc[e] + xv[e];
+    *(f32x4 *)x = f32x4{y[0], y[1], y[2], y[3]};
+    *(f32x4 *)(x + 4) = f32x4{y[4], y[5], y[6], y[7]};
+    if (conv_scale) {
+      cx_load8(conv_scale + kb * 8, sc);
+#pragma unroll
+      for (int e = 0; e < 8; e++) y[e] = sc[e] * y[e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = 0.f;
+  }
+  h8 hi, lo;
+  split_n<8>(y, hi, lo);
+  B[(size_t)blockIdx.x * (CD / 8) + kb] = hi;
+  B[blo / 8 + (size_t)blockIdx.x * (CD / 8) + kb] = lo;
+}
+
+// A conv's output rows, and the next stage's first B from each while the block
+// holds it (cx_pack_kernel): UP, the transposed conv: step to = 2 t + r is rows
+// r CD .. of column t; else the input conv, scaled per row.  n, nc: the
+// output's steps and columns; nci: the conv chunk's columns.  For outputs of
+// one chunk.  Grid: nc / 2 blocks of 128.
+template <bool UP, int NS>
+__global__ __launch_bounds__(128) void cx_conv_pack_kernel(const float *C, int nci, const float *rs, int n, int nc,
+                                                           float *X, const uint16_t *g, float eps, h8 *B) {
+  const int to = blockIdx.x, kb = threadIdx.x;
+  float y[8];
+  if (to < n) {
+    __shared__ float red[2];
+    const int t = UP ? to >> 1 : to, m = (UP ? (to & 1) * CD : 0) + kb * 8;
+    cx_val8<NS>(C, UP ? 2 * CD : CD, nci, t, m, y);
+    if (!UP) {
+      float sc[8];
+      cx_load8(rs + kb * 8, sc);
+#pragma unroll
+      for (int e = 0; e < 8; e++) y[e] = sc[e] * y[e];
+    }
+    float *x = X + (size_t)to * CD + kb * 8;
+    *(f32x4 *)x = f32x4{y[0], y[1], y[2], y[3]};
+    *(f32x4 *)(x + 4) = f32x4{y[4], y[5], y[6], y[7]};
+    float ss = 0.f, gv[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) ss = fmaf(y[e], y[e], ss);
+    ss = wave_sum(ss);
+    if ((kb & 63) == 0) red[kb >> 6] = ss;
+    __syncthreads();
+    const float r = 1.0f / sqrtf((red[0] + red[1]) / (float)CD + eps);
+    cx_load8h(g + kb * 8, gv);
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = y[e] * r * gv[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = 0.f;
+  }
+  cx_put(B, nc, CD / 8, kb, to, y);
+}
+
 // SwiGLU of the stacked gate/up projection (batchedSwiGLU,
 // src/shaders.ts:1697-1716), written as the packed B of the down projection
 // (k = hidden unit).  Grid: (nt, CHID / 8 / 256) of 256; columns t >= n are 0.

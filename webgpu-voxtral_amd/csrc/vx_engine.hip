@@ -2020,10 +2020,19 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
     int ns = 1;
     if (!rc) rc = cx_gemm(e, e->cx_ain, CD, CKIN, nc, n, &ns);
     gm_with_slices(ns, [&](auto NS) {
-      hipLaunchKernelGGL(cx_scale_rows_epi_kernel<NS>, dim3(n, CD / 256), blk, 0, st, e->cx_c, CD, nc, t0,
-                         e->cx_rs_in, CD, e->cx_x, CD);
+      if (n == T)
+        hipLaunchKernelGGL((cx_conv_pack_kernel<false, NS>), dim3(nc / 2), dim3(128), 0, st, e->cx_c, nc,
+                           e->cx_rs_in, n, nc, e->cx_x, w.L[0][0].attn_norm, CX_NORM_EPS, e->cx_b);
+      else
+        hipLaunchKernelGGL(cx_scale_rows_epi_kernel<NS>, dim3(n, CD / 256), blk, 0, st, e->cx_c, CD, nc, t0,
+                           e->cx_rs_in, CD, e->cx_x, CD);
     });
   });
+  // In an utterance of one chunk per stage, each conv's epilogue packs the
+  // next stage's first B and each stage's last residual the next conv's rows
+  // (8 launches fewer); a stage of several chunks has one B for all of them
+  // and packs chunk by chunk.
+  bool packed = T <= e->cx_chunk;
   int TT = T, at = VX_CODEC_STOP_INPUT_CONV;
   float *x = e->cx_x, *x2 = e->cx_x2;
   static const int kWindow[CX_STAGES] = {2, 4, 8, 16};  // src/engine.ts:1507
@@ -2032,9 +2041,12 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
     // chunk needs of it, the last keys and values of each layer, is its halo
     // (two per layer, written and read in turn)
     int parity = 0;
+    const bool whole = TT <= e->cx_chunk;
+    const int before = s < CX_STAGES - 1 ? 1 : CK_OUT - 1;  // rows of the next conv before a step's own
     chunks(TT, [&](int t0, int n, int nc) {
-      hipLaunchKernelGGL(cx_pack_kernel, dim3(nc / 2), blk, 0, st, x, CD, t0, n, nc, w.L[s][0].attn_norm,
-                         CX_NORM_EPS, e->cx_b);
+      if (!packed)
+        hipLaunchKernelGGL(cx_pack_kernel, dim3(nc / 2), blk, 0, st, x, CD, t0, n, nc, w.L[s][0].attn_norm,
+                           CX_NORM_EPS, e->cx_b);
       for (int l = 0; l < CX_LPS; l++) {
         const CodecLayerW &L = w.L[s][l];
         const size_t halo = (size_t)CX_HALO * 2 * CD;
@@ -2063,6 +2075,10 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
           if (l + 1 < CX_LPS)
             hipLaunchKernelGGL((cx_resid_pack_kernel<true, NS>), dim3(nc / 2), dim3(128), 0, st, e->cx_c, nc, t0,
                                n, L.ffn_scale, x, w.L[s][l + 1].attn_norm, CX_NORM_EPS, e->cx_b);
+          else if (whole)
+            hipLaunchKernelGGL(cx_resid_rows_kernel<NS>, dim3(before + nc / 2), dim3(128), 0, st, e->cx_c, nc, n,
+                               L.ffn_scale, x, s < CX_STAGES - 1 ? e->cx_s_up[s] : nullptr, before,
+                               (size_t)(before + nc / 2) * CD, e->cx_b);
           else
             hipLaunchKernelGGL((cx_resid_pack_kernel<false, NS>), dim3(n), dim3(128), 0, st, e->cx_c, nc, t0, n,
                                L.ffn_scale, x, nullptr, 0.f, nullptr);
@@ -2075,12 +2091,19 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
     // ConvTranspose1d(1024 -> 1024, k = 4, stride 2), output trimmed to 2 TT
     chunks(TT, [&](int t0, int n, int nc) {
       const int rows = nc / 2 + 1;
-      hipLaunchKernelGGL(cx_pack_rows_kernel, dim3(rows), dim3(128), 0, st, x, e->cx_s_up[s], 1, t0, n,
-                         (size_t)rows * CD, e->cx_b);
+      if (!whole)
+        hipLaunchKernelGGL(cx_pack_rows_kernel, dim3(rows), dim3(128), 0, st, x, e->cx_s_up[s], 1, t0, n,
+                           (size_t)rows * CD, e->cx_b);
       int ns = 1;
       if (!rc) rc = cx_gemm(e, e->cx_aup[s], 2 * CD, CKUP, nc, n, &ns, rows);
+      packed = 2 * TT <= e->cx_chunk;
+      const int nco = 2 * gm_cols(2 * n);
       gm_with_slices(ns, [&](auto NS) {
-        hipLaunchKernelGGL(cx_up_epi_kernel<NS>, dim3(n, 2 * CD / 256), blk, 0, st, e->cx_c, nc, t0, x2);
+        if (packed)
+          hipLaunchKernelGGL((cx_conv_pack_kernel<true, NS>), dim3(nco / 2), dim3(128), 0, st, e->cx_c, nc,
+                             (const float *)nullptr, 2 * n, nco, x2, w.L[s + 1][0].attn_norm, CX_NORM_EPS, e->cx_b);
+        else
+          hipLaunchKernelGGL(cx_up_epi_kernel<NS>, dim3(n, 2 * CD / 256), blk, 0, st, e->cx_c, nc, t0, x2);
       });
     });
     std::swap(x, x2);
@@ -2097,8 +2120,9 @@ static int codec_run(vx_engine *e, int T, int stop, const float **res, size_t *c
   // [240 t, 240 t + 240)
   chunks(TT, [&](int t0, int n, int nc) {
     const int rows = nc / 2 + CK_OUT - 1;
-    hipLaunchKernelGGL(cx_pack_rows_kernel, dim3(rows), dim3(128), 0, st, x, (const float *)nullptr, CK_OUT - 1, t0,
-                       n, (size_t)rows * CD, e->cx_b);
+    if (TT > e->cx_chunk)
+      hipLaunchKernelGGL(cx_pack_rows_kernel, dim3(rows), dim3(128), 0, st, x, (const float *)nullptr, CK_OUT - 1,
+                         t0, n, (size_t)rows * CD, e->cx_b);
     int ns = 1;
     if (!rc) rc = cx_gemm(e, e->cx_aout, CPATCH_ROWS, CKOUT, nc, n, &ns, rows);
     gm_with_slices(ns, [&](auto NS) {
