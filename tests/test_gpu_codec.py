@@ -76,6 +76,15 @@ def test_chunked_gemms(oracle_codec):
         g.destroy()
 
 
+@pytest.mark.parametrize("T", [17, 40])
+def test_column_tiles_of_the_thin_grid(engine, oracle_codec, T):
+    """17 frames (136 steps in the last stage, 192 columns) and 40 (320): the
+    output conv's 256 rows run in 3 and 5 column tiles of the thin grid, the
+    other products where the grids change over; every stage, the same bar."""
+    print(f"[codec] {T} frames, all intermediates", flush=True)
+    check_all(engine, oracle_codec, *random_codes(T, 100 + T))
+
+
 def test_chunks_hand_on_their_last_keys(oracle_codec):
     """33 frames in 128-token chunks: stage 2 runs 132 tokens in two chunks
     (window 8) and stage 3 264 in three (window 16), so each of both layers'

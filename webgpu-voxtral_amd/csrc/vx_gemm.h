@@ -276,11 +276,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-// Thin grid, for chunks of at most GT_MAXN columns: the product is then bound
+// Thin grid, for chunks of few columns: the product is then bound
 // by the weight stream (two flops per weight byte and column), so what
 // matters is bytes in flight on every CU and few bytes of everything else.
-// Block (x, s): BM = 32 RT weight rows, K slice s of gridDim.y, all NT
-// columns.  A k-tile's BM + 2 NT rows are staged as above (ring of S stages,
+// Block (x, s, z): BM = 32 RT weight rows, K slice s of gridDim.y, columns
+// z NT .. + NT (all of them, up to GT_MAXN).  A k-tile's BM + 2 NT rows are staged as above (ring of S stages,
 // 48-72 KB, so two or three blocks share a CU and one's barriers run under
 // the others' loads), but the four waves split the k-tile's 64 halves, 16
 // each, instead of its rows: every staged byte is read from LDS once (rows
@@ -335,7 +335,8 @@ __global__ __launch_bounds__(256) void gemm_thin_kernel(const uint16_t *__restri
   constexpr int S = G::S;
   extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, h = lane >> 5;
-  const int m0 = blockIdx.x * G::BM, nk = K / GM_BK;
+  const int m0 = blockIdx.x * G::BM, nk = K / GM_BK, col0 = blockIdx.z * NT;
+  B += (size_t)col0 * ldb;
   const int k0 = (int)(blockIdx.y * nk / gridDim.y), cnt = (int)((blockIdx.y + 1) * nk / gridDim.y) - k0;
   // direct load i of this wave fills stage rows 8 (4 i + wave) .. + 8: weight
   // rows for i < RT, then the B rows (hi, lo)
@@ -396,7 +397,7 @@ __global__ __launch_bounds__(256) void gemm_thin_kernel(const uint16_t *__restri
     fill = fill + 1 == S ? 0 : fill + 1;
   }
   float *red = (float *)gm_smem;
-  C += (size_t)blockIdx.y * NT * ldc;
+  C += ((size_t)blockIdx.y * gridDim.z * NT + col0) * ldc;
 #pragma unroll
   for (int i = 0; i < RT; i++) {
     __syncthreads();
@@ -409,7 +410,7 @@ __global__ __launch_bounds__(256) void gemm_thin_kernel(const uint16_t *__restri
     __syncthreads();
     for (int o = tid; o < NT * 8; o += 256) {
       const int col = o >> 3, m = 4 * (o & 7);
-      if (col < n) {
+      if (col0 + col < n) {
         gm_f32x4 v = *(const gm_f32x4 *)(red + col * G::RW + m);
 #pragma unroll
         for (int w = 1; w < 4; w++) v += *(const gm_f32x4 *)(red + (w * 2 * NT + col) * G::RW + m);
@@ -472,8 +473,8 @@ inline int gemm_share_slices(int m_tiles, int nk, int L) {
 inline GemmPlan gemm_thin_plan(int M, int K, int nt, int cus) {
   GemmPlan p;
   const int nk = K / GM_BK;
-  p.thin = nt == 64 || M / 64 * 8 >= 3 * cus ? 2 : 1;
-  const int blocks = M / (32 * p.thin);
+  p.thin = nt >= 64 || M / 64 * 8 >= 3 * cus ? 2 : 1;
+  const int blocks = M / (32 * p.thin) * (nt > GT_MAXN ? nt / GT_MAXN : 1);
   while (p.ks < 8 && blocks * p.ks * 2 * 2 <= 9 * cus &&
          nk / (p.ks * 2) >= (blocks * p.ks < cus ? 2 : 4))
     p.ks *= 2;
@@ -526,9 +527,14 @@ inline GemmPlan gemm_tiled_plan(int M, int K, int nt, int cus, size_t c_cap) {
 }
 
 // cus: the device's compute units (8 XCDs).  Shapes must satisfy
-// M % 256 == 0, K % 64 == 0, nt = gm_cols(n).
+// M % 256 == 0, K % 64 == 0, nt = gm_cols(n).  From 64 columns on the thin grid
+// is the faster one for outputs of up to 2^17 elements, whose few 256-row
+// tiles leave the device idle (GEMM and a reader of C, us, thin / tiled: 2048 x
+// 2048 at 64 columns 11.2 / 13.0, 1024 x 4096 at 128 12.5 / 15.7, 256 x 7168 at
+// 256 13.7 / 19.2), and about equal or slower past that (1024 x 1024 at 192
+// 12.4 / 12.0, 3072 x 1024 at 64 12.5 / 12.4, at 192 17.4 / 15.1).
 inline GemmPlan gemm_plan(int M, int K, int nt, int cus, size_t c_cap) {
-  if (nt < GT_MAXN || (nt == GT_MAXN && M <= 2048)) return gemm_thin_plan(M, K, nt, cus);
+  if (nt < GT_MAXN || (size_t)M * nt <= (size_t)1 << 17) return gemm_thin_plan(M, K, nt, cus);
   return gemm_tiled_plan(M, K, nt, cus, c_cap);
 }
 
@@ -572,8 +578,8 @@ inline hipError_t gemm_setup() {
 inline void gemm_launch(const GemmPlan &p, hipStream_t st, const uint16_t *W, int M, int K, const uint16_t *B,
                         int ldb, size_t blo, int nt, int n, float *C) {
   if (p.thin)
-    gm_with_thin(p.thin, nt, (size_t)M * K >= (size_t)8 << 20, [&](auto kernel, int lds) {
-      hipLaunchKernelGGL(kernel, dim3(M / (32 * p.thin), p.ks), dim3(256), lds, st, W, K, B, ldb, blo, n, C, M);
+    gm_with_thin(p.thin, std::min(nt, GT_MAXN), (size_t)M * K >= (size_t)8 << 20, [&](auto kernel, int lds) {
+      hipLaunchKernelGGL(kernel, dim3(M / (32 * p.thin), p.ks, std::max(nt / GT_MAXN, 1)), dim3(256), lds, st, W, K, B, ldb, blo, n, C, M);
     });
   else if (p.wide)
     hipLaunchKernelGGL(gemm_kernel<GmWide>, dim3(p.grid), dim3(512), GmWide::LDS, st, W, M, K, B, ldb, blo, nt, C, M,
