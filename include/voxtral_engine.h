@@ -158,7 +158,7 @@ int vx_backbone_step(vx_engine *e, int32_t token, int32_t embed_mode,
 /* The prefill loop of generate(), src/engine.ts:2457-2472 (one
  * backboneStep per prompt token, voice rows replacing the embeddings of
  * tokens [audio_start, audio_start + audio_count)), run as batched MFMA
- * GEMMs over chunks of up to 256 tokens from the current position.  Leaves
+ * GEMMs over chunks of up to 1024 tokens from the current position.  Leaves
  * the KV cache, the residual stream, W.normed (last token) and the position
  * as n_tokens single steps would (no LM head).  voice: f32[audio_count][dim]
  * or NULL. */

@@ -492,3 +492,22 @@ def test_lm_head_argmax_ties():
             assert top in ties and top == O.argmax(logits), (ties, top)
     finally:
         g.destroy()
+
+
+@pytest.mark.parametrize("count", [1, 5, 64, 3071])
+def test_partial_reads_and_writes_stay_in_bounds(count):
+    """Operands cross through a staging copy of 16-byte words: a write of
+    `count` values leaves the rest of the buffer, a read of `count` the rest of
+    the caller's array."""
+    g = gpu_engine(n_layers=1, max_seq=32)
+    try:
+        base = np.arange(3072, dtype=np.float32)
+        g.debug_write("hidden", base)
+        g.debug_write("hidden", -1 - base[:count])
+        assert np.array_equal(g.debug_read("hidden", 3072),
+                              np.concatenate([-1 - base[:count], base[count:]]))
+        out = np.full(count + 8, 7.0, np.float32)
+        g._check(g._lib.vx_read(g._h, b"hidden", out.ctypes.data, count))
+        assert np.array_equal(out, np.concatenate([-1 - base[:count], np.full(8, 7.0, np.float32)]))
+    finally:
+        g.destroy()

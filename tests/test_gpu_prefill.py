@@ -1,4 +1,4 @@
-"""Batched prefill (vx_prefill: MFMA GEMMs over chunks of up to 256 tokens)
+"""Batched prefill (vx_prefill: MFMA GEMMs over chunks of up to 1024 tokens)
 against the reference semantics, one backboneStep per prompt token
 (src/engine.ts:2457-2472), as restated by the oracle: the KV cache of every
 layer, the last token's W.normed and the position afterwards, with voice
@@ -36,7 +36,7 @@ def check_kv(g, o, layers, npos, bar=1e-3):
 @pytest.mark.parametrize("n,a_start,a_count,layers", [(40, 5, 8, 2), (7, 0, 0, 2), (256, 2, 64, 2),
                                                     (520, 100, 218, 1)])
 def test_prefill_matches_single_steps(n, a_start, a_count, layers):
-    """One chunk: GEMM columns sized to the prompt (2 x n rounded up to 128)."""
+    """One chunk: GEMM columns sized to the prompt (16, 32 or a multiple of 64, hi and lo)."""
     print(f"[prefill] {layers} layers, {n} tokens, voice rows {a_start}+{a_count}", flush=True)
     g = gpu_engine(n_layers=layers, max_seq=1024)
     o = oracle_engine(n_layers=layers, max_seq=1024)

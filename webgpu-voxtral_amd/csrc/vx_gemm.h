@@ -291,8 +291,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // order and only the live columns col < n are written.  NTW: the weight loads
 // carry the non-temporal hint, as each weight is read by one block only.
 // Weights cycled from HBM, all of M x K = 18432 x 3072 (113 MB): 16 columns
-// 21.6 us (23.8 without the hint), 32 columns 26.7 us, where the split grid
-// takes 54 us (at its 128 columns) and the decode GEMV 18.4 us for one;
+// 21.6 us (23.8 without the hint), 32 columns 26.7 us, where the tiled grid
+// took 54 us (at its 128 columns) and the decode GEMV 18.4 us for one;
 // 3072 x 9216: 11.7 and 14.0 us against 25; 1024 x 1024: 2.6 and 2.8 us
 // against 6.5.
 constexpr int GT_MAXN = 64;
