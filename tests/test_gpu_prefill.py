@@ -215,6 +215,33 @@ def test_prefill_context_ends_inside_a_key_tile(pos0, n, kv_f16):
         o.close()
 
 
+@pytest.mark.parametrize("bad", [16, 29, 32])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("kv_f16", [False, True])
+def test_non_finite_token_leaves_earlier_blocks(kv_f16, value, bad):
+    """A token whose input is not finite makes its own K/V rows so; the
+    attention's blocks of 16 tokens before it hide those keys, and 0 times
+    their values must stay 0: every layer's rows of the earlier blocks are
+    bit-equal to those of the prompt without it."""
+    n = 50
+    print(f"[prefill] {n} tokens, token {bad} is {value}, f16 KV {kv_f16}", flush=True)
+    g = gpu_engine(n_layers=2, max_seq=64, kv_f16=kv_f16)
+    try:
+        x = np.random.default_rng(bad).standard_normal((n, 3072)).astype(np.float32)
+        first = bad // 16 * 16  # of the bad token's block
+        g.prefill(np.full(n, 24), 0, n, x)
+        want = [g.read_kv(l, w, 0, first) for l in (0, 1) for w in (0, 1)]
+        x[bad] = value
+        g.position = 0
+        g.prefill(np.full(n, 24), 0, n, x)
+        got = [g.read_kv(l, w, 0, first) for l in (0, 1) for w in (0, 1)]
+        assert not np.isfinite(g.read_kv(0, 1, bad, 1)).all()
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b)
+    finally:
+        g.destroy()
+
+
 def test_prefill_argument_errors():
     import voxtral_amd as V
     g = gpu_engine(n_layers=1, max_seq=64)

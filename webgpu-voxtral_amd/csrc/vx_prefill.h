@@ -437,6 +437,27 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     if (it + PFA_KG < ntile) load_tile(it + PFA_KG, (i + 1) & 1);
+    // The last tile's keys past kend are later blocks', hidden from every token
+    // of this one, but 0 times a value that is not finite is NaN: they are
+    // zeroed, two of the eight fragments by each wave, 8 slots a lane, key
+    // 16 kt + 4 grp + q in slot 4 kt + q.  (A token that is not finite still
+    // reaches the up to 15 before it in its own block.)  In LDS and not on the
+    // fragments as they are read: a second copy of the product's loop takes 140
+    // registers, past the 128 that let two blocks share a CU.  Prompts of 9 to
+    // 1300 tokens take what they took (within 1%).
+    if (i == iters - 1 && kend % PFA_K) {  // uniform over the block
+      if (it == ntile - 1) {
+        u32x4 keep, *f = (u32x4 *)(ring + (i & 1) * TILE + (EXACT ? 1 : 2) * PFA_PART) + 2 * hw * 64 + lane;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int key = kb + 16 * (j >> 1) + 4 * grp + 2 * (j & 1);
+          keep[j] = (key < kend ? 0xFFFFu : 0u) | (key + 1 < kend ? 0xFFFF0000u : 0u);
+        }
+#pragma unroll
+        for (int k = 0; k < (EXACT ? 2 : 4); k++) f[(k & 1) * 64 + (k >> 1) * (PFA_PART / 16)] &= keep;
+      }
+      __syncthreads();
+    }
     if (it >= ntile) continue;  // uniform over the group
     const h8 *kh = (const h8 *)(ring + (i & 1) * TILE) + lane, *kl = kh + PFA_PART / 16;
     const h8 *vh = kh + (EXACT ? 1 : 2) * (PFA_PART / 16), *vl = vh + PFA_PART / 16;
