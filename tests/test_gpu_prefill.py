@@ -7,6 +7,7 @@ import os
 
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 from vxtest import gpu_engine, max_rel_err, oracle_engine, tts_prompt, voice_rows
@@ -213,6 +214,81 @@ def test_prefill_context_ends_inside_a_key_tile(pos0, n, kv_f16):
     finally:
         g.destroy()
         o.close()
+
+
+SHAPES = {"attention_norm": (3072,), "attention.wq": (4096, 3072), "attention.wk": (1024, 3072),
+          "attention.wv": (1024, 3072), "attention.wo": (3072, 4096), "ffn_norm": (3072,),
+          "feed_forward.w1": (9216, 3072), "feed_forward.w3": (9216, 3072), "feed_forward.w2": (3072, 9216)}
+
+
+def weight_name(layer, part):
+    return f"layers.{layer}.{part}.weight"
+
+
+def layer_f64(g, layer, x, full=True):
+    """One backbone layer over the rows x [n][3072] at positions 0 .. n - 1 in
+    64-bit torch on the engine's weights: (attention's contribution to each
+    row, output rows, K rows, V rows); the first two are None without `full`."""
+    def w(part):
+        bits = g.read_tensor(weight_name(layer, part), int(np.prod(SHAPES[part])))
+        return torch.from_numpy(bits.view(np.float16).astype(np.float64)).reshape(SHAPES[part])
+
+    def norm(x, part):
+        return x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-5) * w(part)
+
+    def rope(y):
+        ang = torch.arange(n, dtype=torch.float64)[:, None] * 1e6 ** (-torch.arange(0, 128, 2, dtype=torch.float64) / 128)
+        c, s = torch.cos(ang)[:, None], torch.sin(ang)[:, None]
+        y = y.reshape(n, -1, 64, 2)
+        return torch.stack([y[..., 0] * c - y[..., 1] * s, y[..., 0] * s + y[..., 1] * c], -1).reshape(n, -1)
+
+    n = x.shape[0]
+    h = norm(x, "attention_norm")
+    k, v = rope(h @ w("attention.wk").t()), h @ w("attention.wv").t()
+    if not full:
+        return None, None, k.numpy(), v.numpy()
+    q = rope(h @ w("attention.wq").t())
+    hide = torch.ones((n, n), dtype=torch.bool).tril().logical_not()
+    a = torch.empty_like(q)
+    for i in range(32):
+        qi, ki, vi = q[:, 128 * i:128 * i + 128], k[:, i // 4 * 128:i // 4 * 128 + 128], v[:, i // 4 * 128:i // 4 * 128 + 128]
+        a[:, 128 * i:128 * i + 128] = torch.softmax((qi @ ki.t() / 128 ** 0.5).masked_fill(hide, -np.inf), -1) @ vi
+    a = a @ w("attention.wo").t()
+    x = x + a
+    h = norm(x, "ffn_norm")
+    f = torch.nn.functional.silu(h @ w("feed_forward.w1").t()) * (h @ w("feed_forward.w3").t())
+    return a.numpy(), x + f @ w("feed_forward.w2").t(), k.numpy(), v.numpy()
+
+
+def rel_l2(got, ref):
+    return float(np.linalg.norm(np.asarray(got, np.float64) - ref) / np.linalg.norm(ref))
+
+
+def test_prompt_attention_small_queries():
+    """Queries around 0.02 against keys around 140, so that scores are of
+    order 1 although the queries' lo halves are f16 subnormals: their quantum,
+    2^-24, must be the query's own and not that of a scaled-down one.  The
+    attention's contribution to the last token against 64 bits.  Bound: a lo
+    half is off by up to 2^-25, 1.7e-8 rms, against 0.02 a 1e-6 relative error
+    of each term and so about that of a score; scores of 2-3 make it 3e-6 of
+    the probabilities.  Seen: 1.8e-6, and 1.5e-5 where the queries were split in
+    units of 0.13."""
+    n = 64
+    print(f"[prefill] {n} tokens, small queries", flush=True)
+    g = gpu_engine(n_layers=1, max_seq=96)
+    try:
+        for part, by in (("attention.wq", 1 / 64), ("attention.wk", 128.0), ("feed_forward.w2", 0.0)):
+            bits = g.read_tensor(weight_name(0, part), int(np.prod(SHAPES[part])))
+            g.load_tensor(weight_name(0, part), (bits.view(np.float16) * np.float16(by)).view(np.uint16).reshape(SHAPES[part]))
+        x = np.random.default_rng(4).standard_normal((n, 3072)).astype(np.float32)
+        g.prefill(np.full(n, 24), 0, n, x)
+        a, _, k, _ = layer_f64(g, 0, torch.from_numpy(x).double())
+        assert rel_l2(g.read_kv(0, 0, 0, n), k) < 1e-6
+        err = rel_l2(g.debug_read("hidden", 3072).astype(np.float64) - x[-1], a[-1])
+        print(f"[prefill] small queries: {err:.3g}", flush=True)
+        assert err < 5e-6
+    finally:
+        g.destroy()
 
 
 @pytest.mark.parametrize("bad", [16, 29, 32])

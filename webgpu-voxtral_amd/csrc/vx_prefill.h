@@ -408,18 +408,24 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
   };
   if (grp_k < ntile) load_tile(grp_k, 0);
 
-  // Q^T operand of S^T (token t, dims 32c + 8grp..+8), hi and lo, in units
-  // that make a score log2(e) / sqrt(128) q.k (the softmax is of powers of
-  // two); padding tokens zero
+  // The softmax is of powers of two, exp2(s scale - m) with m the largest s
+  // scale: v_exp_f32 is off by 8.3e-8 at most and 2.0e-8 rms over [-126, 0], as
+  // expf is (4.7 M arguments), and flushes what is below 2^-126, of sums of at
+  // least 1.  The scale is applied to the score, in the exponent's fma, not to
+  // q: a query is split in its own units, since lo halves of a q smaller by
+  // 0.13 reach the f16 subnormals, whose quantum is fixed (queries of 0.02
+  // against keys of 140: error of the attention 1.5e-5, and 1.8e-6 this way).
+  const float scale = 1.44269504f / sqrtf((float)HD);
+  // Q^T operand of S^T (token t, dims 32c + 8grp..+8), hi and lo; padding
+  // tokens zero
   h8 qh[HD / 32], ql[HD / 32];
   {
-    const float scale = 1.44269504f / sqrtf((float)HD);
     const float *qp = Q + (size_t)min(t, n - 1) * QD + h * HD + 8 * grp;
 #pragma unroll
     for (int c = 0; c < HD / 32; c++) {
       f32x4 a = *(const f32x4 *)(qp + 32 * c), b = *(const f32x4 *)(qp + 32 * c + 4);
       if (t >= n) a = b = f32x4{0.f, 0.f, 0.f, 0.f};
-      split8(a * scale, b * scale, qh[c], ql[c]);
+      split8(a, b, qh[c], ql[c]);
     }
   }
   float m = -INFINITY, l = 0.f;
@@ -486,7 +492,7 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
       if (edge && kb + 16 * (q >> 2) + 4 * grp + (q & 3) > last) p[q] = -INFINITY;
       mx = fmaxf(mx, p[q]);
     }
-    mx = pfa_max4(mx);
+    mx = pfa_max4(mx) * scale;
     if (__builtin_amdgcn_ballot_w64(mx > m)) {  // some token's maximum grows
       // a token whose keys all lie before this tile's start keeps m = -inf
       // (only in groups other than 0: key 0 <= last is in tile 0)
@@ -501,7 +507,7 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
     float ps = 0.f;
 #pragma unroll
     for (int q = 0; q < 8; q++) {
-      p[q] = __builtin_amdgcn_exp2f(p[q] - base);  // hidden keys: 0
+      p[q] = __builtin_amdgcn_exp2f(fmaf(p[q], scale, -base));  // hidden keys: 0
       ps += p[q];
     }
     l += pfa_sum4(ps);
