@@ -408,8 +408,8 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
   };
   if (grp_k < ntile) load_tile(grp_k, 0);
 
-  // The softmax is of powers of two, exp2(s scale - m) with m the largest s
-  // scale: v_exp_f32 is off by 8.3e-8 at most and 2.0e-8 rms over [-126, 0], as
+  // The softmax is of powers of two, exp2(s scale - ms) with ms = m scale, m the
+  // largest s: v_exp_f32 is off by 8.3e-8 at most and 2.0e-8 rms over [-126, 0], as
   // expf is (4.7 M arguments), and flushes what is below 2^-126, of sums of at
   // least 1.  The scale is applied to the score, in the exponent's fma, not to
   // q: a query is split in its own units, since lo halves of a q smaller by
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
       split8(a, b, qh[c], ql[c]);
     }
   }
-  float m = -INFINITY, l = 0.f;
+  float m = -INFINITY, ms = -INFINITY, l = 0.f;
   f32x4 o[HD / 16];
 #pragma unroll
   for (int dt = 0; dt < HD / 16; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -440,30 +440,28 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
     // other stage any more
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    if (it == ntile - 1 && kend % PFA_K) {
+      // The last tile's keys past kend are later blocks', hidden from every
+      // token of this one, but 0 times a value that is not finite is NaN: each
+      // lane zeroes those of the 16 bytes of V^T it brought, fragments hw and
+      // hw + 4, whose slot 4 kt + q is key 16 kt + 4 grp + q.  (A token that is
+      // not finite still reaches the up to 15 before it in its own block.)  Here
+      // it needs no barrier of its own; with one, after this one, it took 0.9 us
+      // of 13.8 at 256 tokens, and masks on the fragments as the product reads
+      // them cost registers past the 128 that let two blocks share a CU.
+      u32x4 keep, *f = (u32x4 *)(ring + (i & 1) * TILE + (EXACT ? 1 : 2) * PFA_PART) + hw * 64 + lane;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int key = kb + 16 * (j >> 1) + 4 * grp + 2 * (j & 1);
+        keep[j] = (key < kend ? 0xFFFFu : 0u) | (key + 1 < kend ? 0xFFFF0000u : 0u);
+      }
+#pragma unroll
+      for (int k = 0; k < (EXACT ? 2 : 4); k++) f[k * 256] &= keep;  // hi, then lo
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    }
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     if (it + PFA_KG < ntile) load_tile(it + PFA_KG, (i + 1) & 1);
-    // The last tile's keys past kend are later blocks', hidden from every token
-    // of this one, but 0 times a value that is not finite is NaN: they are
-    // zeroed, two of the eight fragments by each wave, 8 slots a lane, key
-    // 16 kt + 4 grp + q in slot 4 kt + q.  (A token that is not finite still
-    // reaches the up to 15 before it in its own block.)  In LDS and not on the
-    // fragments as they are read: a second copy of the product's loop takes 140
-    // registers, past the 128 that let two blocks share a CU.  Prompts of 9 to
-    // 1300 tokens take what they took (within 1%).
-    if (i == iters - 1 && kend % PFA_K) {  // uniform over the block
-      if (it == ntile - 1) {
-        u32x4 keep, *f = (u32x4 *)(ring + (i & 1) * TILE + (EXACT ? 1 : 2) * PFA_PART) + 2 * hw * 64 + lane;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int key = kb + 16 * (j >> 1) + 4 * grp + 2 * (j & 1);
-          keep[j] = (key < kend ? 0xFFFFu : 0u) | (key + 1 < kend ? 0xFFFF0000u : 0u);
-        }
-#pragma unroll
-        for (int k = 0; k < (EXACT ? 2 : 4); k++) f[(k & 1) * 64 + (k >> 1) * (PFA_PART / 16)] &= keep;
-      }
-      __syncthreads();
-    }
     if (it >= ntile) continue;  // uniform over the group
     const h8 *kh = (const h8 *)(ring + (i & 1) * TILE) + lane, *kl = kh + PFA_PART / 16;
     const h8 *vh = kh + (EXACT ? 1 : 2) * (PFA_PART / 16), *vl = vh + PFA_PART / 16;
@@ -492,18 +490,19 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
       if (edge && kb + 16 * (q >> 2) + 4 * grp + (q & 3) > last) p[q] = -INFINITY;
       mx = fmaxf(mx, p[q]);
     }
-    mx = pfa_max4(mx) * scale;
+    mx = pfa_max4(mx);
     if (__builtin_amdgcn_ballot_w64(mx > m)) {  // some token's maximum grows
       // a token whose keys all lie before this tile's start keeps m = -inf
       // (only in groups other than 0: key 0 <= last is in tile 0)
-      const float mnew = fmaxf(m, mx);
-      const float corr = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mnew);
-      m = mnew;
+      m = fmaxf(m, mx);
+      const float msnew = m * scale;
+      const float corr = msnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(ms - msnew);
+      ms = msnew;
       l *= corr;
 #pragma unroll
       for (int dt = 0; dt < HD / 16; dt++) o[dt] = o[dt] * corr;
     }
-    const float base = m == -INFINITY ? 0.f : m;
+    const float base = ms == -INFINITY ? 0.f : ms;
     float ps = 0.f;
 #pragma unroll
     for (int q = 0; q < 8; q++) {
@@ -528,7 +527,7 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
   __syncthreads();  // every group is done with its stages
   if (grp_k > 0) {
     float *r = red + ((grp_k - 1) * 4 + hw) * PFA_RED * 64 + lane;
-    r[0] = m;
+    r[0] = ms;
     r[64] = l;
 #pragma unroll
     for (int dt = 0; dt < HD / 16; dt++)
@@ -537,17 +536,17 @@ __global__ __launch_bounds__(256 * PFA_KG) void pf_attn_mfma_kernel(const float 
   }
   __syncthreads();
   if (grp_k > 0) return;
-  float mm = m;
+  float mm = ms;
 #pragma unroll
   for (int g = 1; g < PFA_KG; g++) mm = fmaxf(mm, red[((g - 1) * 4 + hw) * PFA_RED * 64 + lane]);
-  const float c0 = __builtin_amdgcn_exp2f(m - mm);  // m is finite in group 0
+  const float c0 = __builtin_amdgcn_exp2f(ms - mm);  // ms is finite in group 0
   l *= c0;
 #pragma unroll
   for (int dt = 0; dt < HD / 16; dt++) o[dt] = o[dt] * c0;
 #pragma unroll
   for (int g = 1; g < PFA_KG; g++) {
     const float *rg = red + ((g - 1) * 4 + hw) * PFA_RED * 64 + lane;
-    const float cg = __builtin_amdgcn_exp2f(rg[0] - mm);  // m = -inf: 0
+    const float cg = __builtin_amdgcn_exp2f(rg[0] - mm);  // ms = -inf: 0
     l += rg[64] * cg;
 #pragma unroll
     for (int dt = 0; dt < HD / 16; dt++)
