@@ -8,6 +8,7 @@ import os
 import numpy as np
 import pytest
 
+import codec_f64
 import oracle as O
 import voxtral_amd as V
 from vxtest import SEED, STD, gpu_engine, max_rel_err
@@ -99,6 +100,27 @@ def test_chunks_hand_on_their_last_keys(oracle_codec):
         check_all(g, oracle_codec, *random_codes(33, 33))
     finally:
         g.destroy()
+
+
+def test_long_decode_at_the_default_chunk(engine, oracle_codec):
+    """150 frames, 1200 steps in the last stage: its 1024-step chunk takes the
+    256 x 128 tiles and hands its keys on, and the stages before it are one
+    chunk each, so the packing passes from the convs' epilogues to the chunks.
+    Every stage's end against 64 bits.  The audio's bar lies between the 2-norm
+    errors seen with hi and lo products in sums of their own (1.61e-6) and with
+    one sum for both, which rounds twice as often (1.87e-6, and at 250 frames
+    more with fewer K slices)."""
+    T = 150
+    print(f"[codec] {T} frames at the default chunk", flush=True)
+    sem, ac = random_codes(T, T)
+    ref = codec_f64.decode({n: oracle_codec.weight(n) for n in oracle_codec.names()}, sem, ac)
+    for name in V.CODEC_STOPS:
+        got = engine.codec_decode_to(sem, ac, name).ravel().astype(np.float64)
+        r = ref[name].ravel()
+        err = np.linalg.norm(got - r) / np.linalg.norm(r)
+        print(f"[codec] {name}: {err:.4g}", flush=True)
+        assert max_rel_err(got, r) < BAR, name
+    assert name == "audio" and err < 1.75e-6
 
 
 def test_codes_outside_the_tables(engine, oracle_codec):

@@ -453,13 +453,14 @@ __global__ __launch_bounds__(64 * CXA_WAVES) void cx_attn_kernel(const float *C,
       const int key = t - W + 1 + j;                    // this lane's key, LDS row qi + j
       const bool in = j < W && t0 + key >= 0;
       const float *kr = ks + (in ? qi + j : qi + W - 1) * CXA_LD + 4 * p, *qr = qs + qi * CXA_LD + 4 * p;
-      float dot = 0.f;
+      f32x4 d4 = f32x4{0.f, 0.f, 0.f, 0.f};  // four sums of 8: in one of 32 the scores are a few ulps further off
 #pragma unroll
       for (int i = 0; i < CHDIM / 16; i++) {
         const f32x4 a = *(const f32x4 *)(qr + 16 * i), b = *(const f32x4 *)(kr + 16 * i);
 #pragma unroll
-        for (int e = 0; e < 4; e++) dot = fmaf(a[e], b[e], dot);
+        for (int e = 0; e < 4; e++) d4[e] = fmaf(a[e], b[e], d4[e]);
       }
+      float dot = (d4[0] + d4[1]) + (d4[2] + d4[3]);
       dot += __shfl_xor(dot, 1, 64);
       dot += __shfl_xor(dot, 2, 64);
       const float sc = in ? dot * scale - slope * (float)(t - key) : -INFINITY;

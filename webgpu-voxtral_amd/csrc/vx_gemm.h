@@ -5,16 +5,19 @@
 // B + col ldb, its f16 residual (lo) from B + blo + col ldb (16-byte
 // aligned), as the producer kernels write them.  ldb = K for packed
 // columns; a causal convolution's columns overlap (ldb = channels, K = taps x
-// channels), so its input is packed once and not once per tap.  Hi and lo go through the same MFMA
-// accumulator, so the product keeps f32 accuracy.  The K range is split
+// channels), so its input is packed once and not once per tap.  Hi and lo both go through MFMA with f32
+// accumulators, so the product keeps f32 accuracy.  The K range is split
 // into S_out slices whose partial sums land in S_out consecutive [nt][M]
 // blocks of C; the consumer adds them (fixed order, so results are
 // deterministic).
 //
 // Tiles: 256 weight rows x CN columns (2 CN B rows: hi and lo) per block of
 // eight waves.  Four compute: wave w owns 32 RT weight rows and 64 columns, as
-// RT x 2 tiles of v_mfma_f32_32x32x16_f16 (hi and lo accumulate into the same
-// tile).  Four load: a k-tile is 64 halves, 128 bytes of each of the 256 + 2 CN
+// RT x 2 tiles of v_mfma_f32_32x32x16_f16, hi and lo in sums of their own for
+// the 256 x 64 tile, added at the end (the lo products then don't round the hi
+// sum a second time in each step: error of a 250-frame codec decode against 64
+// bits 1.93e-6 in one sum, 1.64e-6 in two, at the same time), in one sum for the
+// 256 x 128 tile, whose registers hold no second.  Four load: a k-tile is 64 halves, 128 bytes of each of the 256 + 2 CN
 // rows, brought to LDS by direct loads (global_load_lds_dwordx4, 1 KB per
 // instruction = 8 rows) into a ring of DA weight stages and DB stages of B.
 //
@@ -72,6 +75,7 @@ __device__ __forceinline__ void gm_direct(const uint16_t *src, unsigned char *ld
 template <int RT_, int WC_, int DA_, int DB_>
 struct GmShape {
   static constexpr int RT = RT_, WC = WC_, DA = DA_, DB = DB_;
+  static constexpr int SUMS = RT == 2 ? 2 : 1;        // accumulators per tile: hi and lo, or one for both
   static constexpr int CN = GM_BN * WC;               // columns per tile
   static constexpr int ASTAGE = GM_BM * GM_ROWB;      // 32 KB
   static constexpr int BSTAGE = 2 * CN * GM_ROWB;     // 16 KB per 64 columns
@@ -82,30 +86,33 @@ struct GmShape {
 using GmNarrow = GmShape<2, 1, 3, 3>;  // 256 x 64, 144 KB
 using GmWide = GmShape<4, 2, 3, 2>;    // 256 x 128, 160 KB: the weights, which come from HBM, two k-tiles ahead
 
-template <int RT>
-__device__ __forceinline__ void gm_mfma(gm_f32x16 (&acc)[RT][2], const gm_h8 (&fr)[RT + 4]) {
+template <int SUMS, int RT>
+__device__ __forceinline__ void gm_mfma(gm_f32x16 (&acc)[SUMS][RT][2], const gm_h8 (&fr)[RT + 4]) {
 #pragma unroll
   for (int hl = 0; hl < 2; hl++)
 #pragma unroll
     for (int i = 0; i < RT; i++)
 #pragma unroll
       for (int j = 0; j < 2; j++)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[i], fr[RT + 2 * hl + j], acc[i][j], 0, 0, 0);
+        acc[hl % SUMS][i][j] =
+            __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[i], fr[RT + 2 * hl + j], acc[hl % SUMS][i][j], 0, 0, 0);
 }
 
-// acc[i][j][e] is weight row 32 i + 8 (e / 4) + 4 h + e % 4 of the wave's,
-// column 32 j + r: written as C[col][m] with float4 stores
-template <int RT>
-__device__ __forceinline__ void gm_store(const gm_f32x16 (&acc)[RT][2], float *cp, int ldc, bool zero) {
+// acc[.][i][j][e] is weight row 32 i + 8 (e / 4) + 4 h + e % 4 of the wave's,
+// column 32 j + r: the sums added and written as C[col][m] with float4 stores
+template <int SUMS, int RT>
+__device__ __forceinline__ void gm_store(const gm_f32x16 (&acc)[SUMS][RT][2], float *cp, int ldc, bool zero) {
 #pragma unroll
   for (int i = 0; i < RT; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int j = 0; j < 2; j++) {
+      gm_f32x16 v = acc[0][i][j];
+      if (SUMS == 2) v += acc[SUMS - 1][i][j];
 #pragma unroll
       for (int g4 = 0; g4 < 4; g4++)
         *(gm_f32x4 *)(cp + (size_t)j * 32 * ldc + i * 32 + 8 * g4) =
-            zero ? gm_f32x4{0.f, 0.f, 0.f, 0.f}
-                 : gm_f32x4{acc[i][j][4 * g4], acc[i][j][4 * g4 + 1], acc[i][j][4 * g4 + 2], acc[i][j][4 * g4 + 3]};
+            zero ? gm_f32x4{0.f, 0.f, 0.f, 0.f} : gm_f32x4{v[4 * g4], v[4 * g4 + 1], v[4 * g4 + 2], v[4 * g4 + 3]};
+    }
 }
 
 // KS > 0: block = K slice of one tile (K / 64 k-tiles in KS near-equal runs),
@@ -208,14 +215,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int col0 = c * S::CN + wc * 64;
   const bool live = col0 < nt;
   float *cw = C + (size_t)(col0 + r) * ldc + wr * 32 * RT + 4 * h;
-  gm_f32x16 acc[RT][2];
+  gm_f32x16 acc[S::SUMS][RT][2];
   auto zero_acc = [&]() {
 #pragma unroll
-    for (int i = 0; i < RT; i++)
+    for (int s = 0; s < S::SUMS; s++)
 #pragma unroll
-      for (int jj = 0; jj < 2; jj++)
+      for (int i = 0; i < RT; i++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) acc[i][jj][e] = 0.f;
+        for (int jj = 0; jj < 2; jj++)
+#pragma unroll
+          for (int e = 0; e < 16; e++) acc[s][i][jj][e] = 0.f;
   };
   zero_acc();
   // zeros for the C blocks past each tile whose last segment is this block's
@@ -223,7 +232,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int mt = g0 / nk; mt <= last / nk; mt++) {
       if ((mt + 1) * nk - 1 > last) break;  // the tile goes on in the next block
       for (int sl = j - mt * nk / Lshare + 1; sl < ns; sl++)
-        gm_store<RT>(acc, cw + sl * slot_stride + mt * GM_BM, ldc, true);
+        gm_store(acc, cw + sl * slot_stride + mt * GM_BM, ldc, true);
     }
   // fragment f of step q: weight rows 32 RT wr + 32 f + r, B rows hi / lo
   // 64 wc + 32 j + r; every row's key is (r >> 1) & 7
@@ -246,7 +255,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int f = 0; f < RT + 4; f++) to[f] = frag(pa, pb, q, f);
-    gm_mfma<RT>(acc, fr);
+    gm_mfma(acc, fr);
 #pragma unroll
     for (int k = 0; k < RT + 4; k++) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -266,7 +275,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     step(f1, f0, 0);  // the next k-tile's first fragments (past the last: unused)
     if (c_kt == nk - 1 || g == last) {
       const int slot = ks > 0 ? j : j - c_mt * nk / Lshare;  // this segment's C block
-      if (live) gm_store<RT>(acc, cw + slot * slot_stride + c_mt * GM_BM, ldc, false);
+      if (live) gm_store(acc, cw + slot * slot_stride + c_mt * GM_BM, ldc, false);
       zero_acc();
     }
     if (++c_kt == nk) {
