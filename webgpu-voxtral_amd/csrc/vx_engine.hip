@@ -22,6 +22,7 @@
 #include "vx_prefill.h"
 #include "vx_codec.h"
 #include "vx_gemm.h"
+#include "vx_stage.h"
 #include "vx_loader.h"
 #include "vx_tokenizer.h"
 
@@ -139,7 +140,7 @@ struct vx_engine {
   double *tp_params = nullptr;
   uint32_t *h_frame = nullptr;  // [2][1 + NAC], pinned, written by the frame's last kernels
   uint32_t *d_frame = nullptr;  // h_frame's device address
-  // pinned staging of the calls' host operands and results (struct Stage):
+  // pinned staging of the calls' host operands and results (class Stage):
   // [0, STAGE_BYTES) in, then as much out
   unsigned char *h_stage = nullptr, *d_stage = nullptr;
   hipEvent_t ev_frame[2] = {nullptr, nullptr};
@@ -586,72 +587,6 @@ static int run_step_hold(vx_engine *e) {
   return run_seq(e, &e->hold_exec, enqueue_backbone_hold);
 }
 
-// ---------------------------------------------------------------- staging
-// A call's host operands and results cross the bus through pinned memory that
-// a small kernel on the engine's stream reads or writes.  hipMemcpyAsync on
-// the caller's pageable memory costs the host 10-20 us a copy (its own
-// staging, and a wait for each copy back), which a small call pays two to five
-// times: a two-layer step at 3900 positions took 144 us for 110 us of
-// kernels.  Every call that stages waits for the stream before it returns, so
-// the buffer is free at the next.
-constexpr size_t STAGE_BYTES = (size_t)1 << 20;  // each way; larger operands are copied as before
-
-// bytes: a multiple of 4; both addresses are 16-byte aligned
-__global__ __launch_bounds__(256) void stage_copy_kernel(const uint32_t *src, uint32_t *dst, int bytes) {
-  const int i = 4 * (blockIdx.x * 256 + threadIdx.x), left = bytes / 4 - i;
-  if (left >= 4) *(u32x4 *)(dst + i) = *(const u32x4 *)(src + i);
-  else
-    for (int q = 0; q < left; q++) dst[i + q] = src[i + q];
-}
-
-// One call's operands and results.  finish() waits for the stream and hands
-// the results over.
-struct Stage {
-  vx_engine *e;
-  size_t in_at = 0, out_at = 0;
-  int n = 0;
-  struct {
-    void *dst;
-    size_t at, bytes;
-  } outs[4];
-  explicit Stage(vx_engine *e_) : e(e_) {}
-  void copy(void *dst, const void *src, size_t bytes) {
-    hipLaunchKernelGGL(stage_copy_kernel, dim3((bytes + 4095) / 4096), dim3(256), 0, e->st, (const uint32_t *)src,
-                       (uint32_t *)dst, (int)bytes);
-  }
-  int in(void *dev, const void *src, size_t bytes) {
-    if (bytes == 0) return VX_OK;
-    if (bytes % 4 || in_at + bytes > STAGE_BYTES) {
-      HIPCHK(e, hipMemcpyAsync(dev, src, bytes, hipMemcpyHostToDevice, e->st));
-      return VX_OK;
-    }
-    memcpy(e->h_stage + in_at, src, bytes);
-    copy(dev, e->d_stage + in_at, bytes);
-    in_at += align256(bytes);
-    return VX_OK;
-  }
-  int out(void *dst, const void *dev, size_t bytes) {
-    if (bytes == 0) return VX_OK;
-    if (n == 4 || bytes % 4 || ((uintptr_t)dev & 15) || out_at + bytes > STAGE_BYTES) {
-      HIPCHK(e, hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, e->st));
-      return VX_OK;
-    }
-    const size_t at = STAGE_BYTES + out_at;
-    copy(e->d_stage + at, dev, bytes);
-    outs[n].dst = dst;
-    outs[n].at = at;
-    outs[n++].bytes = bytes;
-    out_at += align256(bytes);
-    return VX_OK;
-  }
-  int finish() {
-    LAUNCHCHK(e);
-    HIPCHK(e, hipStreamSynchronize(e->st));
-    for (int i = 0; i < n; i++) memcpy(outs[i].dst, e->h_stage + outs[i].at, outs[i].bytes);
-    return VX_OK;
-  }
-};
-
 // ---------------------------------------------------------------- helpers
 __global__ void set_int_kernel(int *p, int v) { *p = v; }
 __global__ void set_u32_kernel(uint32_t *p, const uint32_t v0) { *p = v0; }
@@ -662,7 +597,10 @@ static int check_ready(vx_engine *e) {
   return VX_OK;
 }
 
-static int prepare_input(vx_engine *e, int32_t token, int32_t mode, const float *pre) {
+static Stage staging(vx_engine *e) { return Stage(e->st, e->h_stage, e->d_stage); }
+
+// the step's input row; io: the call's staging, which it finishes
+static int prepare_input(vx_engine *e, Stage &io, int32_t token, int32_t mode, const float *pre) {
   if (e->host_pos >= e->max_seq)
     return fail(e, VX_E_RANGE, "position %d reaches max_seq_len %d", e->host_pos, e->max_seq);
   switch (mode) {
@@ -680,7 +618,7 @@ static int prepare_input(vx_engine *e, int32_t token, int32_t mode, const float 
       break;
     case VX_EMBED_PRECOMPUTED:
       if (!pre) return fail(e, VX_E_INVALID, "precomputed embedding is NULL");
-      if (int rc = Stage(e).in(e->x, pre, DIM * sizeof(float))) return rc;
+      HIPCHK(e, io.in(e->x, pre, DIM * sizeof(float)));
       break;
     case VX_EMBED_CODES:
       hipLaunchKernelGGL(multi_codebook_kernel, dim3(DIM / 256), dim3(256), 0, e->st, e->audio_emb,
@@ -1402,17 +1340,18 @@ int vx_backbone_step(vx_engine *e, int32_t token, int32_t mode, const float *pre
   if (!e) return VX_E_INVALID;
   int rc = check_ready(e);
   if (rc) return rc;
-  if ((rc = prepare_input(e, token, mode, pre))) return rc;
+  Stage io = staging(e);
+  if ((rc = prepare_input(e, io, token, mode, pre))) return rc;
   if ((rc = run_step(e))) return rc;
   e->host_pos++;
   if (lm_head) {
     enqueue_lm_head(e);
     LAUNCHCHK(e);
   }
-  Stage io(e);
-  if (argmax_out && lm_head && (rc = io.out(argmax_out, e->argmax_res, 4))) return rc;
-  if (normed_out && (rc = io.out(normed_out, e->normed, DIM * 4))) return rc;
-  return io.finish();
+  if (argmax_out && lm_head) HIPCHK(e, io.out(argmax_out, e->argmax_res, 4));
+  if (normed_out) HIPCHK(e, io.out(normed_out, e->normed, DIM * 4));
+  HIPCHK(e, io.finish());
+  return VX_OK;
 }
 
 // One eager step that stages the reference's per-layer read points
@@ -1422,10 +1361,10 @@ int vx_backbone_step(vx_engine *e, int32_t token, int32_t mode, const float *pre
 // formed here by the final-norm kernel with the layer's gains: the fused
 // prologue's formula x * (1 / sqrt(sum x^2 / dim + eps)) * w, its sum of
 // squares added in another order.
-static int debug_layers_step(vx_engine *e, int32_t token, int32_t mode, const float *pre) {
+static int debug_layers_step(vx_engine *e, Stage &io, int32_t token, int32_t mode, const float *pre) {
   int rc = check_ready(e);
   if (rc) return rc;
-  if ((rc = prepare_input(e, token, mode, pre))) return rc;
+  if ((rc = prepare_input(e, io, token, mode, pre))) return rc;
   const float eps = e->cfg.norm_eps;
   auto stage = [&](int row) { return e->layer_stage + (size_t)row * DIM; };
   HIPCHK(e, hipMemcpyAsync(stage(0), e->x, DIM * 4, hipMemcpyDeviceToDevice, e->st));
@@ -1453,27 +1392,29 @@ static int debug_layers_step(vx_engine *e, int32_t token, int32_t mode, const fl
 int vx_backbone_step_layers(vx_engine *e, int32_t token, int32_t mode, const float *pre,
                             float *layer_out) {
   if (!e || !layer_out) return VX_E_INVALID;
-  int rc = debug_layers_step(e, token, mode, pre);
+  Stage io = staging(e);
+  int rc = debug_layers_step(e, io, token, mode, pre);
   if (rc) return rc;
   for (int l = 0; l < e->cfg.n_layers; l++)
     for (int k = 0; k < 2; k++)
       HIPCHK(e, hipMemcpyAsync(layer_out + (size_t)(2 * l + k) * DIM,
                                e->layer_stage + (size_t)(2 + 4 * l + 2 * k) * DIM, DIM * 4,
                                hipMemcpyDeviceToHost, e->st));
-  HIPCHK(e, hipStreamSynchronize(e->st));
+  HIPCHK(e, io.finish());
   return VX_OK;
 }
 
 int vx_debug_backbone_layers(vx_engine *e, int32_t token, int32_t mode, const float *pre, float *embed,
                              float *layers) {
   if (!e || (!embed && !layers)) return VX_E_INVALID;
-  int rc = debug_layers_step(e, token, mode, pre);
+  Stage io = staging(e);
+  int rc = debug_layers_step(e, io, token, mode, pre);
   if (rc) return rc;
   if (embed) HIPCHK(e, hipMemcpyAsync(embed, e->layer_stage, DIM * 4, hipMemcpyDeviceToHost, e->st));
   if (layers)
     HIPCHK(e, hipMemcpyAsync(layers, e->layer_stage + DIM, (size_t)e->cfg.n_layers * 4 * DIM * 4,
                              hipMemcpyDeviceToHost, e->st));
-  HIPCHK(e, hipStreamSynchronize(e->st));
+  HIPCHK(e, io.finish());
   return VX_OK;
 }
 
@@ -1483,14 +1424,15 @@ int vx_fm_forward(vx_engine *e, const float *noise, float *sem_logits, uint32_t 
   int rc = check_ready(e);
   if (rc) return rc;
   if ((rc = ensure_tproj(e))) return rc;
-  Stage io(e);
-  if (noise && (rc = io.in(e->noise, noise, NAC * 4))) return rc;
+  Stage io = staging(e);
+  if (noise) HIPCHK(e, io.in(e->noise, noise, NAC * 4));
   enqueue_fm(e, noise ? e->noise : nullptr, false);
   LAUNCHCHK(e);
-  if (sem_logits && (rc = io.out(sem_logits, e->sem_logits, SEMV * 4))) return rc;
-  if (codes && (rc = io.out(codes, e->codes, NAC * 4))) return rc;
-  if (x_final && (rc = io.out(x_final, e->xh + (size_t)e->nsteps() * NAC, NAC * 4))) return rc;
-  return io.finish();
+  if (sem_logits) HIPCHK(e, io.out(sem_logits, e->sem_logits, SEMV * 4));
+  if (codes) HIPCHK(e, io.out(codes, e->codes, NAC * 4));
+  if (x_final) HIPCHK(e, io.out(x_final, e->xh + (size_t)e->nsteps() * NAC, NAC * 4));
+  HIPCHK(e, io.finish());
+  return VX_OK;
 }
 
 int vx_set_semantic_code(vx_engine *e, uint32_t code) {
@@ -1546,9 +1488,10 @@ int vx_read(vx_engine *e, const char *name, float *dst, size_t count) {
   for (auto &b : t)
     if (!strcmp(b.n, name)) {
       if (count > b.cnt) return fail(e, VX_E_INVALID, "%s holds %zu values", name, b.cnt);
-      Stage io(e);
-      if (int rc = io.out(dst, b.p, count * 4)) return rc;
-      return io.finish();
+      Stage io = staging(e);
+      HIPCHK(e, io.out(dst, b.p, count * 4));
+      HIPCHK(e, io.finish());
+      return VX_OK;
     }
   return fail(e, VX_E_INVALID, "Unknown buffer: %s", name);
 }
@@ -1560,9 +1503,10 @@ int vx_write(vx_engine *e, const char *name, const float *src, size_t count) {
   else if (!strcmp(name, "hidden")) dst = e->x;
   else return fail(e, VX_E_INVALID, "Unknown writable buffer: %s", name);
   if (count > (size_t)DIM) return fail(e, VX_E_INVALID, "%s holds %d values", name, DIM);
-  Stage io(e);
-  if (int rc = io.in(dst, src, count * 4)) return rc;
-  return io.finish();
+  Stage io = staging(e);
+  HIPCHK(e, io.in(dst, src, count * 4));
+  HIPCHK(e, io.finish());
+  return VX_OK;
 }
 
 static uint16_t host_f2h(float f) {  // IEEE round-to-nearest-even
@@ -1779,20 +1723,20 @@ int vx_prefill(vx_engine *e, const int32_t *tokens, int32_t n_tokens, int32_t au
   const bool has_voice = voice && audio_count > 0;
   for (int c0 = 0; c0 < n_tokens; c0 += e->pf_chunk) {
     const int n = std::min(e->pf_chunk, n_tokens - c0);
-    Stage io(e);
-    if ((rc = io.in(e->pf_tok, tokens + c0, (size_t)n * 4))) return rc;
+    Stage io = staging(e);
+    HIPCHK(e, io.in(e->pf_tok, tokens + c0, (size_t)n * 4));
     // voice rows of this chunk, at chunk-local offsets
     int vs = 0, vc = 0;
     if (has_voice) {
       const int a = std::max(c0, audio_start), b = std::min(c0 + n, audio_start + audio_count);
       if (a < b) {
-        if ((rc = io.in(e->pf_voice, voice + (size_t)(a - audio_start) * DIM, (size_t)(b - a) * DIM * 4))) return rc;
+        HIPCHK(e, io.in(e->pf_voice, voice + (size_t)(a - audio_start) * DIM, (size_t)(b - a) * DIM * 4));
         vs = a;
         vc = b - a;
       }
     }
     if ((rc = enqueue_prefill_chunk(e, n, c0, vs, vc, vc > 0))) return rc;
-    if ((rc = io.finish())) return rc;  // the host buffers above are reused per chunk
+    HIPCHK(e, io.finish());  // the host buffers above are reused per chunk
   }
   return VX_OK;
 }
@@ -1854,8 +1798,9 @@ int vx_sample_top_p(vx_engine *e, const float *logits, int32_t n, int32_t valid,
     *code = sample_top_p(l.data(), n, top_p, temperature, state);
     return VX_OK;
   }
-  // the kernel reads its operands from the pinned in half (33 KB, once) and
-  // leaves the code and the advanced generator state in the out half
+  // the kernel reads its operands from the pinned in half (33 KB, once), where
+  // it also advances the generator state in place, and leaves the code in the
+  // out half
   constexpr size_t kParams = (size_t)TP_MAXN * 4, kState = kParams + 16;
   static_assert(kParams % 16 == 0 && kState + 8 <= STAGE_BYTES, "staging layout");
   const double params[2] = {top_p, temperature};
@@ -1863,11 +1808,12 @@ int vx_sample_top_p(vx_engine *e, const float *logits, int32_t n, int32_t valid,
   memcpy(h, logits, (size_t)n * 4);
   memcpy(h + kParams, params, 16);
   memcpy(h + kState, state, 8);
+  Stage io = staging(e);
+  io.hold();
   hipLaunchKernelGGL(topp_sample_kernel, dim3(1), dim3(TP_NT), 0, e->st, (const float *)d, n, valid,
                      (const double *)(d + kParams), (uint64_t *)(d + kState), (uint32_t *)(d + STAGE_BYTES),
                      (const int *)nullptr, (uint32_t *)nullptr);
-  LAUNCHCHK(e);
-  HIPCHK(e, hipStreamSynchronize(e->st));
+  HIPCHK(e, io.finish());
   memcpy(code, h + STAGE_BYTES, 4);
   memcpy(state, h + kState, 8);
   return VX_OK;
@@ -2150,16 +2096,16 @@ static int codec_decode_impl(vx_engine *e, const uint32_t *semantic, const uint3
                 vx_codec_stop_count(n_frames, stop));
   if ((rc = codec_prepare(e)) || (rc = codec_reserve(e, n_frames)) || (rc = pf_gemm_setup(e)))
     return rc;
-  Stage io(e);
-  if ((rc = io.in(e->cx_sem, semantic, (size_t)n_frames * 4)) ||
-      (rc = io.in(e->cx_ac, acoustic, (size_t)n_frames * NAC * 4)))
-    return rc;
+  Stage io = staging(e);
+  HIPCHK(e, io.in(e->cx_sem, semantic, (size_t)n_frames * 4));
+  HIPCHK(e, io.in(e->cx_ac, acoustic, (size_t)n_frames * NAC * 4));
   const float *res = nullptr;
   size_t count = 0;
   if ((rc = codec_run(e, n_frames, stop, &res, &count))) return rc;
   LAUNCHCHK(e);
-  if ((rc = io.out(out, res, count * 4))) return rc;
-  return io.finish();
+  HIPCHK(e, io.out(out, res, count * 4));
+  HIPCHK(e, io.finish());
+  return VX_OK;
 }
 
 size_t vx_codec_stop_count(int32_t n_frames, int32_t stop) {
@@ -2262,7 +2208,8 @@ int vx_generate(vx_engine *e, const int32_t *tokens, int32_t n_tokens, int32_t a
     on_stage(user, 1, -1.0);
   }
   // AUDIO token kick (src/engine.ts:2478-2487)
-  if ((rc = prepare_input(e, 24, VX_EMBED_TOKEN, nullptr))) return rc;
+  Stage io = staging(e);  // these inputs stage nothing
+  if ((rc = prepare_input(e, io, 24, VX_EMBED_TOKEN, nullptr))) return rc;
   if ((rc = run_step(e))) return rc;
   e->host_pos++;
 
@@ -2277,7 +2224,7 @@ int vx_generate(vx_engine *e, const int32_t *tokens, int32_t n_tokens, int32_t a
     uint32_t codes[NAC];
     for (int f = 0; f < max_frames; f++) {
       if (f > 0) {
-        if ((rc = prepare_input(e, 0, VX_EMBED_CODES, nullptr))) return rc;
+        if ((rc = prepare_input(e, io, 0, VX_EMBED_CODES, nullptr))) return rc;
         if ((rc = run_step(e))) return rc;
         e->host_pos++;
       }
