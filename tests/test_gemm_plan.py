@@ -1,8 +1,10 @@
 """The GEMM plans (vx_gemm.h, gemm_plan) on the CPU: for every product shape of
-the prefill and the codec and every chunk length, the blocks that the kernel
-derives from a plan cover each (row tile, column tile, k-tile) once, write C
-blocks below the count the consumer sums, leave none of those unwritten, and
-fit C."""
+the prefill and the codec and chunk lengths up to 1024, the blocks that the
+kernels derive from a plan, by the same index arithmetic restated here, cover
+each (row tile, column tile, k-tile) once, write C blocks below the count the
+consumer sums, leave none of those unwritten, and fit C.  Which weights stream
+with the non-temporal hint, and which plans the GPU tests of long prompts and
+decodes run."""
 import os
 import subprocess
 
@@ -21,10 +23,28 @@ static int check(int M, int K, int n, int cus, size_t cap) {
   const GemmPlan p = gemm_plan(M, K, nt, cus, cap);
   if (nt < n || p.slices < 1 || p.slices > 8 || (size_t)p.slices * nt * M > cap) return 1;
   if (p.thin) {  // block (x, s, z): 32 thin rows, k-tiles s nk / ks .., columns z NT ..
-    const int NT = nt < GT_MAXN ? nt : GT_MAXN;
-    bool have = false;
-    gm_with_thin(p.thin, NT, false, [&](auto, int lds) { have = lds > 0 && lds <= 160 * 1024; });
-    return !have || M % (32 * p.thin) || nt % NT || p.ks != p.slices || p.ks > nk;
+    const int NT = nt < GT_MAXN ? nt : GT_MAXN, BM = 32 * p.thin, GX = M / BM, GZ = nt / GT_MAXN > 1 ? nt / GT_MAXN : 1;
+    for (bool hint : {false, true}) {
+      bool have = false;
+      gm_with_thin(p.thin, NT, hint, [&](auto, int lds) { have = lds > 0 && lds <= 160 * 1024; });
+      if (!have) return 8;
+    }
+    std::vector<char> seen((size_t)(M / 32) * (nt / 16) * nk, 0);  // 32 rows x 16 columns x k-tile
+    for (int bx = 0; bx < GX; bx++)
+      for (int s = 0; s < p.ks; s++)
+        for (int z = 0; z < GZ; z++) {
+          const int k0 = s * nk / p.ks, k1 = (s + 1) * nk / p.ks;
+          if (k0 >= k1) return 9;
+          for (int m = bx * BM; m < bx * BM + BM; m += 32)
+            for (int c = z * NT; c < z * NT + NT; c += 16)
+              for (int k = k0; k < k1; k++) {
+                if (m >= M || c >= nt) return 10;
+                seen[((size_t)(m / 32) * (nt / 16) + c / 16) * nk + k]++;
+              }
+        }
+    for (char v : seen)
+      if (v != 1) return 11;
+    return p.ks != p.slices;  // block (., s, .) writes C block s of ks
   }
   const int CN = p.wide ? GmWide::CN : GmNarrow::CN, n_tiles = (nt + CN - 1) / CN, m_tiles = M / GM_BM;
   if (nt % 64) return 2;
@@ -71,6 +91,16 @@ int main() {
   };
   for (auto &s : pf) all(s[0], s[1], (size_t)2048 * 18432);
   for (auto &s : cx) all(s[0], s[1], (size_t)2048 * 8192);
+  // streamed past the caches: the prompt's matrices and the codec's gate/up, no other of the codec's
+  for (auto &s : pf) bad += !gemm_thin_hint(s[0], s[1]);
+  for (auto &s : cx) bad += gemm_thin_hint(s[0], s[1]) != (s[0] == 8192);
+  // the plans that GPU tests of 700 and 1030 tokens and of 150 frames run: whole-tile shares of
+  // 256 x 128 tiles, at an odd multiple of 64 columns too, and the 256 x 128 tile in the codec
+  for (int n : {700, 1024}) {
+    const GemmPlan p = gemm_plan(18432, 3072, gm_cols(n), 256, (size_t)2048 * 18432);
+    bad += !p.wide || p.ks != 0 || p.slices != 1;
+  }
+  bad += gm_cols(700) % 128 != 64 || !gemm_plan(8192, 1024, 1024, 256, (size_t)2048 * 8192).wide;
   return bad != 0;
 }
 """

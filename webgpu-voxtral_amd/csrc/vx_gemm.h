@@ -580,15 +580,24 @@ inline hipError_t gemm_setup() {
   return e;
 }
 
-// n: the live columns of the nt (the thin grid writes only those).  A thin
-// weight stream of a matrix past the L2s' size (32 MB) is non-temporal; the
-// codec's matrices (2-17 MB, 298 MB in all) stay allocating, so that a
-// decode of a few frames finds part of them in the 256 MB last-level cache.
+// Whether the thin grid streams a matrix's weights with the non-temporal hint:
+// from 16 MiB on, the prompt's four matrices and the codec's gate/up (8192 x
+// 1024).  A decode of few frames reads the codec's 298 MB of weights once; with
+// gate/up, a third of them, streamed past the 256 MB last-level cache, more of
+// the rest is found there by the next decode.  Decodes of 13 frames one after
+// the other take 436 us, with a line above gate/up 450, without a line (all
+// matrices hinted) 450, at 8 MiB 446; behind other work 450, 450, 453 and 454;
+// decodes of 1, 4 and 32 frames and prompts of 9 to 32 tokens are within 3% on
+// every line.
+inline bool gemm_thin_hint(int M, int K) { return (size_t)M * K * 2 >= (size_t)16 << 20; }
+
+// n: the live columns of the nt (the thin grid writes only those)
 inline void gemm_launch(const GemmPlan &p, hipStream_t st, const uint16_t *W, int M, int K, const uint16_t *B,
                         int ldb, size_t blo, int nt, int n, float *C) {
   if (p.thin)
-    gm_with_thin(p.thin, std::min(nt, GT_MAXN), (size_t)M * K >= (size_t)8 << 20, [&](auto kernel, int lds) {
-      hipLaunchKernelGGL(kernel, dim3(M / (32 * p.thin), p.ks, std::max(nt / GT_MAXN, 1)), dim3(256), lds, st, W, K, B, ldb, blo, n, C, M);
+    gm_with_thin(p.thin, std::min(nt, GT_MAXN), gemm_thin_hint(M, K), [&](auto kernel, int lds) {
+      hipLaunchKernelGGL(kernel, dim3(M / (32 * p.thin), p.ks, std::max(nt / GT_MAXN, 1)), dim3(256), lds, st, W, K,
+                         B, ldb, blo, n, C, M);
     });
   else if (p.wide)
     hipLaunchKernelGGL(gemm_kernel<GmWide>, dim3(p.grid), dim3(512), GmWide::LDS, st, W, M, K, B, ldb, blo, nt, C, M,
