@@ -264,6 +264,32 @@ def rel_l2(got, ref):
     return float(np.linalg.norm(np.asarray(got, np.float64) - ref) / np.linalg.norm(ref))
 
 
+@pytest.mark.parametrize("n", [700, 1030])
+def test_prefill_long_chunks(n):
+    """The GEMM grids of long prompts at the default chunk: shares of whole
+    tiles with 256 x 128 tiles over an odd multiple of 64 columns (700 tokens:
+    704), and a full 1024-token chunk with a short one behind it.  Layer 1's
+    K/V rows depend on every product of layer 0 for every token; all of both
+    layers' rows against 64 bits.  4e-5 relative: four times the 9.6e-6 seen,
+    in K at the last positions, where the f32 rope angle is that far off; a
+    column tile or K slice gone wrong is 1e-2 and more."""
+    print(f"[prefill] 2 layers, {n} tokens in default chunks", flush=True)
+    g = gpu_engine(n_layers=2, max_seq=1088)
+    try:
+        x = np.random.default_rng(n).standard_normal((n, 3072)).astype(np.float32)
+        g.prefill(np.full(n, 24), 0, n, x)
+        _, y, *kv0 = layer_f64(g, 0, torch.from_numpy(x).double())
+        kv1 = layer_f64(g, 1, y, full=False)[2:]
+        for l, kv in ((0, kv0), (1, kv1)):
+            for w in (0, 1):
+                got = g.read_kv(l, w, 0, n)
+                errs = [rel_l2(got[r:r + 64], kv[w][r:r + 64]) for r in range(0, n, 64)]
+                print(f"[prefill] layer {l} {'KV'[w]}: worst 64 rows {max(errs):.3g}", flush=True)
+                assert max(errs) < 4e-5, (l, w, errs)
+    finally:
+        g.destroy()
+
+
 def test_prompt_attention_small_queries():
     """Queries around 0.02 against keys around 140, so that scores are of
     order 1 although the queries' lo halves are f16 subnormals: their quantum,
