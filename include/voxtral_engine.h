@@ -73,7 +73,10 @@ typedef struct vx_config {
 int vx_config_default(vx_config *cfg);
 
 /* new VoxtralEngine({config, maxSeqLen}) + init(), src/engine.ts:301-340.
- * max_seq_len: KV slots per layer (reference default 4096). */
+ * max_seq_len: KV slots per layer (reference default 4096), at most 2^20.
+ * Device memory beside the weights: the cache, 8 KB a slot and layer (f16: 4
+ * KB), and as much as one layer of it again for the prompt attention's
+ * operands (f32: 32 MB at 4096 slots, 8.6 GB at 2^20). */
 int vx_create(const vx_config *cfg, int32_t max_seq_len, vx_engine **out);
 
 /* destroy(), src/engine.ts:2621-2632 */

@@ -21,18 +21,21 @@
 // rows, brought to LDS by direct loads (global_load_lds_dwordx4, 1 KB per
 // instruction = 8 rows) into a ring of DA weight stages and DB stages of B.
 //
-// What bounds it is the operands' way to the matrix cores, and power.  The
-// 256 x 64 tile's 48 KB of direct loads per k-tile alone take 1180 clocks (41
-// bytes a clock and CU) against 1024 of MFMA; issued by the computing waves
-// (an earlier form) each also held up its wave's MFMAs by 35-41 clocks: 1500
-// clocks a k-tile, 2970 for the 256 x 128 tile, whose MFMAs take 2048.  Hence
-// loaders of their own: four, as one wave issues a direct load only every 60
-// clocks (a single loader took 1.69 us per 256 x 128 k-tile, four 1.25, the
-// computing waves 1.32).  Under full load the clock falls to 1.5 GHz, so bytes
-// moved count twice: the 256 x 128 tile moves 64 KB for twice the MFMAs of the
-// 256 x 64 tile's 48 KB and reads 8 fragments for 16 MFMAs, not 6 for 8.
-// Issued rates at 1024 columns: gate/up (18432 x 3072) 0.91 PFLOP/s, QKV 0.89,
-// where one 8192^3 f16 product of the vendor library reaches 1.18 on this card.
+// What bounds it is power, then the matrix cores and the operands' way to them.
+// Parts left out in a copy, per k-tile of the 256 x 64 tile (192 blocks): whole
+// 1580 clocks, 0.94-1.01 us at 1.6 GHz; without the LDS reads more clocks at a
+// higher clock, the same time; without the direct loads 0.74 us; the loads alone
+// 0.51 us (43 bytes a clock and CU); the MFMAs alone 0.65 us, 1205 clocks for
+// 1024 of issue.  A wave that issues a direct load beside its MFMAs holds them
+// up by 39 clocks, and one wave issues a load every 70 clocks; hence loaders of
+// their own, and four of them: QKV at 1024 columns took 97 us with the loads
+// issued by the computing waves, 102 with one loader wave, 87 with four.  The
+// 256 x 128 tile moves 64 KB for twice the MFMAs of the 256 x 64 tile's 48 KB
+// and reads 8 fragments for 16 MFMAs, not 6 for 8: 1.41-1.50 us a k-tile, 1.5
+// times the narrow one's.
+// Issued rates in prompts: 1024 columns gate/up (18432 x 3072) 1.06 PFLOP/s, QKV
+// 1.01; 256 columns 0.88 and 0.65; one 8192^3 f16 product of the vendor library
+// reaches 1.18 on this card.
 //
 // A block works through k-tiles g0 .. g1 - 1 of one column tile's sequence
 // g = mt nk + kt.  Two ways to cut it:
@@ -498,10 +501,10 @@ inline GemmPlan gemm_thin_plan(int M, int K, int nt, int cus) {
 // in 1 .. 8 slices while that is at most one block per CU; with more tiles
 // than CUs, equal shares, or shares of whole tiles (no tile is cut: one
 // slice).  c_cap: floats that C holds.
-// The figures are a fit to 560 timed plans (88 shapes of K 896 .. 9216, M 256
-// .. 18432 and 64 .. 1024 columns, GEMM plus a reader of C, a copy of 200 MB
-// before each, as other kernels run between a prompt's products): the plan
-// picked is 0.3% slower than the best of them on average and 8% at most.
+// The figures are a fit to timed plans (GEMM plus a reader of C, a copy of 200 MB
+// before each, as other kernels run between a prompt's products).  Of 831 plans
+// of 83 shapes (K 896 .. 9216, M 1024 .. 18432, 64 .. 1024 columns) the one
+// picked is 0.17% slower than the best of its shape on average, 4.4% at most.
 inline GemmPlan gemm_tiled_plan(int M, int K, int nt, int cus, size_t c_cap) {
   GemmPlan best;
   double best_us = -1;
